@@ -135,3 +135,77 @@ def test_a_clamped_step_stops_what_is_not_a_number(hip):
         out.append(hip.layerLifBackward(go, float("nan") * one, None, x, f["ckpt_v"], None, zero, None, am, None, one,
                                         one, lo, True, 2, True, True, 1, 0.5, 1.0))
     assert torch.equal(out[0][0].isnan(), out[1][0].isnan()) and not bool(out[1][0][:, :100].isnan().any())
+
+
+def steep(hip, b, t, m, syn, quiet=()):
+    """A layer without leak whose potential sits on the threshold in every step but the ``quiet`` ones, with a surrogate so
+    narrow that every such step multiplies the adjoint by 1 - c s = -19: 32 of them by 8e40, more than a float holds."""
+    one, zero = torch.ones(b * m, device="cuda"), torch.zeros(b * m, device="cuda")
+    x = torch.ones(b, t, m, device="cuda")
+    for lo, hi in quiet:
+        x[:, lo:hi] = 0.0
+    a_syn = zero if syn else None                      # forgets at once: the current is the input
+    kw = dict(early=False, norm=False, cap=-1)
+    args = (x, zero, zero if syn else None, one, a_syn, one, one, None, False, kw["cap"], kw["early"], kw["norm"])
+    post, pre = hip.layerLifForward(*args, wantRecords=True), hip.layerLifForward(*args, wantPreReset=True)
+    p0 = 0.05
+
+    def backward(mode, go, gv, gi, rec=None):
+        hip.backwardTimeSplit(mode)
+        return hip.layerLifBackward(go, gv, gi, x, post["ckpt_v"], post["ckpt_i"], zero, zero if syn else None, one, a_syn,
+                                    one, one, None, False, -1, False, False, 1, p0, 1.0, gradVRec=rec)
+    v = pre["v_rec"]
+    sg = torch.exp(-(v - 1.0).abs().double() / p0) / p0
+    want = lambda go, gv, gi, rec=None: adjoint64(
+        x, go, sg, v, post["i_rec"] if syn else x, post["v_rec"], zero, zero, gv, gi, rec,
+        torch.zeros_like(x) if rec is not None and syn else None, one, a_syn, one, None, False, False)
+    return backward, want, zero
+
+
+@pytest.mark.parametrize("syn", [False, True])
+@pytest.mark.parametrize("rec", [False, True])
+@pytest.mark.parametrize("t", [96, 1000, 1100])
+def test_chunks_whose_factors_overflow_pass_nothing_on_where_nothing_enters(hip, syn, rec, t):
+    """A loss on the first steps only: exactly 0 enters every chunk but the first from later steps, whatever its factors.
+    Three steps with factors of 19: about ten roundings, and the exponential's error of 2e-7 three times."""
+    b, m = 2, 20
+    backward, want, zero = steep(hip, b, t, m, syn)
+    go = torch.zeros(b, t, m, device="cuda")
+    go[:, :3] = torch.randn(b, 3, m, generator=gen(1)).cuda()
+    qv = torch.zeros_like(go) if rec else None
+    w, got, one = want(go, zero, zero, qv), backward(1, go, zero, zero, qv), backward(0, go, zero, zero, qv)
+    for z in (got, one):
+        assert bool(z[0].isfinite().all()) and not bool(z[0][:, 3:].any())
+        for mine, ideal in ((z[0], w[0]), (z[1], w[1]), (z[3], w[3])) + (((z[2], w[2]),) if syn else ()):
+            assert float((mine.double() - ideal).norm()) <= 2e-6 * float(ideal.norm())
+
+
+@pytest.mark.parametrize("syn", [False, True])
+def test_a_small_gradient_through_a_chunk_whose_factors_overflow(hip, syn):
+    """1e-30 at the final state grows by 8e40 within one chunk: infinity times 1e-30 would be infinite."""
+    b, t, m = 2, 96, 20
+    backward, want, zero = steep(hip, b, t, m, syn, quiet=((0, 32), (64, 96)))
+    go, gv = torch.zeros(b, t, m, device="cuda"), torch.full((b * m,), 1e-30, device="cuda")
+    w, got, one = want(go, gv, zero), backward(1, go, gv, zero), backward(0, go, gv, zero)
+    assert float(w[0].abs().max()) > 1e10
+    for z in (got, one):                               # 32 factors: three roundings and the exponential's error each
+        assert float((z[0].double() - w[0]).norm()) <= 2e-5 * float(w[0].norm())
+    assert torch.equal(got[0], one[0])                 # passed on step by step, as one lane per neuron does it
+
+
+def test_a_gradient_that_is_no_number_among_ordinary_neurons(hip):
+    """One neuron's final state has a gradient that is no number: its block passes on chunk by chunk, the others fold."""
+    b, t, m = 1, 300, 200
+    x = (torch.randn(b, t, m, generator=gen(1)) * 0.8 + 0.4).cuda()
+    one, zero = torch.ones(m, device="cuda"), torch.zeros(m, device="cuda")
+    f = hip.layerLifForward(x, zero, zero, 0.9 * one, 0.5 * one, one, one, None, False, 2, True, True)
+    go, gv = torch.randn(b, t, m, generator=gen(2)).cuda(), zero.clone()
+    gv[70] = float("nan")
+    out = []
+    for mode in (0, 1):
+        hip.backwardTimeSplit(mode)
+        out.append(hip.layerLifBackward(go, gv, zero, x, f["ckpt_v"], f["ckpt_i"], zero, zero, 0.9 * one, 0.5 * one, one, one,
+                                        None, False, 2, True, True, 1, 0.5, 1.0)[0])
+    assert torch.equal(out[0].isnan(), out[1].isnan()) and bool(out[1][:, :, 70].isnan().all())
+    assert int(out[1].isnan().sum()) == t
+    assert float((out[0] - out[1]).nan_to_num().norm()) <= 4e-6 * float(out[0].nan_to_num().norm())
