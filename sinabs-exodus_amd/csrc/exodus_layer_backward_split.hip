@@ -20,11 +20,12 @@ namespace {
 // (h_in and hm_in are folded instead of walked), not bit for bit.
 //
 // B, D and U are products of 32 factors a_mem (1 - c s) or a_syn.  Where |1 - c s| stays above 16 (narrow surrogates) B
-// leaves the floats' range, and infinity times an h_in of 0, or of 1e-30, says nothing about h_out.  Any such map, and any
-// h_in that is no number, makes a folded h_in or hm_in that is not finite; then the block passes h and hm through the
-// group's chunks one after the other with the operations of the walk, which is right for every value: 36 us more per group
-// of 32 chunks, (4, 2000, 512) 31 -> 103 against 275 with one lane per neuron.  The vote costs other calls 0.2 to 0.4 us of
-// 7 to 13; sequences of 1000 steps and more gained 2 to 5 % by the flags for clamped steps that it replaced.
+// leaves the floats' range, and infinity times an h_in of 0, or of 1e-30, says nothing about h_out.  A block with such a
+// map passes h and hm through the group's chunks one after the other with the operations of the walk, which is right for
+// every value: 39 us more per group of 32 chunks, (4, 2000, 512) 31 -> 109 against 276 with one lane per neuron.  The waves
+// say so where they publish their maps, which costs other calls 0.1 to 0.4 us of 8 to 10 (a vote of the block on the folded
+// values, one barrier more, 0.2 to 0.9).  Where all maps are finite an h_in that is no number is folded like any other:
+// `stops` has it end at a clamped step as the walk does.
 //
 // What bounds it: the chain of 3 x 32 steps per group and one trip to memory and back, 9-11 us for up to 32 chunks on an
 // otherwise idle machine ((8, 100, 256) 14.5 -> 9.4 us, (64, 300, 10) 16.8 -> 11.0 against the kernel that carried two
@@ -45,6 +46,11 @@ __global__ void __launch_bounds__(SPLIT_LANES) layer_lif_backward_split(const Sp
     typedef BufIO<1, false> IO;
     __shared__ float map_a[SPLIT_LANES], map_b[SPLIT_LANES];
     __shared__ float map_c[SYN ? SPLIT_LANES : 1], map_d[SYN ? SPLIT_LANES : 1], map_u[SYN ? SPLIT_LANES : 1];
+    __shared__ unsigned char stops[SPLIT_LANES];   // 1: h_in ends inside the chunk, 2: it does not get into mu either
+    __shared__ union {
+        unsigned char of_wave[SPLIT_LANES / WAVE];
+        uint64_t all;
+    } wild;                                        // a map of the wave is not finite
     __shared__ float carry_h[SPLIT_NEURONS], carry_m[SPLIT_NEURONS];
     __shared__ double part_m[SPLIT_LANES], part_s[SYN ? SPLIT_LANES : 1];
     const LayerConsts &p = q.p;
@@ -169,20 +175,27 @@ __global__ void __launch_bounds__(SPLIT_LANES) layer_lif_backward_split(const Sp
             map_d[tid] = mq;
             map_u[tid] = mu_u;
         }
+        const unsigned inside = len >= CKPT ? ~0u : (1u << len) - 1u;
+        stops[tid] = ((open & inside) != inside ? 1 : 0) | (len == 0 || !((open >> (len - 1)) & 1u) ? 2 : 0);
+        const auto finite = [](float f) { return fabsf(f) < __builtin_inff(); };
+        const bool tame = finite(hp) && finite(hq) && (!SYN || (finite(mp) && finite(mq) && finite(mu_u)));
+        const bool some = __builtin_amdgcn_ballot_w64(active && !tame) != 0;
+        if ((tid & (WAVE - 1)) == 0) wild.of_wave[tid / WAVE] = some ? 1 : 0;
         __syncthreads();
         // what enters this chunk from later steps
         h = carry_h[lane];
         hm = SYN ? carry_m[lane] : 0.f;
         for (int c = chunks - 1; c > j; --c) {
             const int at_c = (c << neurons_log) + lane;
+            const int stop = stops[at_c];
             if (SYN) {
                 hm = __fadd_rn(map_c[at_c], __fmul_rn(map_u[at_c], hm));
-                hm = __fadd_rn(hm, __fmul_rn(map_d[at_c], h));
+                if (!(stop & 2)) hm = __fadd_rn(hm, __fmul_rn(map_d[at_c], h));
             }
-            h = __fadd_rn(map_a[at_c], __fmul_rn(map_b[at_c], h));
+            h = stop & 1 ? map_a[at_c] : __fadd_rn(map_a[at_c], __fmul_rn(map_b[at_c], h));
         }
-        const bool finite = fabsf(h) < __builtin_inff() && (!SYN || fabsf(hm) < __builtin_inff());
-        if (__syncthreads_or(active && !finite)) {               // chunk after chunk, results in map_a and map_c
+        if (wild.all << (64 - 8 * (blockDim.x / WAVE))) {        // some wave's byte: chunk after chunk, results in map_a, map_c
+            __syncthreads();                                     // everybody has read the maps
             for (int c = chunks - 1; c >= 0; --c) {
                 if (j == c) {
                     h = c == chunks - 1 ? carry_h[lane] : map_a[tid + many];
