@@ -15,9 +15,9 @@ namespace {
 //     h_out = A + B h_in,   hm_out = C + D h_in + U hm_in.
 // A lane rebuilds its chunk, keeps (a, b, vpost, i) of every step, walks it once for (A, B, C, D, U), exchanges them through
 // LDS, folds the maps of the newer chunks into its own (h_in, hm_in), and walks the chunk again with the operations of the
-// one-lane kernel.  A block holds up to 32 chunks of 16 to 64 neurons; longer sequences are walked in groups of chunks,
-// newest first, what leaves a group waiting in LDS for the next.  Results agree with the one-lane kernel's to rounding
-// (h_in and hm_in are folded instead of walked), not bit for bit.
+// one-lane kernel.  A block holds up to 32 chunks of 16 to 64 neurons (see launch); longer sequences are walked in groups
+// of chunks, newest first, what leaves a group waiting in LDS for the next.  Results agree with the one-lane kernel's to
+// rounding (h_in and hm_in are folded instead of walked), not bit for bit.
 //
 // B, D and U are products of 32 factors a_mem (1 - c s) or a_syn.  Where |1 - c s| stays above 16 (narrow surrogates) B
 // leaves the floats' range, and infinity times an h_in of 0, or of 1e-30, says nothing about h_out.  A block with such a
@@ -283,11 +283,27 @@ template <bool SYN, int KIND, int CAPK, bool EXTRA, bool GO1>
 int launch(const SplitArgs &a, int64_t B, hipStream_t s)
 {
     const int64_t n_ck = (a.T + CKPT - 1) / CKPT;
-    const int64_t groups = (n_ck + SPLIT_CHUNKS - 1) / SPLIT_CHUNKS;
+    // 256 registers per lane leave a compute unit eight waves, one block of more than four.  A launch of more such blocks than
+    // there are compute units takes another round of them, so it takes smaller groups of chunks instead: 16 chunks of 32
+    // neurons in the place of 32 of 16, and where that is too many blocks 8 of 32, two blocks to a compute unit.  Without /
+    // with, us: 16 384 neurons 300 steps 26.8 / 21.9, 512 steps 31.0 / 25.4, with synapses 37.7 / 29.6, 2000 steps 171 / 107,
+    // with state records 309 / 203, with a surrogate tensor 188 / 130; 10 240 neurons 300 steps 22.2 / 18.8; 8192 neurons
+    // 1000 steps 41 / 30.  Where one round does, smaller groups only lengthen the chain: 8192 neurons 300 steps 12.5 / 15.8,
+    // 4096 neurons 1000 steps with synapses 25.6 / 28.2.  (Up to 8 chunks of 64 neurons are one round for 16 384 neurons.)
+    const auto blocks = [&](int log) { return ((a.M + (int64_t{1} << log) - 1) >> log) * B; };
+    const int64_t cus = compute_units();
+    int most = SPLIT_CHUNKS, widest = 6;
+    if (n_ck > 16 && blocks(4) > cus) most = 16;
+    if (n_ck > 8 && blocks(5) > cus) {
+        most = 8;
+        widest = 5;
+    }
+    const int64_t groups = (n_ck + most - 1) / most;
     const int chunks = static_cast<int>((n_ck + groups - 1) / groups);
     // as many neurons per block as its lanes hold, but no more than the layer has
     int neurons_log = 4;
-    while (neurons_log < 6 && (chunks << (neurons_log + 1)) <= SPLIT_LANES && (int64_t{1} << neurons_log) < a.M) ++neurons_log;
+    while (neurons_log < widest && (chunks << (neurons_log + 1)) <= SPLIT_LANES && (int64_t{1} << neurons_log) < a.M)
+        ++neurons_log;
     const int64_t blocks_per_batch = (a.M + (int64_t{1} << neurons_log) - 1) >> neurons_log;
     if (blocks_per_batch > 0x7fffffffLL / B) return hipErrorInvalidValue;
     const int lanes = ((chunks << neurons_log) + WAVE - 1) / WAVE * WAVE;

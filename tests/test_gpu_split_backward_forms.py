@@ -110,6 +110,15 @@ def test_against_float64(hip, form, b, t, m):
         assert err(s) <= bound, (name, err(s), err(o))
 
 
+@pytest.mark.parametrize("form", [dict(), dict(syn=True, clamp=True, cap=2, uniform=True), dict(rec=True, tensor=True, syn=True)],
+                         ids=["plain", "syn", "records"])
+@pytest.mark.parametrize("b,t,m", [(5, 545, 1030),     # more than 256 blocks of 16 neurons: groups of up to 16 chunks
+                                   (9, 300, 1030),     # more than 256 blocks of 32: two groups of 5 chunks, the lanes hold 6
+                                   (300, 530, 33), (1200, 290, 3)])   # 17 chunks in groups of 6, 10 in lanes for 8
+def test_groups_of_fewer_chunks_where_the_blocks_are_many(hip, form, b, t, m):
+    test_against_float64(hip, form, b, t, m)
+
+
 def test_a_clamped_step_stops_what_is_not_a_number(hip):
     """A gradient that is no number at the final state ends where the potential was clamped, chunk by chunk as step by
     step."""
