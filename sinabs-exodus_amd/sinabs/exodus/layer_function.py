@@ -124,6 +124,7 @@ class SpikingLayerFunction(torch.autograd.Function):
         tau_mem = rest.pop(0) if ctx.taus[0] else None
         tau_syn = rest.pop(0) if ctx.taus[1] else None
         need = ctx.needs_input_grad
+        need += (False,) * (17 - len(need))             # one entry per argument that the call named
         if all(g is None for g in (grad_spikes, grad_v_last, grad_i_last, grad_total, grad_v_rec, grad_i_rec)):
             return (None,) * 17
         # one value for every spike (a sum as the loss, the spike total behind firing_rate): handed over as it is
@@ -156,8 +157,8 @@ class SpikingLayerFunction(torch.autograd.Function):
             v_mem_init, i_syn_init, alpha_mem, alpha_syn, membrane_subtract, threshold, min_v_mem, apply_min,
             max_spikes, decay_early, norm_input, kind, p0, p1, surr=surr,
             gradVRec=cont(grad_v_rec), gradIRec=cont(grad_i_rec) if syn else None,
-            wantAlphaMemGrad=need[1] or need[15], wantAlphaSynGrad=need[2] or need[16], wantVInitGrad=need[3], wantIInitGrad=need[4],
-            gradUniform=uniform is not None,
+            wantAlphaMemGrad=need[1] or need[15], wantAlphaSynGrad=need[2] or need[16], wantVInitGrad=need[3],
+            wantIInitGrad=need[4], gradUniform=uniform is not None,
         )
         b, _, m = inp.shape
         g_tm = _hip.decayGrad(g_am, tau_mem, b, m) if need[15] else None
@@ -179,7 +180,7 @@ class LeakyLayerFunction(torch.autograd.Function):
             raise ValueError("'inp' must be 3D, (batch, time, neurons)")
         if not inp.is_contiguous():
             raise ValueError("'inp' has to be contiguous.")
-        need_alpha = ctx.needs_input_grad[1] or ctx.needs_input_grad[6]
+        need_alpha = (alpha if tau is None else tau).requires_grad
         if tau is not None:
             alpha, tau = _hip.decayExpand(tau, inp.shape[0], inp.shape[2])
         out, v_last, total = _hip.layerLeakyForward(inp, v_mem_init, alpha, decay_early, norm_input,
