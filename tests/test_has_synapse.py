@@ -25,3 +25,15 @@ def test_a_subclass_with_its_own_time_constant_is_asked():
             return 3.0
     assert Own(tau_mem=20.0)._has_synapse()
     assert not el.LIF(tau_mem=20.0)._has_synapse()
+
+
+@pytest.mark.parametrize("tau_syn", [None, 5.0])
+def test_refused_where_the_time_constant_is(tau_syn):
+    """train_alphas changed by hand: the parameter that would tell is not there."""
+    import sinabs.exodus.layers as el
+    layer = el.IAF(tau_syn=tau_syn)
+    layer.train_alphas = True
+    with pytest.raises(AttributeError):
+        layer.tau_syn_calculated
+    with pytest.raises(AttributeError):
+        layer._has_synapse()
