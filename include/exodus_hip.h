@@ -196,8 +196,8 @@ int exodus_layer_lif_forward(float *out_spikes, float *out_vmem_rec, float *out_
                              int apply_theta_low, int max_num_spikes, int decay_early, int norm_input,
                              int record_pre_reset, int64_t batch, int64_t t, int64_t neurons, void *stream);
 
-/* The same with a total (one double, NULL = not wanted) that is written instead of added to: every wave leaves its count in
- * sum_work, exodus_layer_sum_slots(batch, neurons) doubles that need no initialising, and a second kernel of the call adds
+/* The same with a total (one double, NULL = not wanted) that is written instead of added to: every block leaves its count
+ * in sum_work, exodus_layer_sum_slots(batch, neurons) doubles that need no initialising, and a second kernel of the call adds
  * them up.  Many waves that add to one double at the end of a launch wait for each other; here none does. */
 int exodus_layer_lif_forward_total(float *out_spikes, float *out_vmem_rec, float *out_isyn_rec, float *ckpt_v,
                                    float *ckpt_i, float *v_last, float *i_last, double *spike_sum, double *sum_work,

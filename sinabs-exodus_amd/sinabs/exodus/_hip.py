@@ -88,6 +88,8 @@ def _load() -> ctypes.CDLL:
 
 
 lib = _load()
+# doubles of scratch a layer total wants (exodus_layer_sum_slots): one per so many neurons of a batch element
+_NEURONS_PER_SUM_SLOT = (1 << 20) // int(lib.exodus_layer_sum_slots(1, 1 << 20))
 
 
 class ExodusHipError(RuntimeError):
@@ -464,7 +466,7 @@ def _total_and_work(input: torch.Tensor):
     if input.numel() == 0:
         return torch.zeros((), dtype=torch.float64, device=input.device), None
     return (torch.empty((), dtype=torch.float64, device=input.device),
-            torch.empty(b * ((m + 63) // 64), dtype=torch.float64, device=input.device))
+            torch.empty(b * -(-m // _NEURONS_PER_SUM_SLOT), dtype=torch.float64, device=input.device))
 
 
 def layerLifForward(input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, membrSubtract, theta, thetaLow,
