@@ -64,3 +64,9 @@ def test_several_neurons_per_lane(b, t, m, cap):
     """From 524 288 neurons on a lane holds two, from 1 048 576 on four where their number allows it."""
     check(b, t, m, cap, False, m)
     check(b, t, m, cap, True, m + 1, syn=True)
+
+
+@pytest.mark.parametrize("b,t,m,cap", [(8, 1, 65538, -1), (3, 2, 180002, 2), (4, 3, 262148, -1), (1, 1, 1048580, 1)])
+def test_a_step_or_two_with_several_neurons_per_lane(b, t, m, cap):
+    check(b, t, m, cap, False, m)
+    check(b, t, m, cap, True, m + 1, syn=True)

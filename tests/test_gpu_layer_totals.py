@@ -6,7 +6,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(1, 5, 1), (2, 33, 63), (3, 40, 64), (2, 7, 65), (5, 70, 130), (1, 3, 70001), (40, 17, 4098), (64, 9, 8192),
+SHAPES = [(1, 5, 1), (2, 33, 63), (3, 40, 64), (2, 7, 65), (5, 70, 130), (30, 4, 700), (1, 3, 70001), (40, 17, 4098), (64, 9, 8192),
           (3, 2, 600000), (2, 0, 70), (0, 5, 70)]
 
 

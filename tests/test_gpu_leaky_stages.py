@@ -67,3 +67,10 @@ def test_several_neurons_per_lane(b, t, m, uniform):
     """From 262 144 neurons on a lane holds two, from 524 288 on four where their number allows it."""
     check(b, t, m, False, False, uniform, m)
     check(b, t, m, True, True, uniform, m + 1)
+
+
+@pytest.mark.parametrize("b,t,m", [(5, 1, 60002), (3, 2, 180004), (3, 3, 180004)])
+@pytest.mark.parametrize("uniform", [False, True])
+def test_a_step_or_two_with_several_neurons_per_lane(b, t, m, uniform):
+    check(b, t, m, False, False, uniform, m)
+    check(b, t, m, True, True, uniform, m + 1)
