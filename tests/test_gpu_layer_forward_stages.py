@@ -70,3 +70,9 @@ def test_several_neurons_per_lane(b, t, m, cap):
 def test_a_step_or_two_with_several_neurons_per_lane(b, t, m, cap):
     check(b, t, m, cap, False, m)
     check(b, t, m, cap, True, m + 1, syn=True)
+
+
+@pytest.mark.parametrize("b,t,m", [(4, 120, 131074), (2, 100, 524292)])
+def test_stages_done_again_with_several_neurons_per_lane(b, t, m):
+    """Long enough for waves to go to the exact steps and back several times (two and four neurons per lane)."""
+    check(b, t, m, -1, False, m)
