@@ -30,9 +30,6 @@ namespace {
 #ifndef EXODUS_LEAKY_WAVES
 #define EXODUS_LEAKY_WAVES 8          // waves per CU the leaky kernels want before a lane takes more than one neuron
 #endif
-#ifndef EXODUS_LAYER_CKPT
-#define EXODUS_LAYER_CKPT 32          // steps between checkpoints (a multiple of 32)
-#endif
 #ifndef EXODUS_WHOLE_NEURONS
 #define EXODUS_WHOLE_NEURONS 16       // neurons per step must be a multiple of this for the non-temporal kernel instances
 #endif
@@ -43,7 +40,7 @@ namespace {
 #define EXODUS_LAYER_BWD_WAVES_G1 3   // ... and its instances that stream one tensor less (one gradient value for all): a
                                       // fourth wave fits them only with spills and measures no faster
 #endif
-constexpr int CKPT = EXODUS_LAYER_CKPT;               // steps between checkpoints = length of a backward chunk
+constexpr int CKPT = 32;                              // steps between checkpoints = length of a backward chunk
 constexpr int fwd_unroll(int npl) { return npl == 1 ? 16 : 8; }   // forward steps per software-pipeline stage (divides CKPT / 2)
 constexpr int BLOCK = EXODUS_LAYER_BLOCK;
 constexpr int BWD_BLOCK = EXODUS_LAYER_BWD_BLOCK;

@@ -36,6 +36,7 @@ namespace {
 constexpr int SPLIT_LANES = 512;
 constexpr int SPLIT_CHUNKS = 32;           // most chunks of a group
 constexpr int SPLIT_NEURONS = 64;          // most neurons of a block
+static_assert(CKPT == 32, "a chunk's clamped steps are bits of an unsigned, a_syn^CKPT is squared up, a group spans 2^10 steps");
 
 // EXTRA: gradients on the state records; GO1: one value as the gradient of every spike (see the one-lane kernel)
 template <bool SYN, int KIND, int CAPK, bool EXTRA, bool GO1>
