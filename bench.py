@@ -844,7 +844,7 @@ def main():
     dev = torch.device("cuda:0")
     torch.cuda.set_device(dev)
     if args.one_lane_per_neuron or args.split_any_size:
-        hip.backwardTimeSplit(0 if args.one_lane_per_neuron else 2)
+        hip.backwardTimeSplit(0 if args.one_lane_per_neuron else 3)
     if args.region_map:
         measure_region_map(args, torch, dev)
         return

@@ -67,8 +67,10 @@ template <> __device__ __forceinline__ void lane_put<4>(f32x4 &v, int e, float x
 //     block-uniform base (SGPR pair inside a buffer resource)  +  step * neurons * 4 (SGPR)
 //                                                              +  lane offset (one VGPR, loop-invariant)
 // which is exactly what a buffer instruction adds up by itself, so no access needs vector
-// arithmetic or 64-bit address registers.  num_records is set to the maximum: every access is
-// guarded by the code, not by the hardware range check.
+// arithmetic or 64-bit address registers.  The one-lane backward kernel guards every access by code
+// and sets num_records to the maximum; the forward, the leaky and the split backward kernels give
+// every resource its end and let the hardware's range check drop what lanes and steps past the end
+// of the layer ask for (BEYOND below), so that no branch surrounds a load or a store.
 typedef __amdgpu_buffer_rsrc_t Rsrc;
 // Cache hint of the streamed accesses (bit 1 = non-temporal).  Streaming data that nobody reads twice
 // is marked non-temporal, which measures a few percent faster; but when a step's neurons do not start
