@@ -203,11 +203,12 @@ layer_lif_backward(
 // surrogate evaluated in the kernel, no gradients on state records and at most SPLIT_PLAIN_CHUNKS chunks, and no others,
 // 3: whenever the kernel applies
 std::atomic<int> split_mode{1};
-// batch * neurons up to which mode 1 splits.  The split kernel does half as much again and more in arithmetic and holds
-// fewer waves, so it loses once the one-lane kernel has a wave for every SIMD.  One lane / split, us, without and with
-// synapse: 16 384 neurons, 64 steps 12.7 / 8.9 and 13.9 / 10.6, 300 steps 51 / 26 and 56 / 31, 2000 steps 301 / 176 and
-// 321 / 189; 32 768 neurons 12.7 / 11.3 and 14.0 / 13.1, 54 / 48 and 57 / 57, 318 / 317 and 338 / 360; 65 536 neurons
-// 13.6 / 14.7 and 15 / 17, 63 / 86 and 66 / 104, 343 / 632 and 360 / 709.
+// batch * neurons up to which mode 1 splits: the most at which no form of the call loses by it.  The split kernel does half
+// as much again and more in arithmetic and holds fewer waves.  One lane / split, us, at 16 384 neurons (8, t, 2048), without
+// synapse, with one, with one and state records, with a surrogate tensor: 64 steps 11.0 / 8.1, 12.8 / 9.5, 14.8 / 12.2,
+// 12.7 / 8.0; 300 steps 47.9 / 21.5, 54.6 / 25.4, 60 / 42, 52.8 / 23.3; 2000 steps 287 / 97, 322 / 113, 410 / 210, 317 / 135.
+// At 32 768 neurons: 12.0 / 10.1, 13.9 / 12.3, 17.6 / 21.7, 13.4 / 10.3; 51 / 37, 57 / 45, 64 / 76, 58 / 39; 302 / 183,
+// 337 / 212, 434 / 410, 343 / 255.
 constexpr int64_t SPLIT_MOST_NEURONS = 16384;
 constexpr int64_t SPLIT_PLAIN_CHUNKS = 16;
 
