@@ -28,11 +28,11 @@ namespace {
 // `stops` has it end at a clamped step as the walk does.
 //
 // What bounds it: the chain of 3 x 32 steps per group and one trip to memory and back, 9-11 us for up to 32 chunks on an
-// otherwise idle machine ((8, 100, 256) 14.5 -> 9.4 us, (64, 300, 10) 16.8 -> 11.0 against the kernel that carried two
-// numbers through one walk and needed twice the lanes' registers; (4, 2000, 512) with synapses 302 -> 40 us against one
-// lane per neuron).  512 lanes per block leave 256 registers per lane, which hold the four values of 32 steps.  Sums of a
-// neuron's gradients are fp32 over 8 steps and fp64 beyond: against float64 their error is 0.7 to 0.8 times the one-lane
-// kernel's, that of grad_x the same.
+// otherwise idle machine ((32, 100, 512) 15.6 -> 9.8 us, (64, 300, 10) 16.1 -> 10.1 against a kernel that carried two numbers
+// through one walk, with up to 1024 lanes of 128 registers; (4, 2000, 512) with synapses 302 -> 41 us against one lane per
+// neuron).  512 lanes per block leave 256 registers per lane: the four values of 32 steps and all but 12 to 28 bytes of the
+// rest, 132 to 156 with a synapse and state records, go into them.  Sums of a neuron's gradients are fp32 over 8 steps and
+// fp64 beyond: against float64 their error is 0.7 to 0.8 times the one-lane kernel's, that of grad_x the same.
 constexpr int SPLIT_LANES = 512;
 constexpr int SPLIT_CHUNKS = 32;           // most chunks of a group
 constexpr int SPLIT_NEURONS = 64;          // most neurons of a block
