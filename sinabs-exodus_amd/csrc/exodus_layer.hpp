@@ -255,12 +255,6 @@ __device__ __forceinline__ float reset_amount(float v, const Neuron &n, const Ca
     return taken;
 }
 
-// Neurons per lane of the kernels that support several.  Wider lanes mean wider memory accesses
-// but fewer lanes: stay at the widest width that still gives every compute unit `waves_per_cu`
-// waves, so that small layers are not starved of parallelism (the spiking forward kernel has a long
-// dependent chain per step and wants 16 (with 16 / with 8, in us: (64, 300, 12544) 396 / 418, (16, 500, 49152) 588 / 613,
-// (8, 1000, 66560) 861 / 954); the leaky kernels measure best from 8 on.  `align` is the
-// common alignment (bytes) of all (batch, time, neurons) pointers involved.
 // compute units of the current device, asked for once per device
 inline int compute_units()
 {
@@ -274,16 +268,37 @@ inline int compute_units()
     return cus;
 }
 
-inline int pick_neurons_per_lane(int64_t batch, int64_t neurons, unsigned align, int widest, int waves_per_cu)
+// Neurons per lane of the kernels that support several.  Wider lanes mean wider memory accesses but fewer lanes.
+//   two: from `waves_per_cu` waves per compute unit on.  The spiking forward has a long dependent chain per step and wants 16
+//        (with 16 / with 8, us: (16, 500, 49152) 588 / 613, (8, 1000, 66560) 861 / 954); the leaky kernels measure best from 8 on.
+//   four: only where so many waves are left that memory is all that counts.  Two / four per lane, us, spiking and leaky
+//        forward: 1 M neurons (32, 200, 32768) 319 / 333 and 299 / 314, with synapses (16, 1000, 65536) 1606 / 1624;
+//        2 M (64, 300, 32768) 927 / 960 and 906 / 962; 4 M (32, 300, 131072) 1906 / 1868 and 1870 / 1870.  Where steps do not
+//        fill whole sectors (`whole` false) neighbouring blocks share them, wider blocks share fewer, and four pay sooner:
+//        1.1 M (64, 300, 17000) 584 / 602 and 563 / 576, 2 M (32, 400, 65528) 1452 / 1436 and 1416 / 1398.
+// Where steps fill whole sectors a wider lane is taken only if its blocks spread over the compute units about as evenly as those
+// of one neuron per lane: `even` is the share of lanes that have work while the units that got one block more than the others
+// finish it (and that lie inside the layer).  Memory-bound blocks advance at one pace, so the other units stand idle by then.
+// One / two, us, spiking and leaky forward, leaky backward: (64, 300, 12544), even 0.94 / 0.88, 375 / 394, 355 / 374 and
+// 550 / 566; (40, 250, 11008), 0.96 / 0.89, 176 / 176, 163 / 174 and 252 / 263; where both are even (64, 300, 8192) 227 / 219,
+// 211 / 204 and 322 / 314.  With shared sectors two stay ahead: (64, 300, 17000) 631 / 584.
+// `align` is the common alignment (bytes) of all (batch, time, neurons) pointers involved.
+inline int pick_neurons_per_lane(int64_t batch, int64_t neurons, unsigned align, int widest, int waves_per_cu, bool whole)
 {
     const int cus = compute_units();
-    const int64_t wanted_lanes = static_cast<int64_t>(cus) * waves_per_cu * WAVE;
     const int64_t n = batch * neurons;
 #ifdef EXODUS_FORCE_NPL
     if (EXODUS_FORCE_NPL <= widest) widest = EXODUS_FORCE_NPL;
 #endif
-    if (widest >= 4 && (neurons % 4) == 0 && (align % 16) == 0 && n / 4 >= wanted_lanes) return 4;
-    if (widest >= 2 && (neurons % 2) == 0 && (align % 8) == 0 && n / 2 >= wanted_lanes) return 2;
+    const auto even = [&](int npl) {
+        const int64_t blocks = batch * ((neurons + BLOCK * npl - 1) / (BLOCK * npl)), rounds = (blocks + cus - 1) / cus;
+        return static_cast<double>(n) / (static_cast<double>(rounds) * cus * BLOCK * npl);
+    };
+    for (int npl = widest; npl > 1; npl /= 2) {
+        const int64_t lanes = static_cast<int64_t>(cus) * WAVE * (npl == 2 ? waves_per_cu : (whole ? 64 : 24));
+        if (neurons % npl == 0 && align % (4u * npl) == 0 && n / npl >= lanes && (!whole || even(npl) >= even(1) - 0.03))
+            return npl;
+    }
     return 1;
 }
 
