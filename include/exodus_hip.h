@@ -40,6 +40,13 @@ const char *exodus_hip_error_string(int status);
 #define EXODUS_ERROR_REGIONS_NOT_FOUND (-3)
 #define EXODUS_ERROR_RANGE_IN_USE (-4)
 
+/* The range checks of a forward call's parameters, n values each (NULL = not checked): flags[0] becomes 1 if a value of alpha
+ * or alpha_other lies outside [0, 1], flags[1] if a theta does not exceed its theta_low; nothing else is written, so the caller
+ * clears both.  flags may lie in page-locked host memory.  The reference asks torch and waits for the device in every call
+ * (reference sinabs/exodus/spike.py:183-191). */
+int exodus_check_parameters(int *flags, const float *alpha, const float *alpha_other, const float *theta,
+                            const float *theta_low, int64_t n, void *stream);
+
 /* ---------------------------------------------------------------------------------------------
  * One-to-one counterparts of the reference bindings
  * ------------------------------------------------------------------------------------------- */

@@ -33,6 +33,7 @@ _f = ctypes.c_float
 _SIGNATURES = {
     "exodus_hip_abi_version": ([], _int),
     "exodus_hip_error_string": ([_int], ctypes.c_char_p),
+    "exodus_check_parameters": ([_p] * 5 + [_i64, _p], _int),
     "exodus_lif_forward": ([_p] * 8 + [_int, _int, _i64, _i64, _p], _int),
     "exodus_lif_backward": ([_p] * 6 + [_i64, _i64, _p], _int),
     "exodus_lif_backward_alpha": ([_p] * 8 + [_int, _i64, _i64, _p], _int),
@@ -151,6 +152,15 @@ def _on_device_of(device: torch.device):
     """Device guard for a launch: ``device`` becomes current for the call -- which it nearly always is already, and
     then nothing needs switching."""
     return _NO_GUARD if torch.cuda.current_device() == device.index else torch.cuda.device(device)
+
+
+def checkParameters(flags, alpha, alphaOther, theta, thetaLow) -> None:
+    """Sets flags[0] where a decay factor lies outside [0, 1] and flags[1] where a threshold does not exceed its lower bound;
+    the vectors (or None) have one length.  ``flags`` is a pinned int32 host tensor: read it once the stream has got here."""
+    first = alpha if alpha is not None else thetaLow
+    with _on_device_of(first.device):
+        _check(lib.exodus_check_parameters(_ptr(flags), _ptr(alpha), _ptr(alphaOther), _ptr(theta), _ptr(thetaLow),
+                                           first.numel(), _stream(first)), "exodus_check_parameters")
 
 
 # ------------------------------------------------------------------------------------------

@@ -74,17 +74,19 @@ class SpikingLayerFunction(torch.autograd.Function):
             alpha_syn, tau_syn = _hip.decayExpand(tau_syn, inp.shape[0], inp.shape[2])
         syn = alpha_syn is not None
         apply_min = min_v_mem is not None
-        if check_values:
-            check_parameters([alpha_mem, alpha_syn] if syn else [alpha_mem], threshold, min_v_mem)
-
         max_spikes = -1 if max_num_spikes_per_bin is None else int(max_num_spikes_per_bin)
+        check = check_parameters([alpha_mem, alpha_syn] if syn else [alpha_mem], threshold, min_v_mem, wait=False) if check_values else None
         need_grad = any(ctx.needs_input_grad)
-        res = _hip.layerLifForward(
-            inp, v_mem_init, i_syn_init, alpha_mem, alpha_syn, membrane_subtract, threshold, min_v_mem, apply_min,
-            max_spikes, decay_early, norm_input, wantCheckpoints=need_grad, stateShape=state_shape,
-            wantPreReset=need_grad and kind == _hip.SURR_TENSOR and not record_states,
-            wantRecords=bool(record_states),
-        )
+        try:
+            res = _hip.layerLifForward(
+                inp, v_mem_init, i_syn_init, alpha_mem, alpha_syn, membrane_subtract, threshold, min_v_mem, apply_min,
+                max_spikes, decay_early, norm_input, wantCheckpoints=need_grad, stateShape=state_shape,
+                wantPreReset=need_grad and kind == _hip.SURR_TENSOR and not record_states,
+                wantRecords=bool(record_states),
+            )
+        finally:
+            if check is not None:
+                check.finish()
         ctx.cfg = (syn, apply_min, max_spikes, bool(decay_early), bool(norm_input), kind, p0, p1)
         ctx.surrogate_grad_fn = surrogate_grad_fn if kind == _hip.SURR_TENSOR else None
         ctx.set_materialize_grads(False)

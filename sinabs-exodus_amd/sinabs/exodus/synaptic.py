@@ -52,13 +52,15 @@ class SynapticIntegrateAndFire(torch.autograd.Function):
         check_per_row(alpha_syn=alpha_syn, alpha_mem=alpha_mem, i_syn_init=i_syn_init, v_mem_init=v_mem_init,
                       threshold=threshold, membrane_subtract=membrane_subtract, min_v_mem=min_v_mem)
         apply_min = min_v_mem is not None
-        check_parameters([alpha_mem, alpha_syn], threshold, min_v_mem)
-
-        max_spikes = -1 if max_num_spikes_per_bin is None else int(max_num_spikes_per_bin)
-        spikes, v_mem, i_syn = _hip.synLifForward(
-            inp, v_mem_init, i_syn_init, alpha_mem, alpha_syn, membrane_subtract, threshold, min_v_mem,
-            apply_min, max_spikes, decay_early, norm_input,
-        )
+        check = check_parameters([alpha_mem, alpha_syn], threshold, min_v_mem, wait=False)
+        try:
+            max_spikes = -1 if max_num_spikes_per_bin is None else int(max_num_spikes_per_bin)
+            spikes, v_mem, i_syn = _hip.synLifForward(
+                inp, v_mem_init, i_syn_init, alpha_mem, alpha_syn, membrane_subtract, threshold, min_v_mem,
+                apply_min, max_spikes, decay_early, norm_input,
+            )
+        finally:
+            check.finish()
         ctx.cfg = (apply_min, max_spikes, bool(decay_early), bool(norm_input), kind, p0, p1)
         ctx.set_materialize_grads(False)
         saved = [v_mem, i_syn, v_mem_init, i_syn_init, alpha_mem, alpha_syn, membrane_subtract, threshold]
