@@ -1,7 +1,8 @@
 """Build libexodus_hip.so for gfx950 with hipcc (cross-compiles without a GPU).
 
 Usage:  python build_hip.py
-The library lands next to the Python loader (sinabs/exodus/libexodus_hip.so).  A second, small
+The library lands next to the Python loader (sinabs/exodus/libexodus_hip.so), and beside it the host side of its calls
+(sinabs/exodus/_exodus_torch.so, plain C++ compiled against the installed torch).  A third, small
 library with the streaming probes that only bench.py uses (libexodus_bench_probes.so, next to this
 script) is built in the same go; it is not part of the product.
 """
@@ -17,6 +18,9 @@ SRCS = [os.path.join(HERE, "csrc", f) for f in ("exodus_hip.hip", "exodus_layer.
 SRC = SRCS[0]
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 OUT = os.path.join(HERE, "sinabs", "exodus", "libexodus_hip.so")
+# the host side of the calls (C++ against the installed torch), next to the Python loader
+TORCH_SRC = os.path.join(HERE, "csrc", "exodus_torch.cpp")
+TORCH_OUT = os.path.join(HERE, "sinabs", "exodus", "_exodus_torch.so")
 PROBE_SRC = os.path.join(HERE, "csrc", "bench_probes.hip")
 PROBE_OUT = os.path.join(HERE, "libexodus_bench_probes.so")
 
@@ -29,10 +33,26 @@ FLAGS = [
 ]
 
 
+def _torch_command(out: str) -> list:
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(shutil.which("hipcc") or "/opt/rocm/bin/hipcc")))
+    command = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+               "-DUSE_ROCM"]
+    for path in cpp_extension.include_paths() + [sysconfig.get_paths()["include"], os.path.join(rocm, "include")]:
+        command += ["-isystem", path]
+    command += ["-I", INCLUDE, TORCH_SRC, "-o", out]
+    command += ["-L" + path for path in cpp_extension.library_paths()]
+    return command + ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+
+
 def build(force: bool = True) -> str:
-    deps = SRCS + [PROBE_SRC, os.path.join(HERE, "csrc", "exodus_common.hpp"), os.path.join(HERE, "csrc", "exodus_layer.hpp"), os.path.join(INCLUDE, "exodus_hip.h")]
-    if (not force and os.path.exists(OUT) and os.path.exists(PROBE_OUT)
-            and min(os.path.getmtime(OUT), os.path.getmtime(PROBE_OUT)) >= max(os.path.getmtime(d) for d in deps)):
+    deps = SRCS + [PROBE_SRC, TORCH_SRC, os.path.join(HERE, "csrc", "exodus_common.hpp"), os.path.join(HERE, "csrc", "exodus_layer.hpp"), os.path.join(INCLUDE, "exodus_hip.h")]
+    outs = (OUT, PROBE_OUT, TORCH_OUT)
+    if (not force and all(os.path.exists(o) for o in outs)
+            and min(os.path.getmtime(o) for o in outs) >= max(os.path.getmtime(d) for d in deps)):
         return OUT
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     # hipcc's host pass does not know the gfx-only target feature and says so; that line is harmless
@@ -48,11 +68,13 @@ def build(force: bool = True) -> str:
         # the bench-only probes: one small translation unit, compiled and linked in one step
         procs.append(subprocess.Popen([hipcc] + FLAGS + ["-I", INCLUDE, PROBE_SRC, "-o", PROBE_OUT + ".tmp"],
                                       stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True))
+        procs.append(subprocess.Popen(_torch_command(TORCH_OUT + ".tmp"), stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                                      text=True))
         outputs = [proc.communicate()[0] for proc in procs]
         log = "\n".join(filter(None, (quiet(o).strip() for o in outputs)))
         if any(proc.returncode != 0 for proc in procs):
             sys.stderr.write(log + "\n")
-            raise RuntimeError("hipcc failed compiling libexodus_hip.so / libexodus_bench_probes.so")
+            raise RuntimeError("hipcc failed compiling libexodus_hip.so / libexodus_bench_probes.so / _exodus_torch.so")
         link = subprocess.run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", OUT + ".tmp"] + objs,
                               stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
         log = "\n".join(filter(None, (log, quiet(link.stdout).strip())))
@@ -63,6 +85,7 @@ def build(force: bool = True) -> str:
         sys.stderr.write(log + "\n")
     os.replace(OUT + ".tmp", OUT)
     os.replace(PROBE_OUT + ".tmp", PROBE_OUT)
+    os.replace(TORCH_OUT + ".tmp", TORCH_OUT)
     return OUT
 
 

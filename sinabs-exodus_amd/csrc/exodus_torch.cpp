@@ -1,0 +1,532 @@
+// The host side of the kernel calls in native code: what a call checks, allocates and hands to the C ABI of
+// libexodus_hip.so, between the Python wrappers of _hip.py and the library.  No device code and no state: the library's
+// entry points are bound once at import (bind), the current stream and device are asked for in every call.
+//
+// Why it exists: a training step of a small layer is host time, and the autograd engine runs the backward pass on a thread
+// of its own, where the 55 us of Python and ctypes that a backward pass was took up to 165 (caches and a core of its own).
+// Python and ctypes / these, us per step through the layer, forward and backward: IAF (8, 100, 256) 238 / 149, LIF
+// (32, 100, 512) with a trained time constant 271 / 173, a streamed chunk (1, 10, 1024) without gradients 46 / 27.
+#include <ATen/Functions.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <pybind11/pybind11.h>
+#include <pybind11/stl.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <optional>
+#include <stdexcept>
+#include <string>
+#include <vector>
+
+#include "exodus_hip.h"
+
+namespace py = pybind11;
+
+namespace {
+
+using at::Tensor;
+using Maybe = std::optional<Tensor>;
+using Shape = std::vector<int64_t>;
+
+// ---------------------------------------------------------------------------------------------
+// the library
+// ---------------------------------------------------------------------------------------------
+#define EXODUS_ENTRIES(X)                                                                                               \
+    X(exodus_lif_forward) X(exodus_lif_backward_fused) X(exodus_leaky_forward) X(exodus_leaky_backward_fused)           \
+    X(exodus_layer_sum_slots) X(exodus_layer_checkpoint_interval) X(exodus_layer_lif_forward_total)                     \
+    X(exodus_layer_lif_backward) X(exodus_layer_lif_backward_from_input) X(exodus_layer_leaky_forward_total)            \
+    X(exodus_layer_leaky_backward) X(exodus_decay_expand) X(exodus_decay_work) X(exodus_decay_grad)
+struct Library {
+#define EXODUS_MEMBER(name) decltype(&::name) name = nullptr;
+    EXODUS_ENTRIES(EXODUS_MEMBER)
+#undef EXODUS_MEMBER
+};
+Library lib;
+int64_t interval = 0;                                          // steps between checkpoints
+PyObject *raise_status = nullptr;                              // (status, what): raises for a status other than 0
+
+void bind(const py::dict &addresses, const py::object &on_status)
+{
+#define EXODUS_BIND(name) \
+    lib.name = reinterpret_cast<decltype(lib.name)>(py::cast<uintptr_t>(addresses[#name]));
+    EXODUS_ENTRIES(EXODUS_BIND)
+#undef EXODUS_BIND
+    interval = lib.exodus_layer_checkpoint_interval();
+    Py_XDECREF(raise_status);
+    raise_status = py::object(on_status).release().ptr();
+}
+
+// call a function of the library on the tensor's device and stream, without the interpreter lock
+template <class F>
+void launch(const Tensor &like, const char *what, F &&call)
+{
+    int status;
+    {
+        py::gil_scoped_release unlocked;
+        const c10::DeviceGuard guard(like.device());
+        status = call(static_cast<void *>(c10::hip::getCurrentHIPStream(like.device().index()).stream()));
+    }
+    if (status != 0) py::reinterpret_borrow<py::object>(raise_status)(status, what);
+}
+
+// ---------------------------------------------------------------------------------------------
+// checks
+// ---------------------------------------------------------------------------------------------
+std::string text(c10::IntArrayRef sizes)
+{
+    std::string s = "(";
+    for (size_t i = 0; i < sizes.size(); ++i) s += (i ? ", " : "") + std::to_string(sizes[i]);
+    return s + (sizes.size() == 1 ? ",)" : ")");
+}
+
+[[noreturn]] void refuse(const std::string &why) { throw std::runtime_error(why); }
+
+const Tensor &dev(const Tensor &x, const char *name, const Tensor *like = nullptr)
+{
+    if (!x.is_cuda())
+        refuse(std::string(name) + " must be a tensor on a HIP device (got " + x.device().str() + "); there is no CPU path");
+    if (x.scalar_type() != at::kFloat)
+        refuse(std::string(name) + " must be float32 (got " + c10::toString(x.scalar_type()) + ")");
+    if (!x.is_contiguous()) refuse(std::string(name) + " must be contiguous");
+    if (like && x.device() != like->device()) refuse(std::string(name) + " and the first tensor must be on the same device");
+    return x;
+}
+
+const float *rows(const Tensor &x, const char *name, const Tensor &like, int64_t n)
+{
+    dev(x, name, &like);
+    if (x.dim() != 1 || x.size(0) != n)
+        refuse(std::string(name) + " must have shape (" + std::to_string(n) + ",), got " + text(x.sizes()));
+    return x.const_data_ptr<float>();
+}
+
+const Tensor &present(const Maybe &x, const char *name)
+{
+    if (!x || !x->defined()) throw py::type_error(std::string(name) + " must be a tensor");
+    return *x;
+}
+
+const float *rows(const Maybe &x, const char *name, const Tensor &like, int64_t n)
+{
+    return rows(present(x, name), name, like, n);
+}
+
+const float *same(const Tensor &x, const char *name, const Tensor &like, const char *as)
+{
+    dev(x, name, &like);
+    if (x.sizes() != like.sizes()) refuse(std::string(name) + " must have the shape of " + as);
+    return x.const_data_ptr<float>();
+}
+
+const float *matrix(const Tensor &x, const char *name, const Tensor &like, int64_t n, int64_t t)
+{
+    dev(x, name, &like);
+    if (x.dim() != 2 || x.size(0) != n || x.size(1) != t)
+        refuse(std::string(name) + " must have shape (" + std::to_string(n) + ", " + std::to_string(t) + "), got " +
+               text(x.sizes()));
+    return x.const_data_ptr<float>();
+}
+
+const Tensor &three(const Tensor &x, const char *name, const Tensor *like = nullptr)
+{
+    dev(x, name, like);
+    if (x.dim() != 3) refuse(std::string(name) + " must be 3-D (batch, time, neurons)");
+    return x;
+}
+
+const Tensor &two(const Tensor &x, const char *name)
+{
+    dev(x, name);
+    if (x.dim() != 2) refuse(std::string(name) + " must be 2-D (rows, time)");
+    return x;
+}
+
+bool has(const Maybe &x) { return x && x->defined(); }
+float *out(const Tensor &x) { return x.defined() ? x.mutable_data_ptr<float>() : nullptr; }
+double *out64(const Tensor &x) { return x.defined() ? x.mutable_data_ptr<double>() : nullptr; }
+
+// ---------------------------------------------------------------------------------------------
+// memory
+// ---------------------------------------------------------------------------------------------
+Tensor fresh(c10::IntArrayRef shape, const Tensor &like, at::ScalarType type = at::kFloat)
+{
+    return at::empty(shape, at::TensorOptions().device(like.device()).dtype(type));
+}
+
+// the (batch, time, neurons) and (rows, time) results: `place`, if given, allocates them (shape, like)
+Tensor large(c10::IntArrayRef shape, const Tensor &like, const py::object &place)
+{
+    if (place.is_none()) return fresh(shape, like);
+    return py::cast<Tensor>(place(py::cast(Shape(shape.begin(), shape.end())), like));
+}
+
+int64_t elements(const Shape &shape)
+{
+    int64_t n = 1;
+    for (int64_t s : shape) n *= s;
+    return n;
+}
+
+// a float64 scalar for the sum of a forward call's outputs and the memory the kernels add it up in; both are written by the
+// call (which launches nothing, and leaves the total as it is, when there is nothing to walk)
+void total_and_work(const Tensor &input, Tensor &total, Tensor &work)
+{
+    if (input.numel() == 0) {
+        total = at::zeros({}, at::TensorOptions().device(input.device()).dtype(at::kDouble));
+        return;
+    }
+    total = fresh({}, input, at::kDouble);
+    work = fresh({lib.exodus_layer_sum_slots(input.size(0), input.size(2))}, input, at::kDouble);
+}
+
+Shape state_shape_of(const std::optional<Shape> &asked, int64_t n)
+{
+    if (!asked) return {n};
+    if (elements(*asked) != n)
+        refuse("stateShape " + text(*asked) + " does not hold " + std::to_string(n) + " neurons");
+    return *asked;
+}
+
+// ---------------------------------------------------------------------------------------------
+// layers on (batch, time, neurons)
+// ---------------------------------------------------------------------------------------------
+py::tuple layer_lif_forward(const Tensor &input, const Tensor &v_init, const Maybe &i_init, const Tensor &alpha_mem,
+                            const Maybe &alpha_syn, const Tensor &subtract, const Tensor &theta, const Maybe &theta_low,
+                            bool apply_low, int64_t max_spikes, bool decay_early, bool norm_input, bool want_checkpoints,
+                            bool want_records, bool want_pre_reset, bool want_sum, const Maybe &out_spikes,
+                            const std::optional<Shape> &state_shape, const py::object &place)
+{
+    if (want_records && want_pre_reset) refuse("wantRecords and wantPreReset exclude each other");
+    three(input, "input");
+    const int64_t b = input.size(0), t = input.size(1), m = input.size(2), n = b * m;
+    const bool syn = has(alpha_syn);
+    const float *v0 = rows(v_init, "vmemPostInitial", input, n), *am = rows(alpha_mem, "alphaMem", input, n);
+    const float *c = rows(subtract, "membrSubtract", input, n), *th = rows(theta, "theta", input, n);
+    const float *i0 = syn ? rows(i_init, "isynInitial", input, n) : nullptr;
+    const float *as = syn ? rows(alpha_syn, "alphaSyn", input, n) : nullptr;
+    const float *lo = apply_low ? rows(theta_low, "thetaLow", input, n) : nullptr;
+    const Shape shape{b, t, m}, states = state_shape_of(state_shape, n), kept{b, (t + interval - 1) / interval, m};
+    Tensor spikes = has(out_spikes) ? *out_spikes : large(shape, input, place);
+    if (spikes.sizes() != input.sizes()) refuse("outSpikes must have the shape of input");
+    dev(spikes, "outSpikes", &input);
+    const Tensor v_last = fresh(states, input), i_last = syn ? fresh(states, input) : Tensor();
+    const Tensor ckpt_v = want_checkpoints ? large(kept, input, place) : Tensor();
+    const Tensor ckpt_i = want_checkpoints && syn ? large(kept, input, place) : Tensor();
+    const Tensor v_rec = want_records || want_pre_reset ? large(shape, input, place) : Tensor();
+    const Tensor i_rec = want_records && syn ? large(shape, input, place) : Tensor();
+    Tensor total, work;
+    if (want_sum) total_and_work(input, total, work);
+    if (t == 0) {                                              // nothing to integrate: the final states are the initial ones
+        v_last.copy_(v_init.reshape(states));
+        if (syn) i_last.copy_(i_init->reshape(states));
+    }
+    launch(input, "exodus_layer_lif_forward_total", [&](void *stream) {
+        return lib.exodus_layer_lif_forward_total(
+            out(spikes), out(v_rec), out(i_rec), out(ckpt_v), out(ckpt_i), out(v_last), out(i_last), out64(total), out64(work),
+            input.const_data_ptr<float>(), v0, i0, am, as, c, th, lo, apply_low, static_cast<int>(max_spikes), decay_early,
+            norm_input, want_pre_reset, b, t, m, stream);
+    });
+    return py::make_tuple(spikes, v_last, i_last, ckpt_v, ckpt_i, v_rec, i_rec, total);
+}
+
+// -> (grad_input, alpha_mem, alpha_syn, v_init, i_init)
+py::tuple layer_lif_backward(const Tensor &grad_spikes, const Maybe &grad_v_last, const Maybe &grad_i_last, const Tensor &input,
+                             const Maybe &ckpt_v, const Maybe &ckpt_i, const Maybe &v_init, const Maybe &i_init,
+                             const Tensor &alpha_mem, const Maybe &alpha_syn, const Tensor &subtract, const Tensor &theta,
+                             const Maybe &theta_low, bool apply_low, int64_t max_spikes, bool decay_early, bool norm_input,
+                             int kind, double p0, double p1, const Maybe &grad_input_given, const Maybe &surr_given,
+                             Maybe grad_v_rec, Maybe grad_i_rec, bool want_alpha_mem, bool want_alpha_syn, bool want_v_init,
+                             bool want_i_init, bool uniform, const py::object &place)
+{
+    three(input, "input");
+    const int64_t b = input.size(0), t = input.size(1), m = input.size(2), n = b * m;
+    const bool syn = has(alpha_syn);
+    if (uniform) {
+        if (dev(grad_spikes, "gradSpikes", &input).numel() != 1)
+            refuse("gradSpikes must hold one value when gradUniform is set");
+        if (kind == EXODUS_SURR_TENSOR || has(grad_v_rec) || has(grad_i_rec))
+            refuse("gradUniform needs an in-kernel surrogate and no gradients on the state records");
+    } else {
+        same(three(grad_spikes, "gradSpikes", &input), "gradSpikes", input, "input");
+    }
+    const bool from_input = !has(ckpt_v);
+    const Shape shape{b, t, m}, kept{b, (t + interval - 1) / interval, m};
+    const auto checkpoint = [&](const Maybe &x, const char *name) {
+        if (three(present(x, name), name, &input).sizes() != c10::IntArrayRef(kept))
+            refuse(std::string(name) + " must have shape " + text(kept));
+        return x->const_data_ptr<float>();
+    };
+    const float *cv = from_input ? nullptr : checkpoint(ckpt_v, "ckptV");
+    const float *ci = from_input || !syn ? nullptr : checkpoint(ckpt_i, "ckptI");
+    const float *v0 = rows(v_init, "vmemPostInitial", input, n), *am = rows(alpha_mem, "alphaMem", input, n);
+    const float *c = rows(subtract, "membrSubtract", input, n), *th = rows(theta, "theta", input, n);
+    const float *i0 = syn ? rows(i_init, "isynInitial", input, n) : nullptr;
+    const float *as = syn ? rows(alpha_syn, "alphaSyn", input, n) : nullptr;
+    const auto last = [&](const Maybe &x, const char *name) -> const float * {
+        if (!has(x)) return nullptr;
+        if (dev(*x, name, &input).numel() != n) refuse(std::string(name) + " must hold " + std::to_string(n) + " values");
+        return x->const_data_ptr<float>();
+    };
+    const float *gvl = last(grad_v_last, "gradVLast"), *gil = syn ? last(grad_i_last, "gradILast") : nullptr;
+    const float *lo = apply_low ? rows(theta_low, "thetaLow", input, n) : nullptr;
+    if (has(grad_input_given)) same(three(*grad_input_given, "gradInput", &input), "gradInput", input, "input");
+    const Tensor grad_input = has(grad_input_given) ? *grad_input_given : large(shape, input, place);
+    const float *surr = nullptr;
+    if (kind == EXODUS_SURR_TENSOR) {
+        if (!has(surr_given)) refuse("surr must be given with the shape of input");
+        if (three(*surr_given, "surr", &input).sizes() != input.sizes()) refuse("surr must be given with the shape of input");
+        surr = surr_given->const_data_ptr<float>();
+    }
+    if (!syn) grad_i_rec.reset();
+    const float *gvr = nullptr, *gir = nullptr;
+    if (has(grad_v_rec) || has(grad_i_rec)) {                  // one that is missing while the other is given counts as zero
+        if (!has(grad_v_rec)) grad_v_rec = at::zeros_like(input);
+        if (syn && !has(grad_i_rec)) grad_i_rec = at::zeros_like(input);
+        gvr = same(three(*grad_v_rec, "gradVRec", &input), "gradVRec", input, "input");
+        if (syn) gir = same(three(*grad_i_rec, "gradIRec", &input), "gradIRec", input, "input");
+    }
+    // the kernel writes every neuron's entry of each vector it is given -- unless there is no step to walk: then nothing is
+    // launched, the decay factors have no influence and a gradient on a final state is the gradient of the initial state it
+    // equals (the wanted vectors are rows of one allocation)
+    const bool wanted[4] = {want_alpha_mem, want_v_init, syn && want_alpha_syn, syn && want_i_init};
+    const int64_t many = wanted[0] + wanted[1] + wanted[2] + wanted[3];
+    Tensor block, vectors[4];
+    if (many) {
+        block = t == 0 ? at::zeros({many, n}, input.options()) : fresh({many, n}, input);
+        for (int64_t k = 0, at = 0; k < 4; ++k)
+            if (wanted[k]) vectors[k] = block.select(0, at++);
+    }
+    const Tensor &am_g = vectors[0], &v0_g = vectors[1], &as_g = vectors[2], &i0_g = vectors[3];
+    if (t == 0) {
+        if (v0_g.defined() && gvl) v0_g.copy_(grad_v_last->reshape({-1}));
+        if (i0_g.defined() && gil) i0_g.copy_(grad_i_last->reshape({-1}));
+    }
+    const float *x = input.const_data_ptr<float>(), *gs = grad_spikes.const_data_ptr<float>();
+    const int spikes = static_cast<int>(max_spikes);
+    const float f0 = static_cast<float>(p0), f1 = static_cast<float>(p1);
+    if (from_input)
+        launch(input, "exodus_layer_lif_backward_from_input", [&](void *stream) {
+            return lib.exodus_layer_lif_backward_from_input(
+                out(grad_input), out(am_g), out(as_g), out(v0_g), out(i0_g), gs, gvl, gil, x, v0, i0, am, as, c, th, lo,
+                apply_low, spikes, decay_early, norm_input, kind, f0, f1, surr, gvr, gir, uniform, b, t, m, stream);
+        });
+    else
+        launch(input, "exodus_layer_lif_backward", [&](void *stream) {
+            return lib.exodus_layer_lif_backward(
+                out(grad_input), out(am_g), out(as_g), out(v0_g), out(i0_g), gs, gvl, gil, x, cv, ci, v0, i0, am, as, c, th, lo,
+                apply_low, spikes, decay_early, norm_input, kind, f0, f1, surr, gvr, gir, uniform, b, t, m, stream);
+        });
+    return py::make_tuple(grad_input, am_g, as_g, v0_g, i0_g);
+}
+
+// -> (out, v_last, total)
+py::tuple layer_leaky_forward(const Tensor &input, const Tensor &v_init, const Tensor &alpha, bool decay_early, bool norm_input,
+                              const std::optional<Shape> &state_shape, bool want_sum, const py::object &place)
+{
+    three(input, "input");
+    const int64_t b = input.size(0), t = input.size(1), m = input.size(2), n = b * m;
+    const float *v0 = rows(v_init, "vmemInitial", input, n), *a = rows(alpha, "alpha", input, n);
+    const Shape shape{b, t, m}, states = state_shape_of(state_shape, n);
+    const Tensor result = large(shape, input, place), v_last = fresh(states, input);
+    Tensor total, work;
+    if (want_sum) total_and_work(input, total, work);
+    if (t == 0) v_last.copy_(v_init.reshape(states));
+    launch(input, "exodus_layer_leaky_forward_total", [&](void *stream) {
+        return lib.exodus_layer_leaky_forward_total(out(result), out(v_last), out64(total), out64(work),
+                                                    input.const_data_ptr<float>(), v0, a, decay_early, norm_input, b, t, m,
+                                                    stream);
+    });
+    return py::make_tuple(result, v_last, total);
+}
+
+// -> (grad_input, alpha, v_init)
+py::tuple layer_leaky_backward(const Tensor &grad_out, const Maybe &grad_v_last, const Maybe &forward_out, const Maybe &input,
+                               const Maybe &v_init, const Tensor &alpha, bool decay_early, bool norm_input, bool want_alpha,
+                               const std::optional<Shape> &uniform_shape, const py::object &place)
+{
+    const bool uniform = uniform_shape.has_value();
+    Shape shape;
+    if (uniform) {
+        if (dev(grad_out, "gradOut").numel() != 1) refuse("gradOut must hold one value when shape is given");
+        shape = *uniform_shape;
+        if (shape.size() != 3) throw py::value_error("shape must be (batch, time, neurons)");
+    } else {
+        three(grad_out, "gradOut");
+        shape = grad_out.sizes().vec();
+    }
+    const int64_t b = shape[0], t = shape[1], m = shape[2], n = b * m;
+    const float *a = rows(alpha, "alpha", grad_out, n);
+    const float *gvl = nullptr;
+    if (has(grad_v_last)) {
+        if (dev(*grad_v_last, "gradVLast", &grad_out).numel() != n)
+            refuse("gradVLast must hold " + std::to_string(n) + " values");
+        gvl = grad_v_last->const_data_ptr<float>();
+    }
+    const auto full = [&](const Maybe &x, const char *name) {
+        if (three(present(x, name), name, &grad_out).sizes() != c10::IntArrayRef(shape))
+            refuse(std::string(name) + " must have the shape of gradOut");
+        return x->const_data_ptr<float>();
+    };
+    const float *o = want_alpha ? full(forward_out, "out") : nullptr;
+    const float *v0 = want_alpha ? rows(v_init, "vmemInitial", grad_out, n) : nullptr;
+    const float *x = want_alpha && (decay_early || norm_input) ? full(input, "input") : nullptr;
+    const Tensor grad_input = large(shape, grad_out, place);
+    const int64_t many = want_alpha ? 2 : 1;
+    const Tensor block = t == 0 ? at::zeros({many, n}, grad_out.options()) : fresh({many, n}, grad_out);
+    const Tensor v0_g = block.select(0, 0), a_g = want_alpha ? block.select(0, 1) : Tensor();
+    if (t == 0 && gvl) v0_g.copy_(grad_v_last->reshape({-1}));
+    launch(grad_out, "exodus_layer_leaky_backward", [&](void *stream) {
+        return lib.exodus_layer_leaky_backward(out(grad_input), out(a_g), out(v0_g), grad_out.const_data_ptr<float>(), gvl, o, x,
+                                               v0, a, decay_early, norm_input, uniform, b, t, m, stream);
+    });
+    return py::make_tuple(grad_input, a_g, v0_g);
+}
+
+// -> (alpha, copy of tau)
+py::tuple decay_expand(const Tensor &tau, int64_t batch, int64_t neurons)
+{
+    dev(tau, "tau");
+    const Tensor alpha = fresh({batch * neurons}, tau), kept = fresh(tau.sizes(), tau);
+    launch(tau, "exodus_decay_expand", [&](void *stream) {
+        return lib.exodus_decay_expand(out(alpha), out(kept), tau.const_data_ptr<float>(), batch, neurons, tau.numel(), stream);
+    });
+    return py::make_tuple(alpha, kept);
+}
+
+Tensor decay_grad(const Tensor &grad_alpha, const Tensor &tau, int64_t batch, int64_t neurons)
+{
+    const float *g = rows(grad_alpha, "gradAlpha", dev(tau, "tau"), batch * neurons);
+    if (batch * neurons == 0) return at::zeros_like(tau);
+    const Tensor result = fresh(tau.sizes(), tau);
+    const int64_t wanted = lib.exodus_decay_work(batch, neurons, tau.numel());
+    const Tensor work = wanted ? fresh({wanted}, tau, at::kDouble) : Tensor();
+    launch(tau, "exodus_decay_grad", [&](void *stream) {
+        return lib.exodus_decay_grad(out(result), out64(work), g, tau.const_data_ptr<float>(), batch, neurons, tau.numel(),
+                                     stream);
+    });
+    return result;
+}
+
+// ---------------------------------------------------------------------------------------------
+// what shows that a layer's parameters are the ones of the call before
+// ---------------------------------------------------------------------------------------------
+// per value: a tensor's identity, version, address and shape; anything else as it is
+py::tuple stamps(const py::tuple &values)
+{
+    py::tuple result(values.size());
+    for (size_t k = 0; k < values.size(); ++k) {
+        const py::handle value = values[k];
+        if (THPVariable_Check(value.ptr())) {
+            const Tensor &x = THPVariable_Unpack(value.ptr());
+            py::tuple sizes(x.dim());
+            for (int64_t d = 0; d < x.dim(); ++d) sizes[d] = x.size(d);
+            result[k] = py::make_tuple(reinterpret_cast<uintptr_t>(value.ptr()), x._version(),
+                                       reinterpret_cast<uintptr_t>(x.const_data_ptr()), sizes);
+        } else {
+            result[k] = value;
+        }
+    }
+    return result;
+}
+
+// ---------------------------------------------------------------------------------------------
+// (rows, time) matrices
+// ---------------------------------------------------------------------------------------------
+void lif_forward(const Tensor &spikes, const Tensor &v_mem, const Tensor &input, const Tensor &v_init, const Tensor &alpha,
+                 const Tensor &subtract, const Tensor &theta, const Maybe &theta_low, bool apply_low, int64_t max_spikes)
+{
+    two(input, "input");
+    const int64_t n = input.size(0), t = input.size(1);
+    matrix(spikes, "outputSpikes", input, n, t);
+    matrix(v_mem, "vmem", input, n, t);
+    const float *v0 = rows(v_init, "vmemPostInitial", input, n), *a = rows(alpha, "alpha", input, n);
+    const float *c = rows(subtract, "membrSubtract", input, n), *th = rows(theta, "theta", input, n);
+    const float *lo = apply_low ? rows(theta_low, "thetaLow", input, n) : nullptr;
+    launch(input, "exodus_lif_forward", [&](void *stream) {
+        return lib.exodus_lif_forward(out(spikes), out(v_mem), input.const_data_ptr<float>(), v0, a, c, th, lo, apply_low,
+                                      static_cast<int>(max_spikes), n, t, stream);
+    });
+}
+
+// the per-row gradients of a backward call (every entry is written if there is a step to walk)
+Tensor per_row(const Tensor &alpha, int64_t n, int64_t t)
+{
+    return n == 0 || t == 0 ? at::zeros_like(alpha) : fresh(alpha.sizes(), alpha);
+}
+
+// -> (grad_input, alpha, v_init)
+py::tuple lif_backward_fused(const Tensor &grad_spikes, const Maybe &grad_vmem, const Tensor &v_mem, const Maybe &v_init,
+                             const Tensor &alpha, const Tensor &subtract, const Tensor &theta, const Maybe &theta_low,
+                             bool apply_low, int64_t max_spikes, int kind, double p0, double p1, const Maybe &surr_given,
+                             bool want_alpha, const Maybe &grad_input_given, const py::object &place)
+{
+    two(v_mem, "vmem");
+    const int64_t n = v_mem.size(0), t = v_mem.size(1);
+    const float *gs = matrix(grad_spikes, "gradSpikes", v_mem, n, t);
+    const float *gv = has(grad_vmem) ? matrix(*grad_vmem, "gradVmem", v_mem, n, t) : nullptr;
+    const float *a = rows(alpha, "alpha", v_mem, n), *c = rows(subtract, "membrSubtract", v_mem, n);
+    const float *th = rows(theta, "theta", v_mem, n);
+    const float *lo = apply_low ? rows(theta_low, "thetaLow", v_mem, n) : nullptr;
+    const float *v0 = want_alpha ? rows(v_init, "vmemPostInitial", v_mem, n) : nullptr;
+    const float *surr = kind == EXODUS_SURR_TENSOR ? matrix(present(surr_given, "surr"), "surr", v_mem, n, t) : nullptr;
+    if (has(grad_input_given)) matrix(*grad_input_given, "inputGrad", v_mem, n, t);
+    const Tensor grad_input = has(grad_input_given) ? *grad_input_given : large(v_mem.sizes(), v_mem, place);
+    const Tensor v0_g = per_row(alpha, n, t), a_g = want_alpha ? per_row(alpha, n, t) : Tensor();
+    launch(v_mem, "exodus_lif_backward_fused", [&](void *stream) {
+        return lib.exodus_lif_backward_fused(out(grad_input), out(a_g), out(v0_g), gs, gv, v_mem.const_data_ptr<float>(), surr, v0,
+                                             a, c, th, lo, apply_low, static_cast<int>(max_spikes), kind,
+                                             static_cast<float>(p0), static_cast<float>(p1), n, t, stream);
+    });
+    return py::make_tuple(grad_input, a_g, v0_g);
+}
+
+Tensor leaky_forward(const Tensor &input, const Tensor &v_init, const Tensor &alpha, const Maybe &given, const py::object &place)
+{
+    two(input, "input");
+    const int64_t n = input.size(0), t = input.size(1);
+    const float *v0 = rows(v_init, "vmemInitial", input, n), *a = rows(alpha, "alpha", input, n);
+    if (has(given)) matrix(*given, "output", input, n, t);
+    const Tensor result = has(given) ? *given : large(input.sizes(), input, place);
+    launch(input, "exodus_leaky_forward", [&](void *stream) {
+        return lib.exodus_leaky_forward(out(result), input.const_data_ptr<float>(), v0, a, n, t, stream);
+    });
+    return result;
+}
+
+// -> (grad_input, alpha, v_init)
+py::tuple leaky_backward_fused(const Tensor &grad_out, const Tensor &alpha, const Maybe &forward_out, const Maybe &v_init,
+                               bool want_alpha, const Maybe &grad_input_given, const py::object &place)
+{
+    two(grad_out, "outputGrad");
+    const int64_t n = grad_out.size(0), t = grad_out.size(1);
+    const float *a = rows(alpha, "alpha", grad_out, n);
+    const float *o = want_alpha ? matrix(present(forward_out, "output"), "output", grad_out, n, t) : nullptr;
+    const float *v0 = want_alpha ? rows(v_init, "vmemInitial", grad_out, n) : nullptr;
+    if (has(grad_input_given)) matrix(*grad_input_given, "inputGrad", grad_out, n, t);
+    const Tensor grad_input = has(grad_input_given) ? *grad_input_given : large(grad_out.sizes(), grad_out, place);
+    const Tensor v0_g = per_row(alpha, n, t), a_g = want_alpha ? per_row(alpha, n, t) : Tensor();
+    launch(grad_out, "exodus_leaky_backward_fused", [&](void *stream) {
+        return lib.exodus_leaky_backward_fused(out(grad_input), out(a_g), out(v0_g), grad_out.const_data_ptr<float>(), o, v0, a, n,
+                                               t, stream);
+    });
+    return py::make_tuple(grad_input, a_g, v0_g);
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_exodus_torch, module)
+{
+    module.def("bind", &bind);
+    module.def("layer_lif_forward", &layer_lif_forward);
+    module.def("layer_lif_backward", &layer_lif_backward);
+    module.def("layer_leaky_forward", &layer_leaky_forward);
+    module.def("layer_leaky_backward", &layer_leaky_backward);
+    module.def("stamps", &stamps);
+    module.def("decay_expand", &decay_expand);
+    module.def("decay_grad", &decay_grad);
+    module.def("lif_forward", &lif_forward);
+    module.def("lif_backward_fused", &lif_backward_fused);
+    module.def("leaky_forward", &leaky_forward);
+    module.def("leaky_backward_fused", &leaky_backward_fused);
+}

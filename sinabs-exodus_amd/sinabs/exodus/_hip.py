@@ -89,8 +89,6 @@ def _load() -> ctypes.CDLL:
 
 
 lib = _load()
-# doubles of scratch a layer total wants (exodus_layer_sum_slots): one per so many neurons of a batch element
-_NEURONS_PER_SUM_SLOT = (1 << 20) // int(lib.exodus_layer_sum_slots(1, 1 << 20))
 
 
 class ExodusHipError(RuntimeError):
@@ -115,6 +113,20 @@ def _dev(x: torch.Tensor, name: str, like: Optional[torch.Tensor] = None) -> tor
     if like is not None and x.device != like.device:
         raise RuntimeError(f"{name} and the first tensor must be on the same device")
     return x
+
+
+def _native_module():
+    """The host side of the calls in native code, given this library's entry points."""
+    try:
+        from . import _exodus_torch as native
+    except ImportError as err:
+        raise ImportError(f"{os.path.join(_HERE, '_exodus_torch.so')} cannot be loaded ({err}). Build it with "
+                          "`python build_hip.py` in the package root.") from err
+    native.bind({name: ctypes.cast(getattr(lib, name), _p).value for name in _SIGNATURES}, _check)
+    return native
+
+
+_native = _native_module()
 
 
 def _rows(x: torch.Tensor, name: str, n: int) -> torch.Tensor:
@@ -154,6 +166,14 @@ def _on_device_of(device: torch.device):
     return _NO_GUARD if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
+def _place(like: torch.Tensor, shape: Optional[tuple] = None):
+    """What allocates a call's results of up to the size of ``like`` (or of ``shape``): ``hbm.empty`` after ``hbm.enable()``
+    (memory striped over the regions of HBM), None for the ordinary allocator."""
+    if not isinstance(like, torch.Tensor):
+        return None                            # refused by the call
+    return hbm.empty if hbm.places(like.numel() if shape is None else math.prod(shape), like) else None
+
+
 def checkParameters(flags, alpha, alphaOther, theta, thetaLow) -> None:
     """Sets flags[0] where a decay factor lies outside [0, 1] and flags[1] where a threshold does not exceed its lower bound;
     the vectors (or None) have one length.  ``flags`` is a pinned int32 host tensor: read it once the stream has got here."""
@@ -170,24 +190,8 @@ def checkParameters(flags, alpha, alphaOther, theta, thetaLow) -> None:
 def lifForward(outputSpikes, vmem, input, vmemPostInitial, alpha, membrSubtract, theta, thetaLow,
                applyThetaLow: bool, maxNumSpikes: int) -> None:
     """reference cuda/bindings.cu:14-70; fills the caller-allocated ``outputSpikes`` and ``vmem``."""
-    _dev(input, "input")
-    if input.ndim != 2:
-        raise RuntimeError("input must be 2-D (rows, time)")
-    n, t = input.shape
-    _mat(_dev(outputSpikes, "outputSpikes", input), "outputSpikes", n, t)
-    _mat(_dev(vmem, "vmem", input), "vmem", n, t)
-    for nm, x in (("vmemPostInitial", vmemPostInitial), ("alpha", alpha), ("membrSubtract", membrSubtract),
-                  ("theta", theta)):
-        _rows(_dev(x, nm, input), nm, n)
-    if applyThetaLow:
-        _rows(_dev(thetaLow, "thetaLow", input), "thetaLow", n)
-    else:
-        thetaLow = None
-    with _on_device_of(input.device):
-        _check(lib.exodus_lif_forward(_ptr(outputSpikes), _ptr(vmem), _ptr(input), _ptr(vmemPostInitial),
-                                      _ptr(alpha), _ptr(membrSubtract), _ptr(theta), _ptr(thetaLow),
-                                      int(bool(applyThetaLow)), int(maxNumSpikes), n, t, _stream(input)),
-               "exodus_lif_forward")
+    _native.lif_forward(outputSpikes, vmem, input, vmemPostInitial, alpha, membrSubtract, theta, thetaLow,
+                        bool(applyThetaLow), int(maxNumSpikes))
 
 
 def lifBackward(surr, outputGrad, notClipped, alpha, membrSubtract) -> torch.Tensor:
@@ -230,17 +234,7 @@ def lifBackwardAlpha(surr, outputGrad, vmemPost, vmemPostInitial, notClipped, al
 
 def leakyForward(input, vmemInitial, alpha, *, output=None) -> torch.Tensor:
     """reference cuda/bindings.cu:163-193.  ``output`` (not in the reference) is a preallocated result."""
-    _dev(input, "input")
-    if input.ndim != 2:
-        raise RuntimeError("input must be 2-D (rows, time)")
-    n, t = input.shape
-    _rows(_dev(vmemInitial, "vmemInitial", input), "vmemInitial", n)
-    _rows(_dev(alpha, "alpha", input), "alpha", n)
-    out = hbm.empty_like(input) if output is None else _mat(_dev(output, "output", input), "output", n, t)
-    with _on_device_of(input.device):
-        _check(lib.exodus_leaky_forward(_ptr(out), _ptr(input), _ptr(vmemInitial), _ptr(alpha), n, t,
-                                        _stream(input)), "exodus_leaky_forward")
-    return out
+    return _native.leaky_forward(input, vmemInitial, alpha, output, _place(input))
 
 
 def leakyBackward(outputGrad, alpha) -> torch.Tensor:
@@ -313,26 +307,8 @@ def spikeBackward(surr, outputGrad, notClipped, alpha: float, membrSubtract: flo
 def leakyBackwardFused(outputGrad, alpha, output=None, vmemInitial=None, needAlphaGrad: bool = False,
                        inputGrad: Optional[torch.Tensor] = None):
     """One reverse pass: returns (inputGrad, alphaGrad | None, initGrad)."""
-    _dev(outputGrad, "outputGrad")
-    if outputGrad.ndim != 2:
-        raise RuntimeError("outputGrad must be 2-D (rows, time)")
-    n, t = outputGrad.shape
-    _rows(_dev(alpha, "alpha", outputGrad), "alpha", n)
-    if needAlphaGrad:
-        _mat(_dev(output, "output", outputGrad), "output", n, t)
-        _rows(_dev(vmemInitial, "vmemInitial", outputGrad), "vmemInitial", n)
-    if inputGrad is None:
-        inputGrad = hbm.empty_like(outputGrad)
-    else:
-        _mat(_dev(inputGrad, "inputGrad", outputGrad), "inputGrad", n, t)
-    initGrad = torch.zeros_like(alpha)
-    alphaGrad = torch.zeros_like(alpha) if needAlphaGrad else None
-    with _on_device_of(outputGrad.device):
-        _check(lib.exodus_leaky_backward_fused(_ptr(inputGrad), _ptr(alphaGrad), _ptr(initGrad), _ptr(outputGrad),
-                                               _ptr(output) if needAlphaGrad else None,
-                                               _ptr(vmemInitial) if needAlphaGrad else None, _ptr(alpha), n, t,
-                                               _stream(outputGrad)), "exodus_leaky_backward_fused")
-    return inputGrad, alphaGrad, initGrad
+    return _native.leaky_backward_fused(outputGrad, alpha, output, vmemInitial, bool(needAlphaGrad), inputGrad,
+                                        _place(outputGrad))
 
 
 def lifBackwardFused(gradSpikes, gradVmem, vmem, vmemPostInitial, alpha, membrSubtract, theta, thetaLow,
@@ -343,40 +319,9 @@ def lifBackwardFused(gradSpikes, gradVmem, vmem, vmemPostInitial, alpha, membrSu
 
     ``membrSubtract`` is the plain subtract value here (not pre-multiplied by alpha).
     """
-    _dev(vmem, "vmem")
-    if vmem.ndim != 2:
-        raise RuntimeError("vmem must be 2-D (rows, time)")
-    n, t = vmem.shape
-    _mat(_dev(gradSpikes, "gradSpikes", vmem), "gradSpikes", n, t)
-    if gradVmem is not None:
-        _mat(_dev(gradVmem, "gradVmem", vmem), "gradVmem", n, t)
-    for nm, x in (("alpha", alpha), ("membrSubtract", membrSubtract), ("theta", theta)):
-        _rows(_dev(x, nm, vmem), nm, n)
-    if applyThetaLow:
-        _rows(_dev(thetaLow, "thetaLow", vmem), "thetaLow", n)
-    else:
-        thetaLow = None
-    if needAlphaGrad:
-        _rows(_dev(vmemPostInitial, "vmemPostInitial", vmem), "vmemPostInitial", n)
-    if surrogateKind == SURR_TENSOR:
-        _mat(_dev(surr, "surr", vmem), "surr", n, t)
-    else:
-        surr = None
-    if inputGrad is None:
-        inputGrad = hbm.empty_like(vmem)
-    else:
-        _mat(_dev(inputGrad, "inputGrad", vmem), "inputGrad", n, t)
-    initGrad = torch.zeros_like(alpha)
-    alphaGrad = torch.zeros_like(alpha) if needAlphaGrad else None
-    with _on_device_of(vmem.device):
-        _check(lib.exodus_lif_backward_fused(_ptr(inputGrad), _ptr(alphaGrad), _ptr(initGrad), _ptr(gradSpikes),
-                                             _ptr(gradVmem), _ptr(vmem), _ptr(surr),
-                                             _ptr(vmemPostInitial) if needAlphaGrad else None, _ptr(alpha),
-                                             _ptr(membrSubtract), _ptr(theta), _ptr(thetaLow),
-                                             int(bool(applyThetaLow)), int(maxNumSpikes), int(surrogateKind),
-                                             float(surrP0), float(surrP1), n, t, _stream(vmem)),
-               "exodus_lif_backward_fused")
-    return inputGrad, alphaGrad, initGrad
+    return _native.lif_backward_fused(gradSpikes, gradVmem, vmem, vmemPostInitial, alpha, membrSubtract, theta, thetaLow,
+                                      bool(applyThetaLow), int(maxNumSpikes), int(surrogateKind), float(surrP0),
+                                      float(surrP1), surr, bool(needAlphaGrad), inputGrad, _place(vmem))
 
 
 def synLifForward(input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, membrSubtract, theta, thetaLow,
@@ -458,25 +403,11 @@ LAYER_MAX_NEURONS = 1 << 25
 _CHECKPOINT_INTERVAL = int(lib.exodus_layer_checkpoint_interval())
 
 
+_LAYER_LIF_OUTPUTS = ("spikes", "v_last", "i_last", "ckpt_v", "ckpt_i", "v_rec", "i_rec", "spike_sum")
+
+
 def checkpointInterval() -> int:
     return _CHECKPOINT_INTERVAL
-
-
-def _btm(x: torch.Tensor, name: str, like: Optional[torch.Tensor] = None):
-    _dev(x, name, like)
-    if x.ndim != 3:
-        raise RuntimeError(f"{name} must be 3-D (batch, time, neurons)")
-    return x
-
-
-def _total_and_work(input: torch.Tensor):
-    """A float64 scalar for the sum of a forward call's outputs and the memory the kernels add it up in; both are
-    written by the call (which launches nothing, and leaves the total to us, when there is nothing to walk)."""
-    b, _, m = input.shape
-    if input.numel() == 0:
-        return torch.zeros((), dtype=torch.float64, device=input.device), None
-    return (torch.empty((), dtype=torch.float64, device=input.device),
-            torch.empty(b * -(-m // _NEURONS_PER_SUM_SLOT), dtype=torch.float64, device=input.device))
 
 
 def layerLifForward(input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, membrSubtract, theta, thetaLow,
@@ -488,80 +419,25 @@ def layerLifForward(input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, mem
     ``stateShape`` (product = batch*neurons) gives v_last / i_last that shape instead of a flat vector.
     ``wantRecords`` records potential (after the reset) and synaptic current of every step;
     ``wantPreReset`` records only the potential, before the reset (the surrogate function's argument)."""
-    if wantRecords and wantPreReset:
-        raise RuntimeError("wantRecords and wantPreReset exclude each other")
-    _btm(input, "input")
-    b, t, m = input.shape
-    n = b * m
-    syn = alphaSyn is not None
-    rows = [("vmemPostInitial", vmemPostInitial), ("alphaMem", alphaMem), ("membrSubtract", membrSubtract),
-            ("theta", theta)]
-    if syn:
-        rows += [("isynInitial", isynInitial), ("alphaSyn", alphaSyn)]
-    for nm, x in rows:
-        _rows(_dev(x, nm, input), nm, n)
-    if applyThetaLow:
-        _rows(_dev(thetaLow, "thetaLow", input), "thetaLow", n)
-    else:
-        thetaLow = None
-    # big outputs go where hbm.enable() wants them (memory striped over the regions of HBM)
-    spikes = hbm.empty_like(input) if outSpikes is None else outSpikes
-    if spikes.shape != input.shape:
-        raise RuntimeError("outSpikes must have the shape of input")
-    _dev(spikes, "outSpikes", input)
-    new = lambda *shape: (hbm.empty(shape, input) if len(shape) == 3
-                          else torch.empty(shape, dtype=torch.float32, device=input.device))
-    n_ck = (t + checkpointInterval() - 1) // checkpointInterval()
-    state_shape = (n,) if stateShape is None else tuple(stateShape)
-    if math.prod(state_shape) != n:
-        raise RuntimeError(f"stateShape {state_shape} does not hold {n} neurons")
-    res = dict(spikes=spikes, v_last=new(*state_shape), i_last=new(*state_shape) if syn else None,
-               ckpt_v=new(b, n_ck, m) if wantCheckpoints else None,
-               ckpt_i=new(b, n_ck, m) if (wantCheckpoints and syn) else None,
-               v_rec=new(b, t, m) if (wantRecords or wantPreReset) else None,
-               i_rec=new(b, t, m) if (wantRecords and syn) else None,
-               spike_sum=None)
-    work = None
-    if wantSpikeSum:
-        res["spike_sum"], work = _total_and_work(input)
-    if t == 0:                                   # nothing to integrate: the final states are the initial ones
-        res["v_last"].copy_(vmemPostInitial.reshape(state_shape))
-        if syn:
-            res["i_last"].copy_(isynInitial.reshape(state_shape))
-    with _on_device_of(input.device):
-        _check(lib.exodus_layer_lif_forward_total(
-            _ptr(spikes), _ptr(res["v_rec"]), _ptr(res["i_rec"]), _ptr(res["ckpt_v"]), _ptr(res["ckpt_i"]),
-            _ptr(res["v_last"]), _ptr(res["i_last"]), _ptr(res["spike_sum"]), _ptr(work), _ptr(input), _ptr(vmemPostInitial),
-            _ptr(isynInitial) if syn else None, _ptr(alphaMem), _ptr(alphaSyn) if syn else None, _ptr(membrSubtract),
-            _ptr(theta), _ptr(thetaLow), int(bool(applyThetaLow)), int(maxNumSpikes), int(bool(decayEarly)),
-            int(bool(normInput)), int(bool(wantPreReset)), b, t, m, _stream(input)), "exodus_layer_lif_forward_total")
-    return res
+    return dict(zip(_LAYER_LIF_OUTPUTS, _native.layer_lif_forward(
+        input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, membrSubtract, theta, thetaLow, bool(applyThetaLow),
+        int(maxNumSpikes), bool(decayEarly), bool(normInput), bool(wantCheckpoints), bool(wantRecords), bool(wantPreReset),
+        bool(wantSpikeSum), outSpikes, stateShape, _place(input))))
+
+
+# per value of a tuple: identity, version, address and shape of a tensor, anything else as it is
+stamps = _native.stamps
 
 
 def decayExpand(tau, batch: int, neurons: int):
     """exp(-1 / tau) for every neuron of every batch element, (batch*neurons,), and a copy of ``tau`` for ``decayGrad``
     (the caller's may change until then); ``tau`` holds one value or ``neurons``."""
-    _dev(tau, "tau")
-    alpha = torch.empty(batch * neurons, dtype=torch.float32, device=tau.device)
-    kept = torch.empty_like(tau)
-    with _on_device_of(tau.device):
-        _check(lib.exodus_decay_expand(_ptr(alpha), _ptr(kept), _ptr(tau), batch, neurons, tau.numel(), _stream(tau)),
-               "exodus_decay_expand")
-    return alpha, kept
+    return _native.decay_expand(tau, batch, neurons)
 
 
 def decayGrad(gradAlpha, tau, batch: int, neurons: int):
     """Gradient of ``tau``, in its shape, from that of ``decayExpand(tau, batch, neurons)``."""
-    _rows(_dev(gradAlpha, "gradAlpha", _dev(tau, "tau")), "gradAlpha", batch * neurons)
-    if batch * neurons == 0:
-        return torch.zeros_like(tau)
-    out = torch.empty_like(tau)
-    wanted = int(lib.exodus_decay_work(batch, neurons, tau.numel()))
-    work = torch.empty(wanted, dtype=torch.float64, device=tau.device) if wanted else None
-    with _on_device_of(tau.device):
-        _check(lib.exodus_decay_grad(_ptr(out), _ptr(work), _ptr(gradAlpha), _ptr(tau), batch, neurons, tau.numel(),
-                                     _stream(tau)), "exodus_decay_grad")
-    return out
+    return _native.decay_grad(gradAlpha, tau, batch, neurons)
 
 
 def backwardTimeSplit(mode: int = -1) -> int:
@@ -594,141 +470,29 @@ def layerLifBackward(gradSpikes, gradVLast, gradILast, input, ckptV, ckptI, vmem
     missing while the other is given counts as zero.
     ``ckptV is None`` calls ``exodus_layer_lif_backward_from_input``: the library rebuilds the checkpoints in its
     own fixed device array (``scratchFloats()``) and allocates nothing; concurrent calls on one GPU must not overlap."""
-    _btm(input, "input")
-    b, t, m = input.shape
-    n = b * m
-    syn = alphaSyn is not None
-    if gradUniform:
-        if _dev(gradSpikes, "gradSpikes", input).numel() != 1:
-            raise RuntimeError("gradSpikes must hold one value when gradUniform is set")
-        if surrogateKind == SURR_TENSOR or gradVRec is not None or gradIRec is not None:
-            raise RuntimeError("gradUniform needs an in-kernel surrogate and no gradients on the state records")
-    elif _btm(gradSpikes, "gradSpikes", input).shape != input.shape:
-        raise RuntimeError("gradSpikes must have the shape of input")
-    n_ck = (t + checkpointInterval() - 1) // checkpointInterval()
-    from_input = ckptV is None
-    if not from_input:
-        for nm, x in (("ckptV", ckptV),) + ((("ckptI", ckptI),) if syn else ()):
-            if _btm(x, nm, input).shape != (b, n_ck, m):
-                raise RuntimeError(f"{nm} must have shape ({b}, {n_ck}, {m})")
-    rows = [("vmemPostInitial", vmemPostInitial), ("alphaMem", alphaMem), ("membrSubtract", membrSubtract),
-            ("theta", theta)]
-    if syn:
-        rows += [("isynInitial", isynInitial), ("alphaSyn", alphaSyn)]
-    for nm, x in rows:
-        _rows(_dev(x, nm, input), nm, n)
-    for nm, x in (("gradVLast", gradVLast), ("gradILast", gradILast if syn else None)):
-        if x is not None and _dev(x, nm, input).numel() != n:
-            raise RuntimeError(f"{nm} must hold {n} values")
-    if applyThetaLow:
-        _rows(_dev(thetaLow, "thetaLow", input), "thetaLow", n)
-    else:
-        thetaLow = None
-    if gradInput is None:
-        gradInput = hbm.empty_like(input)
-    elif _btm(gradInput, "gradInput", input).shape != input.shape:
-        raise RuntimeError("gradInput must have the shape of input")
-    if surrogateKind == SURR_TENSOR:
-        if surr is None or _btm(surr, "surr", input).shape != input.shape:
-            raise RuntimeError("surr must be given with the shape of input")
-    else:
-        surr = None
-    if not syn:
-        gradIRec = None
-    if gradVRec is not None or gradIRec is not None:
-        if gradVRec is None:
-            gradVRec = torch.zeros_like(input)
-        if syn and gradIRec is None:
-            gradIRec = torch.zeros_like(input)
-        for nm, x in (("gradVRec", gradVRec), ("gradIRec", gradIRec)):
-            if x is not None and _btm(x, nm, input).shape != input.shape:
-                raise RuntimeError(f"{nm} must have the shape of input")
-    # the kernel writes every neuron's entry of each vector it is given -- unless there is no step to
-    # walk: then nothing is launched, the decay factors have no influence and a gradient on a final
-    # state is the gradient of the initial state it equals
-    # (the wanted vectors are rows of one allocation)
-    wanted = [bool(wantAlphaMemGrad), bool(wantVInitGrad), bool(syn and wantAlphaSynGrad), bool(syn and wantIInitGrad)]
-    block = (torch.zeros if t == 0 else torch.empty)((sum(wanted), n), dtype=torch.float32, device=input.device)
-    taken = iter(block.unbind(0))
-    am_g, v0_g, as_g, i0_g = (next(taken) if w else None for w in wanted)
-    if t == 0:
-        if v0_g is not None and gradVLast is not None:
-            v0_g.copy_(gradVLast.reshape(-1))
-        if i0_g is not None and gradILast is not None:
-            i0_g.copy_(gradILast.reshape(-1))
-    head = (_ptr(gradInput), _ptr(am_g), _ptr(as_g), _ptr(v0_g), _ptr(i0_g), _ptr(gradSpikes), _ptr(gradVLast),
-            _ptr(gradILast) if syn else None, _ptr(input))
-    tail = (_ptr(vmemPostInitial), _ptr(isynInitial) if syn else None, _ptr(alphaMem), _ptr(alphaSyn) if syn else None,
-            _ptr(membrSubtract), _ptr(theta), _ptr(thetaLow), int(bool(applyThetaLow)), int(maxNumSpikes),
-            int(bool(decayEarly)), int(bool(normInput)), int(surrogateKind), float(surrP0), float(surrP1), _ptr(surr),
-            _ptr(gradVRec), _ptr(gradIRec), int(bool(gradUniform)), b, t, m, _stream(input))
-    with _on_device_of(input.device):
-        if from_input:
-            _check(lib.exodus_layer_lif_backward_from_input(*head, *tail), "exodus_layer_lif_backward_from_input")
-        else:
-            _check(lib.exodus_layer_lif_backward(*head, _ptr(ckptV), _ptr(ckptI) if syn else None, *tail),
-                   "exodus_layer_lif_backward")
-    return gradInput, am_g, as_g, v0_g, i0_g
+    return _native.layer_lif_backward(
+        gradSpikes, gradVLast, gradILast, input, ckptV, ckptI, vmemPostInitial, isynInitial, alphaMem, alphaSyn, membrSubtract,
+        theta, thetaLow, bool(applyThetaLow), int(maxNumSpikes), bool(decayEarly), bool(normInput), int(surrogateKind),
+        float(surrP0), float(surrP1), gradInput, surr, gradVRec, gradIRec, bool(wantAlphaMemGrad), bool(wantAlphaSynGrad),
+        bool(wantVInitGrad), bool(wantIInitGrad), bool(gradUniform), _place(input))
 
 
 def layerLeakyForward(input, vmemInitial, alpha, decayEarly: bool, normInput: bool,
                       stateShape: Optional[tuple] = None, wantSum: bool = False):
     """Leaky-integrator layer on (batch, time, neurons): returns (out, v_last), or with ``wantSum``
     (out, v_last, out_sum) where out_sum is a float64 scalar holding the sum of all outputs."""
-    _btm(input, "input")
-    b, t, m = input.shape
-    n = b * m
-    _rows(_dev(vmemInitial, "vmemInitial", input), "vmemInitial", n)
-    _rows(_dev(alpha, "alpha", input), "alpha", n)
-    state_shape = (n,) if stateShape is None else tuple(stateShape)
-    if math.prod(state_shape) != n:
-        raise RuntimeError(f"stateShape {state_shape} does not hold {n} neurons")
-    out = hbm.empty_like(input)
-    v_last = torch.empty(state_shape, dtype=torch.float32, device=input.device)
-    total, work = _total_and_work(input) if wantSum else (None, None)
-    if t == 0:
-        v_last.copy_(vmemInitial.reshape(state_shape))
-    with _on_device_of(input.device):
-        _check(lib.exodus_layer_leaky_forward_total(_ptr(out), _ptr(v_last), _ptr(total), _ptr(work), _ptr(input),
-                                                    _ptr(vmemInitial), _ptr(alpha), int(bool(decayEarly)),
-                                                    int(bool(normInput)), b, t, m, _stream(input)),
-               "exodus_layer_leaky_forward_total")
-    return (out, v_last, total) if wantSum else (out, v_last)
+    res = _native.layer_leaky_forward(input, vmemInitial, alpha, bool(decayEarly), bool(normInput), stateShape, bool(wantSum),
+                                      _place(input))
+    return res if wantSum else res[:2]
 
 
 def layerLeakyBackward(gradOut, gradVLast, out, input, vmemInitial, alpha, decayEarly: bool, normInput: bool,
                        needAlphaGrad: bool, shape: Optional[tuple] = None):
     """Returns (gradInput, alphaGrad | None, vInitGrad).  With ``shape`` = (batch, time, neurons), ``gradOut`` is a
     one-element tensor whose value is the gradient of every output (the gradient of a sum)."""
-    uniform = shape is not None
-    if uniform:
-        if _dev(gradOut, "gradOut").numel() != 1:
-            raise RuntimeError("gradOut must hold one value when shape is given")
-        b, t, m = (int(v) for v in shape)
-    else:
-        _btm(gradOut, "gradOut")
-        b, t, m = gradOut.shape
-    n = b * m
-    _rows(_dev(alpha, "alpha", gradOut), "alpha", n)
-    if gradVLast is not None and _dev(gradVLast, "gradVLast", gradOut).numel() != n:
-        raise RuntimeError(f"gradVLast must hold {n} values")
-    need_x = needAlphaGrad and (decayEarly or normInput)
-    if needAlphaGrad:
-        if tuple(_btm(out, "out", gradOut).shape) != (b, t, m):
-            raise RuntimeError("out must have the shape of gradOut")
-        _rows(_dev(vmemInitial, "vmemInitial", gradOut), "vmemInitial", n)
-    if need_x and tuple(_btm(input, "input", gradOut).shape) != (b, t, m):
-        raise RuntimeError("input must have the shape of gradOut")
-    grad_input = hbm.empty((b, t, m), gradOut)
-    block = torch.zeros((2 if needAlphaGrad else 1, n), dtype=torch.float32, device=gradOut.device)
-    v_init_grad = block[0]
-    alpha_grad = block[1] if needAlphaGrad else None
-    if t == 0 and gradVLast is not None:
-        v_init_grad.copy_(gradVLast.reshape(-1))
-    with _on_device_of(gradOut.device):
-        _check(lib.exodus_layer_leaky_backward(
-            _ptr(grad_input), _ptr(alpha_grad), _ptr(v_init_grad), _ptr(gradOut), _ptr(gradVLast),
-            _ptr(out) if needAlphaGrad else None, _ptr(input) if need_x else None,
-            _ptr(vmemInitial) if needAlphaGrad else None, _ptr(alpha), int(bool(decayEarly)), int(bool(normInput)),
-            int(uniform), b, t, m, _stream(gradOut)), "exodus_layer_leaky_backward")
-    return grad_input, alpha_grad, v_init_grad
+    if shape is not None:
+        shape = tuple(int(v) for v in shape)
+    return _native.layer_leaky_backward(gradOut, gradVLast, out, input, vmemInitial, alpha, bool(decayEarly), bool(normInput),
+                                        bool(needAlphaGrad), shape, _place(gradOut, shape))
+
+

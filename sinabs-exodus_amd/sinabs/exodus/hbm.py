@@ -427,6 +427,11 @@ def _wanted(nbytes: int, device: torch.device) -> bool:
             and bool(_active.sizes[STRIPED]))
 
 
+def places(count: int, like: torch.Tensor) -> bool:
+    """Whether ``empty`` puts a tensor of ``count`` elements of ``like``'s kind elsewhere than the ordinary allocator does."""
+    return _wanted(count * like.element_size(), like.device)
+
+
 def empty_like(like: torch.Tensor) -> torch.Tensor:
     """``torch.empty_like(like)`` (contiguous) -- after ``enable()``, and for 1 MiB or more, in the striped range."""
     if not _wanted(like.numel() * like.element_size(), like.device):

@@ -31,6 +31,10 @@ def _one_value(grad: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     return grad.as_strided((1,), (1,))
 
 
+def _dense(grad: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    return None if grad is None else grad.contiguous()
+
+
 class SpikingLayerFunction(torch.autograd.Function):
     @staticmethod
     def forward(
@@ -91,43 +95,27 @@ class SpikingLayerFunction(torch.autograd.Function):
         ctx.surrogate_grad_fn = surrogate_grad_fn if kind == _hip.SURR_TENSOR else None
         ctx.set_materialize_grads(False)
         if need_grad:
-            saved = [inp, res["ckpt_v"], v_mem_init, alpha_mem, membrane_subtract, threshold]
+            v_pre = None
             if kind == _hip.SURR_TENSOR:
                 # the function's argument is the potential before the reset; a post-reset record plus
                 # what the reset took away gives it back (up to one rounding)
                 v_pre = res["v_rec"]
                 if record_states:
                     v_pre = torch.addcmul(v_pre, res["spikes"], membrane_subtract.view(inp.shape[0], 1, inp.shape[2]))
-                saved.append(v_pre)
-            if syn:
-                saved += [res["ckpt_i"], i_syn_init, alpha_syn]
-            if apply_min:
-                saved.append(min_v_mem)
-            ctx.taus = (tau_mem is not None, tau_syn is not None)
-            saved += [tau for tau in (tau_mem, tau_syn) if tau is not None]
-            ctx.save_for_backward(*saved)
+            ctx.save_for_backward(inp, res["ckpt_v"], res["ckpt_i"], v_mem_init, i_syn_init if syn else None, alpha_mem,
+                                  alpha_syn, membrane_subtract, threshold, min_v_mem, v_pre, tau_mem, tau_syn)
         return (res["spikes"], res["v_last"], res["i_last"] if syn else None, res["spike_sum"],
                 res["v_rec"] if record_states else None, res["i_rec"] if (record_states and syn) else None)
 
     @staticmethod
     def backward(ctx, grad_spikes, grad_v_last, grad_i_last, grad_total, grad_v_rec=None, grad_i_rec=None):
         syn, apply_min, max_spikes, decay_early, norm_input, kind, p0, p1 = ctx.cfg
-        saved = list(ctx.saved_tensors)
-        inp, ckpt_v, v_mem_init, alpha_mem, membrane_subtract, threshold = saved[:6]
-        rest = saved[6:]
-        v_pre = None
-        if kind == _hip.SURR_TENSOR:
-            v_pre, rest = rest[0], rest[1:]
-        ckpt_i = i_syn_init = alpha_syn = None
-        if syn:
-            ckpt_i, i_syn_init, alpha_syn = rest[:3]
-            rest = rest[3:]
-        min_v_mem = rest.pop(0) if apply_min else None
-        tau_mem = rest.pop(0) if ctx.taus[0] else None
-        tau_syn = rest.pop(0) if ctx.taus[1] else None
+        (inp, ckpt_v, ckpt_i, v_mem_init, i_syn_init, alpha_mem, alpha_syn, membrane_subtract, threshold, min_v_mem, v_pre,
+         tau_mem, tau_syn) = ctx.saved_tensors
         need = ctx.needs_input_grad
         need += (False,) * (17 - len(need))             # one entry per argument that the call named
-        if all(g is None for g in (grad_spikes, grad_v_last, grad_i_last, grad_total, grad_v_rec, grad_i_rec)):
+        if (grad_spikes is None and grad_v_last is None and grad_i_last is None and grad_total is None and grad_v_rec is None
+                and grad_i_rec is None):
             return (None,) * 17
         # one value for every spike (a sum as the loss, the spike total behind firing_rate): handed over as it is
         uniform = None
@@ -146,7 +134,6 @@ class SpikingLayerFunction(torch.autograd.Function):
                 grad_spikes = torch.zeros_like(inp)
             if grad_total is not None:
                 grad_spikes = grad_spikes + grad_total.to(grad_spikes.dtype)
-        cont = lambda x: None if x is None else x.contiguous()
         surr = None
         if v_pre is not None:
             # the function sees (batch, time, neurons) potentials and thresholds that broadcast over time
@@ -155,16 +142,15 @@ class SpikingLayerFunction(torch.autograd.Function):
                 surr = ctx.surrogate_grad_fn(v_pre, threshold.view(b, 1, m))
             surr = torch.as_tensor(surr, device=inp.device).to(torch.float32).expand(inp.shape).contiguous()
         grad_input, g_am, g_as, g_v0, g_i0 = _hip.layerLifBackward(
-            cont(grad_spikes), cont(grad_v_last), cont(grad_i_last) if syn else None, inp, ckpt_v, ckpt_i,
+            grad_spikes.contiguous(), _dense(grad_v_last), _dense(grad_i_last) if syn else None, inp, ckpt_v, ckpt_i,
             v_mem_init, i_syn_init, alpha_mem, alpha_syn, membrane_subtract, threshold, min_v_mem, apply_min,
             max_spikes, decay_early, norm_input, kind, p0, p1, surr=surr,
-            gradVRec=cont(grad_v_rec), gradIRec=cont(grad_i_rec) if syn else None,
+            gradVRec=_dense(grad_v_rec), gradIRec=_dense(grad_i_rec) if syn else None,
             wantAlphaMemGrad=need[1] or need[15], wantAlphaSynGrad=need[2] or need[16], wantVInitGrad=need[3],
             wantIInitGrad=need[4], gradUniform=uniform is not None,
         )
-        b, _, m = inp.shape
-        g_tm = _hip.decayGrad(g_am, tau_mem, b, m) if need[15] else None
-        g_ts = _hip.decayGrad(g_as, tau_syn, b, m) if need[16] else None
+        g_tm = _hip.decayGrad(g_am, tau_mem, inp.shape[0], inp.shape[2]) if need[15] else None
+        g_ts = _hip.decayGrad(g_as, tau_syn, inp.shape[0], inp.shape[2]) if need[16] else None
         return ((grad_input if need[0] else None, g_am if need[1] else None, g_as if need[2] else None, g_v0, g_i0)
                 + (None,) * 10 + (g_tm, g_ts))
 
@@ -206,7 +192,6 @@ class LeakyLayerFunction(torch.autograd.Function):
             v_mem_init = out = inp = tau = None
         if grad_out is None and grad_v_last is None and grad_total is None:
             return (None,) * 7
-        cont = lambda x: None if x is None else x.contiguous()
         numel = shape[0] * shape[1] * shape[2]
 
         def grads(grad_input, grad_alpha, grad_init):
@@ -223,12 +208,12 @@ class LeakyLayerFunction(torch.autograd.Function):
             uniform = total if uniform is None else uniform + total
         if uniform is not None and numel > 1:
             grad_input, grad_alpha, grad_init = _hip.layerLeakyBackward(
-                uniform, cont(grad_v_last), out, inp, v_mem_init, alpha, decay_early, norm_input, need_alpha, shape=shape)
+                uniform, _dense(grad_v_last), out, inp, v_mem_init, alpha, decay_early, norm_input, need_alpha, shape=shape)
             return grads(grad_input, grad_alpha, grad_init)
         if grad_out is None:
             grad_out = torch.zeros(shape, dtype=torch.float32, device=alpha.device)
         if grad_total is not None:
             grad_out = grad_out + grad_total.to(grad_out.dtype)
         grad_input, grad_alpha, grad_init = _hip.layerLeakyBackward(
-            cont(grad_out), cont(grad_v_last), out, inp, v_mem_init, alpha, decay_early, norm_input, need_alpha)
+            _dense(grad_out), _dense(grad_v_last), out, inp, v_mem_init, alpha, decay_early, norm_input, need_alpha)
         return grads(grad_input, grad_alpha, grad_init)

@@ -1,0 +1,102 @@
+"""The native host side of the kernel calls: what it refuses, which exceptions callers see, and calls from several threads on
+several streams at once."""
+import threading
+
+import pytest
+import torch
+
+
+def hip():
+    from sinabs.exodus import _hip
+    return _hip
+
+
+def calls(x, r, two):
+    """name -> call with the (batch, time, neurons) tensor x, the per-neuron vector r and the (rows, time) matrix two"""
+    h = hip()
+    return {
+        "layerLifForward": lambda: h.layerLifForward(x, r, None, r, None, r, r, None, False, -1, True, True),
+        "layerLifBackward": lambda: h.layerLifBackward(x, None, None, x, None, None, r, None, r, None, r, r, None, False, -1,
+                                                       True, True, 1, 0.5, 1.0),
+        "layerLeakyForward": lambda: h.layerLeakyForward(x, r, r, True, True),
+        "layerLeakyBackward": lambda: h.layerLeakyBackward(x, None, x, x, r, r, True, True, True),
+        "decayExpand": lambda: h.decayExpand(r, 1, 6),
+        "decayGrad": lambda: h.decayGrad(r, r, 1, 6),
+        "lifForward": lambda: h.lifForward(two, two, two, r, r, r, r, None, False, -1),
+        "lifBackwardFused": lambda: h.lifBackwardFused(two, None, two, r, r, r, r, None, False, -1, 1),
+        "leakyForward": lambda: h.leakyForward(two, r, r),
+        "leakyBackwardFused": lambda: h.leakyBackwardFused(two, r, two, r, True),
+    }
+
+
+NAMES = ("layerLifForward", "layerLifBackward", "layerLeakyForward", "layerLeakyBackward", "decayExpand", "decayGrad",
+         "lifForward", "lifBackwardFused", "leakyForward", "leakyBackwardFused")
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_tensors_that_are_not_on_the_gpu_and_things_that_are_no_tensors(name):
+    with pytest.raises(RuntimeError, match="HIP device"):
+        calls(torch.zeros(1, 4, 6), torch.zeros(6), torch.zeros(6, 4))[name]()
+    with pytest.raises(TypeError):
+        calls([0.0], [0.0], [0.0])[name]()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", NAMES)
+def test_wrong_types_shapes_and_strides(name):
+    x, r, two = torch.rand(1, 4, 6).cuda(), torch.rand(6).cuda() * 0.5 + 0.3, torch.rand(6, 4).cuda()
+    calls(x, r, two)[name]()
+    with pytest.raises(RuntimeError, match="float32"):
+        calls(x.double(), r.double(), two.double())[name]()
+    with pytest.raises(RuntimeError, match="contiguous"):
+        calls(x.transpose(1, 2), r.repeat_interleave(2)[::2], two.t())[name]()
+    if not name.startswith("decay"):
+        with pytest.raises(RuntimeError, match=r"must have shape \(6,\), got \(7,\)"):
+            calls(x, torch.rand(7).cuda(), two)[name]()
+        with pytest.raises(RuntimeError, match="3-D|2-D"):
+            calls(r, r, r)[name]()
+
+
+@pytest.mark.gpu
+def test_a_status_of_the_library_becomes_its_own_exception():
+    h = hip()
+    wide = torch.empty(1, 0, h.LAYER_MAX_NEURONS).cuda()
+    r = torch.empty(h.LAYER_MAX_NEURONS).cuda()
+    x = torch.zeros(1, 1, h.LAYER_MAX_NEURONS).cuda()
+    assert h.layerLeakyForward(wide, r, r, False, False)[0].numel() == 0      # no step: nothing to refuse
+    with pytest.raises(h.ExodusHipError, match="exodus_layer_leaky_forward_total failed"):
+        h.layerLeakyForward(x, r, r, False, False)
+
+
+@pytest.mark.gpu
+def test_threads_on_streams_of_their_own():
+    import sinabs.exodus.layers as el
+    want, got = {}, {}
+
+    def step(k, into):
+        g = torch.Generator(device="cuda").manual_seed(k)
+        layer = el.LIF(tau_mem=10.0 + k, tau_syn=5.0).cuda()
+        x = torch.empty(3 + k, 70, 50, device="cuda").normal_(0.5, 2.0, generator=g).requires_grad_(True)
+        for _ in range(5):
+            layer.reset_states()
+            layer.zero_grad()
+            x.grad = None
+            out = layer(x)
+            out.backward(torch.ones_like(out))
+        torch.cuda.current_stream().synchronize()
+        into[k] = (out.detach().cpu(), x.grad.cpu(), layer.tau_mem.grad.cpu())
+
+    def on_stream(k):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            step(k, got)
+
+    for k in range(4):
+        step(k, want)
+    threads = [threading.Thread(target=on_stream, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k in range(4):
+        for p, q in zip(want[k], got[k]):
+            assert torch.equal(p, q)
