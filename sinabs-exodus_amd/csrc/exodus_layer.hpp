@@ -154,7 +154,7 @@ struct Neuron {
     float xs;           // factor on the input entering the synapse: alpha_syn (decay_early) or 1
     float c, th;        // subtract value, threshold
     float c2;           // 2 * subtract value (exact), what two spikes take away
-    float th2;          // 2 * threshold: from here on a second spike (+inf where th <= 0)
+    float th2;          // 2 * threshold: from here on a second spike (NaN, so never, where th is not positive)
     float thd;          // from here on the spike count needs the quotient v / th (+inf if never)
     float lo;           // lower bound of the potential, -inf without one
     float gate;         // gradients pass where the potential lies above
@@ -169,7 +169,7 @@ __device__ __forceinline__ void settle(Neuron &n)
 
 // spike-count cap as the kernels use it (block-uniform)
 struct Cap {
-    float one, two;     // min(cap, 1), min(cap, 2)
+    float one;          // min(cap, 1)
     unsigned cap;
 };
 
@@ -190,7 +190,7 @@ __device__ __forceinline__ void neuron_load(Neuron &n, const LayerConsts &p, int
     // positive -- takes the quotient.
     // A subtract value whose double is beyond the floats' range goes there, too, so that count * c is exact below n.thd.
     const bool plain = n.th > 0.f && !(fabsf(n.c) > 0x1p126f);
-    n.th2 = plain ? __fadd_rn(n.th, n.th) : __builtin_inff();
+    n.th2 = plain ? __fadd_rn(n.th, n.th) : __builtin_nanf("");
     n.thd = plain ? (CAPK == 0 ? n.th2 : __builtin_inff()) : n.th;
     n.lo = p.apply_low ? p.theta_low[row] : -__builtin_inff();
     // a bound that is no number bounds nothing and lets no gradient pass
@@ -219,13 +219,13 @@ __device__ __forceinline__ float neuron_advance(Neuron &n, float x)
 }
 
 // count = v >= th ? min(unsigned(v / th), cap) : 0   (IEEE division, truncation), in two parts:
-// the count by comparisons, and the quotient for the rare potentials at or above n.thd.
+// the count by comparisons, and the quotient for the rare potentials at or above n.thd (with CAPK == 0 that is where two
+// spikes begin).
 template <int CAPK>
 __device__ __forceinline__ float count_by_compare(float v, const Neuron &n, const Cap &cc)
 {
     const float count = v >= n.th ? (CAPK == 0 ? cc.one : 1.f) : 0.f;
-    if (CAPK == 1) return count;
-    return v >= n.th2 ? (CAPK == 0 ? cc.two : 2.f) : count;
+    return CAPK == 2 && v >= n.th2 ? 2.f : count;
 }
 
 __device__ __forceinline__ float count_by_quotient(float v, const Neuron &n, const Cap &cc)

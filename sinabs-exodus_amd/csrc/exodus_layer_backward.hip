@@ -66,7 +66,6 @@ layer_lif_backward(
     Cap cc;
     cc.cap = p.cap;
     cc.one = p.cap >= 1u ? 1.f : 0.f;
-    cc.two = p.cap >= 2u ? 2.f : cc.one;
     Neuron nr = {};
     if (active) neuron_load<SYN, CAPK>(nr, p, row);
     const float xg = (SYN && p.decay_early) ? nr.as : 1.0f;   // factor between mu and grad_x

@@ -71,7 +71,6 @@ __global__ void __launch_bounds__(SPLIT_LANES) layer_lif_backward_split(const Sp
     Cap cc;
     cc.cap = p.cap;
     cc.one = p.cap >= 1u ? 1.f : 0.f;
-    cc.two = p.cap >= 2u ? 2.f : cc.one;
     Neuron nr = {};
     neuron_load<SYN, CAPK>(nr, p, row);
     const float xg = (SYN && p.decay_early) ? nr.as : 1.0f;      // factor between mu and grad_x
