@@ -213,7 +213,7 @@ int exodus_layer_lif_forward_total(float *out_spikes, float *out_vmem_rec, float
                                    const float *membr_subtract, const float *theta, const float *theta_low,
                                    int apply_theta_low, int max_num_spikes, int decay_early, int norm_input,
                                    int record_pre_reset, int64_t batch, int64_t t, int64_t neurons, void *stream);
-int64_t exodus_layer_sum_slots(int64_t batch, int64_t neurons);
+int64_t exodus_layer_sum_slots(int64_t batch, int64_t neurons);   /* for the current device */
 
 /* Backward of the above.  Re-reads `input`, rebuilds membrane potential and synaptic current of
  * each checkpoint interval from ckpt_v / ckpt_i and walks it in reverse.  grad_v_last /

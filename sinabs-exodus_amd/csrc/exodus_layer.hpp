@@ -302,6 +302,16 @@ inline int pick_neurons_per_lane(int64_t batch, int64_t neurons, unsigned align,
     return 1;
 }
 
+// Lanes per block of the forward and leaky kernels.  Four waves that keep each other at the same step suit memory (see the
+// barriers); but up to two waves per compute unit they only crowd on a few units, whose way to memory their accesses then
+// share, while the others stand idle: one wave per block there, which also leaves no wave without a neuron.  256 / 64 lanes,
+// us, spiking (at most one spike) and leaky forward: (4, 2000, 512) 96.6 / 70.4 and 80.0 / 55.6, (64, 300, 10) 20.2 / 16.1 and
+// 15.0 / 11.3, (24, 250, 1323) with 504 waves 20.9 / 20.2 and 15.7 / 16.7, (32, 250, 2048) with 1024 26.9 / 30.3 and 23.7 / 26.3.
+inline int lanes_per_block(int64_t batch, int64_t neurons)
+{
+    return batch * ((neurons + WAVE - 1) / WAVE) <= 2 * compute_units() ? WAVE : BLOCK;
+}
+
 inline unsigned common_alignment(std::initializer_list<const void *> ptrs)
 {
     uintptr_t bits = 0;

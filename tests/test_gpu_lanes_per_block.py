@@ -1,0 +1,36 @@
+"""Layers on both sides of the rule that gives small layers blocks of one wave: outputs, final states and totals of the forward
+and leaky kernels equal those of a call on every batch element alone, and the totals are the sums of the outputs."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("b,t,m", [
+    (1, 3, 1), (3, 40, 63), (3, 40, 64), (3, 40, 65), (2, 33, 257), (5, 7, 1000),
+    (8, 40, 4096),            # 512 waves: two per compute unit, the last size with one wave per block
+    (8, 40, 4097),            # 520 waves
+    (513, 5, 10), (512, 5, 10),
+])
+def test_small_and_larger_blocks(b, t, m):
+    from sinabs.exodus import _hip as hip
+    g = torch.Generator(device="cuda").manual_seed(b * m)
+    x = torch.empty(b, t, m, device="cuda").normal_(0.2, 0.8, generator=g)
+    go = torch.empty(b, t, m, device="cuda").normal_(0.0, 1.0, generator=g)
+    full = lambda n, v: torch.full((n,), v, device="cuda")
+
+    def every(xx, gg):
+        n = xx.shape[0] * m
+        out, last, total = hip.layerLeakyForward(xx, full(n, 0.1), full(n, 0.9), True, True, wantSum=True)
+        gi, ga, gv = hip.layerLeakyBackward(gg, None, out, xx, full(n, 0.1), full(n, 0.9), True, True, True)
+        f = hip.layerLifForward(xx, full(n, 0.0), full(n, 0.0), full(n, 0.95), full(n, 0.8), full(n, 1.0), full(n, 1.0),
+                                full(n, -1.0), True, -1, True, False)
+        assert float(f["spike_sum"]) == float(f["spikes"].double().sum())
+        mass = float(out.double().abs().sum())
+        assert abs(float(total) - float(out.double().sum())) <= 32 * 2.0 ** -24 * mass   # fp32 sums of at most 32 outputs
+        return out, last, gi, ga, gv, f["spikes"], f["v_last"], f["i_last"], f["ckpt_v"], f["ckpt_i"]
+
+    whole = every(x, go)
+    for k in sorted({0, b // 2, b - 1}):
+        for p, q in zip(whole, every(x[k:k + 1].contiguous(), go[k:k + 1].contiguous())):
+            assert torch.equal(p[k] if p.ndim == 3 else p[k * m:(k + 1) * m], q[0] if q.ndim == 3 else q)
