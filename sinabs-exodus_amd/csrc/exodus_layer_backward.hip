@@ -42,7 +42,7 @@ layer_lif_backward(
 {
     typedef BufIO<1, NT> IO;
     const int64_t b = blockIdx.x / blocks_per_batch;
-    const int64_t m0 = static_cast<int64_t>(blockIdx.x - b * blocks_per_batch) * BWD_BLOCK;
+    const int64_t m0 = static_cast<int64_t>(blockIdx.x - b * blocks_per_batch) * blockDim.x;
     const unsigned lane_off = threadIdx.x;
     // lanes past the end of the layer walk the same loops and meet every barrier, but all memory
     // accesses and all arithmetic sit behind `active`
@@ -217,12 +217,17 @@ int launch_bwd(float *grad_x, float *am_g, float *as_g, float *v0_g, float *i0_g
                const float *gir, const float *ckpt_v, const float *ckpt_i, const LayerConsts &p, float p0, float p1,
                bool uniform, int64_t B, int64_t T, int64_t M, hipStream_t s)
 {
-    const int64_t blocks_per_batch = (M + BWD_BLOCK - 1) / BWD_BLOCK;
+    // One wave per block up to four waves per compute unit, as the forward has it up to two (lanes_per_block): a unit's way to
+    // memory is shared by fewer waves.  256 lanes / 64, us, without synapse: 504 waves (24, 250, 1323) 41.7 / 37.3, 512
+    // (32, 250, 1024) 42.9 / 37.3, 1024 (32, 250, 2048) 53.2 / 45.7, 2048 (64, 300, 2048) 95 / 105; with one 57.4 / 52.7,
+    // - , 69.0 / 65.0, (16, 300, 8192) 110 / 118.
+    const int lanes = B * ((M + WAVE - 1) / WAVE) <= 4 * compute_units() ? WAVE : BWD_BLOCK;
+    const int64_t blocks_per_batch = (M + lanes - 1) / lanes;
     if (blocks_per_batch > 0x7fffffffLL / B) return hipErrorInvalidValue;
     const int64_t blocks = blocks_per_batch * B;
 #define EXODUS_LAUNCH(CK, NT, EX, G1)                                                                              \
     hipLaunchKernelGGL((layer_lif_backward<SYN, KIND, CK, NT, EX, G1>), dim3(static_cast<unsigned>(blocks)),      \
-                       dim3(BWD_BLOCK), 0, s, grad_x, am_g, as_g, v0_g, i0_g, grad_spikes, gvl, gil, x, surr, gvr, \
+                       dim3(lanes), 0, s, grad_x, am_g, as_g, v0_g, i0_g, grad_spikes, gvl, gil, x, surr, gvr, \
                        gir, ckpt_v, ckpt_i, p, p0, p1, p0 != 0.f ? 1.f / p0 : 0.f, blocks_per_batch, T, M)
     if (uniform) {
         // one value as the gradient of every spike: instances exist for the in-kernel surrogates, without

@@ -34,3 +34,28 @@ def test_small_and_larger_blocks(b, t, m):
     for k in sorted({0, b // 2, b - 1}):
         for p, q in zip(whole, every(x[k:k + 1].contiguous(), go[k:k + 1].contiguous())):
             assert torch.equal(p[k] if p.ndim == 3 else p[k * m:(k + 1) * m], q[0] if q.ndim == 3 else q)
+
+
+@pytest.mark.parametrize("b,t,m", [(2, 40, 8200), (16, 40, 4096), (16, 40, 4097)])   # 258, 1024 and 1040 waves
+def test_one_lane_backward_with_both_blocks(b, t, m):
+    from sinabs.exodus import _hip as hip
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.empty(b, t, m, device="cuda").normal_(0.2, 0.8, generator=g)
+    go = torch.empty(b, t, m, device="cuda").normal_(0.0, 1.0, generator=g)
+    full = lambda n, v: torch.full((n,), v, device="cuda")
+
+    def backward(xx, gg):
+        n = xx.shape[0] * m
+        r = (full(n, 0.0), full(n, 0.0))
+        c = (full(n, 0.95), full(n, 0.8), full(n, 1.0), full(n, 1.0), full(n, -1.0), True, -1, True, False)
+        f = hip.layerLifForward(xx, *r, *c)
+        return hip.layerLifBackward(gg, None, None, xx, f["ckpt_v"], f["ckpt_i"], *r, *c, hip.SURR_SINGLE_EXP, 0.5, 1.0)
+
+    mode = hip.backwardTimeSplit(0)
+    try:
+        whole = backward(x, go)
+        for k in (0, b - 1):
+            for p, q in zip(whole, backward(x[k:k + 1].contiguous(), go[k:k + 1].contiguous())):
+                assert torch.equal(p[k] if p.ndim == 3 else p[k * m:(k + 1) * m], q[0] if q.ndim == 3 else q)
+    finally:
+        hip.backwardTimeSplit(mode)
