@@ -204,10 +204,10 @@ layer_lif_backward(
 std::atomic<int> split_mode{1};
 // batch * neurons up to which mode 1 splits: the most at which no form of the call loses by it.  The split kernel does half
 // as much again and more in arithmetic and holds fewer waves.  One lane / split, us, at 16 384 neurons (8, t, 2048), without
-// synapse, with one, with one and state records, with a surrogate tensor: 64 steps 11.0 / 8.1, 12.8 / 9.5, 14.8 / 12.2,
-// 12.7 / 8.0; 300 steps 47.9 / 21.5, 54.6 / 25.4, 60 / 42, 52.8 / 23.3; 2000 steps 287 / 97, 322 / 113, 410 / 210, 317 / 135.
-// At 32 768 neurons: 12.0 / 10.1, 13.9 / 12.3, 17.6 / 21.7, 13.4 / 10.3; 51 / 37, 57 / 45, 64 / 76, 58 / 39; 302 / 183,
-// 337 / 212, 434 / 410, 343 / 255.
+// synapse, with one, with one and state records, with a surrogate tensor: 64 steps 15.1 / 11.6, 15.0 / 12.9, 15.3 / 13.6,
+// 14.1 / 11.2 (launches among them); 300 steps 40 / 23, 43 / 26, 46 / 38, 41 / 24; 2000 steps 223 / 96, 247 / 109, 292 / 177,
+// 234 / 136.  At 32 768 neurons: 15.2 / 11.5, 15.3 / 13.9, 16.7 / 19.2, 15.5 / 11.0; 43 / 38, 49 / 46, 53 / 68, 47 / 39;
+// 233 / 186, 265 / 206, 319 / 339, 258 / 253.
 constexpr int64_t SPLIT_MOST_NEURONS = 16384;
 constexpr int64_t SPLIT_PLAIN_CHUNKS = 16;
 

@@ -11,6 +11,7 @@
 #include <c10/hip/HIPStream.h>
 #include <pybind11/pybind11.h>
 #include <pybind11/stl.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 
@@ -518,16 +519,17 @@ py::tuple leaky_backward_fused(const Tensor &grad_out, const Tensor &alpha, cons
 
 PYBIND11_MODULE(_exodus_torch, module)
 {
-    module.def("bind", &bind);
-    module.def("layer_lif_forward", &layer_lif_forward);
-    module.def("layer_lif_backward", &layer_lif_backward);
-    module.def("layer_leaky_forward", &layer_leaky_forward);
-    module.def("layer_leaky_backward", &layer_leaky_backward);
-    module.def("stamps", &stamps);
-    module.def("decay_expand", &decay_expand);
-    module.def("decay_grad", &decay_grad);
-    module.def("lif_forward", &lif_forward);
-    module.def("lif_backward_fused", &lif_backward_fused);
-    module.def("leaky_forward", &leaky_forward);
-    module.def("leaky_backward_fused", &leaky_backward_fused);
+    // torch's own exceptions reach the caller as what they are (out of memory as torch.OutOfMemoryError)
+    module.def("bind", torch::wrap_pybind_function(bind));
+    module.def("layer_lif_forward", torch::wrap_pybind_function(layer_lif_forward));
+    module.def("layer_lif_backward", torch::wrap_pybind_function(layer_lif_backward));
+    module.def("layer_leaky_forward", torch::wrap_pybind_function(layer_leaky_forward));
+    module.def("layer_leaky_backward", torch::wrap_pybind_function(layer_leaky_backward));
+    module.def("stamps", torch::wrap_pybind_function(stamps));
+    module.def("decay_expand", torch::wrap_pybind_function(decay_expand));
+    module.def("decay_grad", torch::wrap_pybind_function(decay_grad));
+    module.def("lif_forward", torch::wrap_pybind_function(lif_forward));
+    module.def("lif_backward_fused", torch::wrap_pybind_function(lif_backward_fused));
+    module.def("leaky_forward", torch::wrap_pybind_function(leaky_forward));
+    module.def("leaky_backward_fused", torch::wrap_pybind_function(leaky_backward_fused));
 }

@@ -69,6 +69,14 @@ def test_a_status_of_the_library_becomes_its_own_exception():
 
 
 @pytest.mark.gpu
+def test_running_out_of_memory_is_torchs_exception():
+    tau = torch.ones(1).cuda()
+    with pytest.raises(torch.OutOfMemoryError):
+        hip().decayExpand(tau, 1 << 40, 1)
+    assert hip().decayExpand(tau, 4, 1)[0].shape == (4,)
+
+
+@pytest.mark.gpu
 def test_threads_on_streams_of_their_own():
     import sinabs.exodus.layers as el
     want, got = {}, {}
