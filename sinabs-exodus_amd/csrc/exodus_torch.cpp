@@ -15,6 +15,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 
+#include <cstring>
 #include <optional>
 #include <stdexcept>
 #include <string>
@@ -413,23 +414,57 @@ Tensor decay_grad(const Tensor &grad_alpha, const Tensor &tau, int64_t batch, in
 // ---------------------------------------------------------------------------------------------
 // what shows that a layer's parameters are the ones of the call before
 // ---------------------------------------------------------------------------------------------
-// per value: a tensor's identity, version, address and shape; anything else as it is
-py::tuple stamps(const py::tuple &values)
+// An entry stands for a value at one moment: a tensor's holds the tensor itself, its version and a detached alias, so neither
+// its object nor its memory can be given to another tensor while the entry is alive; a number's is its float.
+bool unchanged(PyObject *entry, PyObject *value)
 {
-    py::tuple result(values.size());
-    for (size_t k = 0; k < values.size(); ++k) {
-        const py::handle value = values[k];
-        if (THPVariable_Check(value.ptr())) {
-            const Tensor &x = THPVariable_Unpack(value.ptr());
-            py::tuple sizes(x.dim());
-            for (int64_t d = 0; d < x.dim(); ++d) sizes[d] = x.size(d);
-            result[k] = py::make_tuple(reinterpret_cast<uintptr_t>(value.ptr()), x._version(),
-                                       reinterpret_cast<uintptr_t>(x.const_data_ptr()), sizes);
-        } else {
-            result[k] = value;
-        }
+    if (THPVariable_Check(value)) {
+        if (!PyTuple_CheckExact(entry) || PyTuple_GET_ITEM(entry, 0) != value) return false;
+        const Tensor &x = THPVariable_Unpack(value), &alias = THPVariable_Unpack(PyTuple_GET_ITEM(entry, 2));
+        return PyLong_AsLongLong(PyTuple_GET_ITEM(entry, 1)) == x._version() && alias.const_data_ptr() == x.const_data_ptr() &&
+               alias.sizes() == x.sizes() && alias.strides() == x.strides();
     }
-    return result;
+    if (value == Py_None) return entry == Py_None;
+    if (!PyFloat_CheckExact(entry)) return false;
+    const py::object number = py::reinterpret_steal<py::object>(PyNumber_Float(value));
+    if (!number) {
+        PyErr_Clear();
+        return false;
+    }
+    const double was = PyFloat_AS_DOUBLE(entry), is = PyFloat_AS_DOUBLE(number.ptr());
+    return std::memcmp(&was, &is, sizeof was) == 0;            // bits: a number that is none is itself, -0 is not 0
+}
+
+py::object entry_of(PyObject *value)
+{
+    if (THPVariable_Check(value)) {
+        const Tensor &x = THPVariable_Unpack(value);
+        return py::make_tuple(py::reinterpret_borrow<py::object>(value), static_cast<int64_t>(x._version()), x.detach());
+    }
+    if (value == Py_None) return py::none();
+    py::object number = py::reinterpret_steal<py::object>(PyNumber_Float(value));
+    if (number) return number;
+    PyErr_Clear();                                             // what is no number is never the same again
+    return py::reinterpret_steal<py::object>(PyObject_CallNoArgs(reinterpret_cast<PyObject *>(&PyBaseObject_Type)));
+}
+
+// One entry per value.  `kept` is what an earlier call returned, or None: its entries are handed on for the values that have not
+// changed since, and it is returned itself if none has.
+py::object stamps(const py::object &kept, const py::tuple &values)
+{
+    const size_t n = values.size();
+    const bool comparable = PyTuple_CheckExact(kept.ptr()) && static_cast<size_t>(PyTuple_GET_SIZE(kept.ptr())) == n;
+    size_t same = 0;
+    if (comparable)
+        while (same < n && unchanged(PyTuple_GET_ITEM(kept.ptr(), same), values[same].ptr())) ++same;
+    if (comparable && same == n) return kept;
+    py::tuple result(n);
+    for (size_t k = 0; k < n; ++k) {
+        PyObject *const was = comparable ? PyTuple_GET_ITEM(kept.ptr(), k) : nullptr, *const value = values[k].ptr();
+        result[k] = was && (k < same || (k > same && unchanged(was, value))) ? py::reinterpret_borrow<py::object>(was)
+                                                                             : entry_of(value);
+    }
+    return std::move(result);
 }
 
 // ---------------------------------------------------------------------------------------------

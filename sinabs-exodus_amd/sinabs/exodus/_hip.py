@@ -425,7 +425,8 @@ def layerLifForward(input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, mem
         bool(wantSpikeSum), outSpikes, stateShape, _place(input))))
 
 
-# per value of a tuple: identity, version, address and shape of a tensor, anything else as it is
+# stamps(kept, values): a tuple with one entry per value, the entries of ``kept`` (an earlier result, or None) where a value is
+# unchanged since, and ``kept`` itself where all are
 stamps = _native.stamps
 
 
