@@ -204,8 +204,8 @@ int exodus_layer_lif_forward(float *out_spikes, float *out_vmem_rec, float *out_
                              int record_pre_reset, int64_t batch, int64_t t, int64_t neurons, void *stream);
 
 /* The same with a total (one double, NULL = not wanted) that is written instead of added to: every block leaves its count
- * in sum_work, exodus_layer_sum_slots(batch, neurons) doubles that need no initialising, and a second kernel of the call adds
- * them up.  Many waves that add to one double at the end of a launch wait for each other; here none does. */
+ * in sum_work, exodus_layer_sum_slots(batch, neurons) doubles that need no initialising (one per so many neurons of a batch
+ * element, the same number for every size and device), and a second kernel of the call adds them up.  Many waves that add to one double at the end of a launch wait for each other; here none does. */
 int exodus_layer_lif_forward_total(float *out_spikes, float *out_vmem_rec, float *out_isyn_rec, float *ckpt_v,
                                    float *ckpt_i, float *v_last, float *i_last, double *spike_sum, double *sum_work,
                                    const float *input, const float *vmem_post_initial,
@@ -213,7 +213,7 @@ int exodus_layer_lif_forward_total(float *out_spikes, float *out_vmem_rec, float
                                    const float *membr_subtract, const float *theta, const float *theta_low,
                                    int apply_theta_low, int max_num_spikes, int decay_early, int norm_input,
                                    int record_pre_reset, int64_t batch, int64_t t, int64_t neurons, void *stream);
-int64_t exodus_layer_sum_slots(int64_t batch, int64_t neurons);   /* for the current device */
+int64_t exodus_layer_sum_slots(int64_t batch, int64_t neurons);
 
 /* Backward of the above.  Re-reads `input`, rebuilds membrane potential and synaptic current of
  * each checkpoint interval from ckpt_v / ckpt_i and walks it in reverse.  grad_v_last /

@@ -178,7 +178,6 @@ void total_and_work(const Tensor &input, Tensor &total, Tensor &work)
         total = at::zeros({}, at::TensorOptions().device(input.device()).dtype(at::kDouble));
         return;
     }
-    const c10::DeviceGuard guard(input.device());               // the number of slots depends on the device
     total = fresh({}, input, at::kDouble);
     work = fresh({lib.exodus_layer_sum_slots(input.size(0), input.size(2))}, input, at::kDouble);
 }

@@ -56,6 +56,16 @@ def test_layer_entry_points_reject_too_wide_layers_before_touching_the_device():
     assert _hip.lib.exodus_layer_lif_forward(*([null] * 16), 0, -1, 1, 1, 0, 0, 4, 8, null) == 0   # empty batch
 
 
+def test_slots_of_the_totals_scale_with_the_layer():
+    """One answer per neurons of a batch element holds for every size (callers keep it), and covers blocks of one wave."""
+    from sinabs.exodus import _hip
+    slots = _hip.lib.exodus_layer_sum_slots
+    per_slot = (1 << 20) // slots(1, 1 << 20)
+    for b in (1, 3, 64, 513, 4096):
+        for m in (1, 63, 64, 65, 255, 256, 257, 512, 1323, 4096, 12544, 131072, 1 << 24):
+            assert slots(b, m) == b * -(-m // per_slot) >= b * -(-m // 64)
+
+
 def test_backward_without_allocation_rejects_what_its_scratch_cannot_hold():
     """The size check of exodus_layer_lif_backward_from_input comes before anything touches a device:
     one batch element whose checkpoints exceed the fixed scratch array is refused with the library's
