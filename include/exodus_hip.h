@@ -29,7 +29,8 @@
 extern "C" {
 #endif
 
-/* ABI version of this header; bumped on any signature change. */
+/* ABI version of this header; bumped on any change of a signature or of what an entry point asks of its caller.  An added entry
+ * point leaves it as it is: whoever needs that one looks whether the library has it. */
 #define EXODUS_HIP_ABI_VERSION 8
 
 int exodus_hip_abi_version(void);

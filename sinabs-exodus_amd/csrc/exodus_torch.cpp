@@ -35,6 +35,7 @@ using Shape = std::vector<int64_t>;
 // the library
 // ---------------------------------------------------------------------------------------------
 #define EXODUS_ENTRIES(X)                                                                                               \
+    X(exodus_hip_abi_version)                                                                                           \
     X(exodus_lif_forward) X(exodus_lif_backward_fused) X(exodus_leaky_forward) X(exodus_leaky_backward_fused)           \
     X(exodus_layer_sum_slots) X(exodus_layer_checkpoint_interval) X(exodus_layer_lif_forward_total)                     \
     X(exodus_layer_lif_backward) X(exodus_layer_lif_backward_from_input) X(exodus_layer_leaky_forward_total)            \
@@ -50,10 +51,16 @@ PyObject *raise_status = nullptr;                              // (status, what)
 
 void bind(const py::dict &addresses, const py::object &on_status)
 {
+    Library given;
 #define EXODUS_BIND(name) \
-    lib.name = reinterpret_cast<decltype(lib.name)>(py::cast<uintptr_t>(addresses[#name]));
+    given.name = reinterpret_cast<decltype(given.name)>(py::cast<uintptr_t>(addresses[#name]));
     EXODUS_ENTRIES(EXODUS_BIND)
 #undef EXODUS_BIND
+    const int version = given.exodus_hip_abi_version();        // the signatures above are those of one version of the header
+    if (version != EXODUS_HIP_ABI_VERSION)
+        throw py::import_error("the library has ABI version " + std::to_string(version) + ", _exodus_torch was built for " +
+                               std::to_string(EXODUS_HIP_ABI_VERSION));
+    lib = given;
     interval = lib.exodus_layer_checkpoint_interval();
     Py_XDECREF(raise_status);
     raise_status = py::object(on_status).release().ptr();

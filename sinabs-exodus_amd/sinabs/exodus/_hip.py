@@ -78,13 +78,16 @@ def _load() -> ctypes.CDLL:
             "(needs hipcc; cross-compiles for gfx950 without a GPU). There is no CPU fallback."
         )
     lib = ctypes.CDLL(LIB_PATH)
+    missing = [name for name in _SIGNATURES if not hasattr(lib, name)]     # a library of the same version may be older
+    if missing:
+        raise ImportError(f"{LIB_PATH} is not a library of this package or an older one: it lacks {', '.join(missing)}")
     for name, (argtypes, restype) in _SIGNATURES.items():
-        fn = getattr(lib, name)  # AttributeError here = library/header mismatch
+        fn = getattr(lib, name)
         fn.argtypes = argtypes
         fn.restype = restype
     got = lib.exodus_hip_abi_version()
     if got != ABI_VERSION:
-        raise ImportError(f"libexodus_hip.so has ABI version {got}, this package expects {ABI_VERSION}")
+        raise ImportError(f"{LIB_PATH} has ABI version {got}, this package expects {ABI_VERSION}")
     return lib
 
 

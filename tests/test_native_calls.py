@@ -1,5 +1,9 @@
 """The native host side of the kernel calls: what it refuses, which exceptions callers see, and calls from several threads on
 several streams at once."""
+import ctypes
+import os
+import subprocess
+import sys
 import threading
 
 import pytest
@@ -39,6 +43,25 @@ def test_tensors_that_are_not_on_the_gpu_and_things_that_are_no_tensors(name):
         calls(torch.zeros(1, 4, 6), torch.zeros(6), torch.zeros(6, 4))[name]()
     with pytest.raises(TypeError):
         calls([0.0], [0.0], [0.0])[name]()
+
+
+def test_library_of_another_version_is_refused():
+    """Neither the Python nor the native half takes it, and the native half keeps the library it has."""
+    h, native = hip(), hip()._native
+    addresses = {name: ctypes.cast(getattr(h.lib, name), ctypes.c_void_p).value for name in h._SIGNATURES}
+    other = ctypes.CFUNCTYPE(ctypes.c_int)(lambda: h.ABI_VERSION - 1)
+    wrong = {**{name: 0 for name in addresses}, "exodus_hip_abi_version": ctypes.cast(other, ctypes.c_void_p).value}
+    with pytest.raises(ImportError, match=f"version {h.ABI_VERSION - 1}"):
+        native.bind(wrong, h._check)
+    native.bind(addresses, h._check)
+
+
+def test_library_without_an_entry_point_is_named():
+    probes = os.path.join(os.path.dirname(hip().__file__), "..", "..", "libexodus_bench_probes.so")
+    got = subprocess.run([sys.executable, "-c", "import sinabs.exodus.layers"], capture_output=True, text=True,
+                         env={**os.environ, "EXODUS_HIP_LIBRARY": os.path.abspath(probes),
+                              "PYTHONPATH": os.path.join(os.path.dirname(hip().__file__), "..", "..")})
+    assert got.returncode != 0 and "ImportError" in got.stderr and "exodus_check_parameters" in got.stderr, got.stderr
 
 
 @pytest.mark.gpu
