@@ -19,6 +19,7 @@
 #include <optional>
 #include <stdexcept>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "exodus_hip.h"
@@ -30,6 +31,11 @@ namespace {
 using at::Tensor;
 using Maybe = std::optional<Tensor>;
 using Shape = std::vector<int64_t>;
+// results of a call, None in Python where undefined
+using Two = std::tuple<Tensor, Tensor>;
+using Three = std::tuple<Tensor, Tensor, Tensor>;
+using Five = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor>;
+using Eight = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor>;
 
 // ---------------------------------------------------------------------------------------------
 // the library
@@ -66,17 +72,19 @@ void bind(const py::dict &addresses, const py::object &on_status)
     raise_status = py::object(on_status).release().ptr();
 }
 
-// call a function of the library on the tensor's device and stream, without the interpreter lock
+// call a function of the library on the tensor's device and stream
 template <class F>
 void launch(const Tensor &like, const char *what, F &&call)
 {
     int status;
     {
-        py::gil_scoped_release unlocked;
         const c10::DeviceGuard guard(like.device());
         status = call(static_cast<void *>(c10::hip::getCurrentHIPStream(like.device().index()).stream()));
     }
-    if (status != 0) py::reinterpret_borrow<py::object>(raise_status)(status, what);
+    if (status != 0) {
+        py::gil_scoped_acquire locked;
+        py::reinterpret_borrow<py::object>(raise_status)(status, what);
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -167,6 +175,7 @@ Tensor fresh(c10::IntArrayRef shape, const Tensor &like, at::ScalarType type = a
 Tensor large(c10::IntArrayRef shape, const Tensor &like, const py::object &place)
 {
     if (place.is_none()) return fresh(shape, like);
+    py::gil_scoped_acquire locked;
     return py::cast<Tensor>(place(py::cast(Shape(shape.begin(), shape.end())), like));
 }
 
@@ -200,7 +209,7 @@ Shape state_shape_of(const std::optional<Shape> &asked, int64_t n)
 // ---------------------------------------------------------------------------------------------
 // layers on (batch, time, neurons)
 // ---------------------------------------------------------------------------------------------
-py::tuple layer_lif_forward(const Tensor &input, const Tensor &v_init, const Maybe &i_init, const Tensor &alpha_mem,
+Eight layer_lif_forward(const Tensor &input, const Tensor &v_init, const Maybe &i_init, const Tensor &alpha_mem,
                             const Maybe &alpha_syn, const Tensor &subtract, const Tensor &theta, const Maybe &theta_low,
                             bool apply_low, int64_t max_spikes, bool decay_early, bool norm_input, bool want_checkpoints,
                             bool want_records, bool want_pre_reset, bool want_sum, const Maybe &out_spikes,
@@ -236,11 +245,11 @@ py::tuple layer_lif_forward(const Tensor &input, const Tensor &v_init, const May
             input.const_data_ptr<float>(), v0, i0, am, as, c, th, lo, apply_low, static_cast<int>(max_spikes), decay_early,
             norm_input, want_pre_reset, b, t, m, stream);
     });
-    return py::make_tuple(spikes, v_last, i_last, ckpt_v, ckpt_i, v_rec, i_rec, total);
+    return {spikes, v_last, i_last, ckpt_v, ckpt_i, v_rec, i_rec, total};
 }
 
 // -> (grad_input, alpha_mem, alpha_syn, v_init, i_init)
-py::tuple layer_lif_backward(const Tensor &grad_spikes, const Maybe &grad_v_last, const Maybe &grad_i_last, const Tensor &input,
+Five layer_lif_backward(const Tensor &grad_spikes, const Maybe &grad_v_last, const Maybe &grad_i_last, const Tensor &input,
                              const Maybe &ckpt_v, const Maybe &ckpt_i, const Maybe &v_init, const Maybe &i_init,
                              const Tensor &alpha_mem, const Maybe &alpha_syn, const Tensor &subtract, const Tensor &theta,
                              const Maybe &theta_low, bool apply_low, int64_t max_spikes, bool decay_early, bool norm_input,
@@ -326,11 +335,11 @@ py::tuple layer_lif_backward(const Tensor &grad_spikes, const Maybe &grad_v_last
                 out(grad_input), out(am_g), out(as_g), out(v0_g), out(i0_g), gs, gvl, gil, x, cv, ci, v0, i0, am, as, c, th, lo,
                 apply_low, spikes, decay_early, norm_input, kind, f0, f1, surr, gvr, gir, uniform, b, t, m, stream);
         });
-    return py::make_tuple(grad_input, am_g, as_g, v0_g, i0_g);
+    return {grad_input, am_g, as_g, v0_g, i0_g};
 }
 
 // -> (out, v_last, total)
-py::tuple layer_leaky_forward(const Tensor &input, const Tensor &v_init, const Tensor &alpha, bool decay_early, bool norm_input,
+Three layer_leaky_forward(const Tensor &input, const Tensor &v_init, const Tensor &alpha, bool decay_early, bool norm_input,
                               const std::optional<Shape> &state_shape, bool want_sum, const py::object &place)
 {
     three(input, "input");
@@ -346,11 +355,11 @@ py::tuple layer_leaky_forward(const Tensor &input, const Tensor &v_init, const T
                                                     input.const_data_ptr<float>(), v0, a, decay_early, norm_input, b, t, m,
                                                     stream);
     });
-    return py::make_tuple(result, v_last, total);
+    return {result, v_last, total};
 }
 
 // -> (grad_input, alpha, v_init)
-py::tuple layer_leaky_backward(const Tensor &grad_out, const Maybe &grad_v_last, const Maybe &forward_out, const Maybe &input,
+Three layer_leaky_backward(const Tensor &grad_out, const Maybe &grad_v_last, const Maybe &forward_out, const Maybe &input,
                                const Maybe &v_init, const Tensor &alpha, bool decay_early, bool norm_input, bool want_alpha,
                                const std::optional<Shape> &uniform_shape, const py::object &place)
 {
@@ -389,18 +398,18 @@ py::tuple layer_leaky_backward(const Tensor &grad_out, const Maybe &grad_v_last,
         return lib.exodus_layer_leaky_backward(out(grad_input), out(a_g), out(v0_g), grad_out.const_data_ptr<float>(), gvl, o, x,
                                                v0, a, decay_early, norm_input, uniform, b, t, m, stream);
     });
-    return py::make_tuple(grad_input, a_g, v0_g);
+    return {grad_input, a_g, v0_g};
 }
 
 // -> (alpha, copy of tau)
-py::tuple decay_expand(const Tensor &tau, int64_t batch, int64_t neurons)
+Two decay_expand(const Tensor &tau, int64_t batch, int64_t neurons)
 {
     dev(tau, "tau");
     const Tensor alpha = fresh({batch * neurons}, tau), kept = fresh(tau.sizes(), tau);
     launch(tau, "exodus_decay_expand", [&](void *stream) {
         return lib.exodus_decay_expand(out(alpha), out(kept), tau.const_data_ptr<float>(), batch, neurons, tau.numel(), stream);
     });
-    return py::make_tuple(alpha, kept);
+    return {alpha, kept};
 }
 
 Tensor decay_grad(const Tensor &grad_alpha, const Tensor &tau, int64_t batch, int64_t neurons)
@@ -499,7 +508,7 @@ Tensor per_row(const Tensor &alpha, int64_t n, int64_t t)
 }
 
 // -> (grad_input, alpha, v_init)
-py::tuple lif_backward_fused(const Tensor &grad_spikes, const Maybe &grad_vmem, const Tensor &v_mem, const Maybe &v_init,
+Three lif_backward_fused(const Tensor &grad_spikes, const Maybe &grad_vmem, const Tensor &v_mem, const Maybe &v_init,
                              const Tensor &alpha, const Tensor &subtract, const Tensor &theta, const Maybe &theta_low,
                              bool apply_low, int64_t max_spikes, int kind, double p0, double p1, const Maybe &surr_given,
                              bool want_alpha, const Maybe &grad_input_given, const py::object &place)
@@ -521,7 +530,7 @@ py::tuple lif_backward_fused(const Tensor &grad_spikes, const Maybe &grad_vmem, 
                                              a, c, th, lo, apply_low, static_cast<int>(max_spikes), kind,
                                              static_cast<float>(p0), static_cast<float>(p1), n, t, stream);
     });
-    return py::make_tuple(grad_input, a_g, v0_g);
+    return {grad_input, a_g, v0_g};
 }
 
 Tensor leaky_forward(const Tensor &input, const Tensor &v_init, const Tensor &alpha, const Maybe &given, const py::object &place)
@@ -538,7 +547,7 @@ Tensor leaky_forward(const Tensor &input, const Tensor &v_init, const Tensor &al
 }
 
 // -> (grad_input, alpha, v_init)
-py::tuple leaky_backward_fused(const Tensor &grad_out, const Tensor &alpha, const Maybe &forward_out, const Maybe &v_init,
+Three leaky_backward_fused(const Tensor &grad_out, const Tensor &alpha, const Maybe &forward_out, const Maybe &v_init,
                                bool want_alpha, const Maybe &grad_input_given, const py::object &place)
 {
     two(grad_out, "outputGrad");
@@ -553,7 +562,7 @@ py::tuple leaky_backward_fused(const Tensor &grad_out, const Tensor &alpha, cons
         return lib.exodus_leaky_backward_fused(out(grad_input), out(a_g), out(v0_g), grad_out.const_data_ptr<float>(), o, v0, a, n,
                                                t, stream);
     });
-    return py::make_tuple(grad_input, a_g, v0_g);
+    return {grad_input, a_g, v0_g};
 }
 
 }  // namespace
@@ -562,15 +571,18 @@ PYBIND11_MODULE(_exodus_torch, module)
 {
     // torch's own exceptions reach the caller as what they are (out of memory as torch.OutOfMemoryError)
     module.def("bind", torch::wrap_pybind_function(bind));
-    module.def("layer_lif_forward", torch::wrap_pybind_function(layer_lif_forward));
-    module.def("layer_lif_backward", torch::wrap_pybind_function(layer_lif_backward));
-    module.def("layer_leaky_forward", torch::wrap_pybind_function(layer_leaky_forward));
-    module.def("layer_leaky_backward", torch::wrap_pybind_function(layer_leaky_backward));
+    // The calls run without the interpreter lock from their checks to their launch: an allocation may have to free memory and
+    // wait for the device, and other Python threads go on meanwhile.  One release for all of it, as taking the lock back is what
+    // a busy interpreter makes a caller wait for.
+    module.def("layer_lif_forward", torch::wrap_pybind_function_no_gil(layer_lif_forward));
+    module.def("layer_lif_backward", torch::wrap_pybind_function_no_gil(layer_lif_backward));
+    module.def("layer_leaky_forward", torch::wrap_pybind_function_no_gil(layer_leaky_forward));
+    module.def("layer_leaky_backward", torch::wrap_pybind_function_no_gil(layer_leaky_backward));
     module.def("stamps", torch::wrap_pybind_function(stamps));
-    module.def("decay_expand", torch::wrap_pybind_function(decay_expand));
-    module.def("decay_grad", torch::wrap_pybind_function(decay_grad));
-    module.def("lif_forward", torch::wrap_pybind_function(lif_forward));
-    module.def("lif_backward_fused", torch::wrap_pybind_function(lif_backward_fused));
-    module.def("leaky_forward", torch::wrap_pybind_function(leaky_forward));
-    module.def("leaky_backward_fused", torch::wrap_pybind_function(leaky_backward_fused));
+    module.def("decay_expand", torch::wrap_pybind_function_no_gil(decay_expand));
+    module.def("decay_grad", torch::wrap_pybind_function_no_gil(decay_grad));
+    module.def("lif_forward", torch::wrap_pybind_function_no_gil(lif_forward));
+    module.def("lif_backward_fused", torch::wrap_pybind_function_no_gil(lif_backward_fused));
+    module.def("leaky_forward", torch::wrap_pybind_function_no_gil(leaky_forward));
+    module.def("leaky_backward_fused", torch::wrap_pybind_function_no_gil(leaky_backward_fused));
 }

@@ -5,6 +5,7 @@ import os
 import subprocess
 import sys
 import threading
+import time
 
 import pytest
 import torch
@@ -97,6 +98,47 @@ def test_running_out_of_memory_is_torchs_exception():
     with pytest.raises(torch.OutOfMemoryError):
         hip().decayExpand(tau, 1 << 40, 1)
     assert hip().decayExpand(tau, 4, 1)[0].shape == (4,)
+
+
+@pytest.mark.gpu
+def test_other_threads_run_while_an_allocation_waits():
+    """The allocator at its limit gives cached memory back, for which it waits for the device: here for a kernel of half a second."""
+    tau = torch.ones(1).cuda()
+    began, ended = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    torch.cuda._sleep(1000)
+    began.record()
+    torch.cuda._sleep(10_000_000)
+    ended.record()
+    torch.cuda.synchronize()
+    cycles = int(10_000_000 * 500 / began.elapsed_time(ended))
+    torch.cuda.empty_cache()
+    torch.empty(1 << 30, dtype=torch.uint8, device="cuda")                 # cached, free
+    gaps, stop = [], threading.Event()
+
+    def tick():
+        last = time.perf_counter()
+        while not stop.is_set():
+            time.sleep(0.002)
+            now = time.perf_counter()
+            gaps.append(now - last)
+            last = now
+
+    other = threading.Thread(target=tick)
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (64 << 20)) / total)
+    try:
+        other.start()
+        torch.cuda._sleep(cycles)
+        start = time.perf_counter()
+        with pytest.raises(torch.OutOfMemoryError):
+            hip().decayExpand(tau, 1 << 31, 1)
+        waited = time.perf_counter() - start
+    finally:
+        stop.set()
+        other.join()
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        torch.cuda.synchronize()
+    assert waited > 0.2 and max(gaps) < waited / 2, (waited, max(gaps))
 
 
 @pytest.mark.gpu
