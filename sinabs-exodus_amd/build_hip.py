@@ -33,6 +33,13 @@ FLAGS = [
 ]
 
 
+def built_for() -> str:
+    """What the host side of the calls is compiled against and works with: torch's C++ interfaces change with its version."""
+    import torch
+
+    return f"torch {torch.__version__}, Python {sys.version_info[0]}.{sys.version_info[1]};"
+
+
 def _torch_command(out: str) -> list:
     import sysconfig
 
@@ -43,16 +50,23 @@ def _torch_command(out: str) -> list:
                "-DUSE_ROCM"]
     for path in cpp_extension.include_paths() + [sysconfig.get_paths()["include"], os.path.join(rocm, "include")]:
         command += ["-isystem", path]
-    command += ["-I", INCLUDE, TORCH_SRC, "-o", out]
+    command += [f'-DEXODUS_BUILT_FOR="{built_for()}"', "-I", INCLUDE, TORCH_SRC, "-o", out]
     command += ["-L" + path for path in cpp_extension.library_paths()]
     return command + ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
 
 
-def build(force: bool = True) -> str:
+def up_to_date() -> bool:
+    """Whether everything is built, from the sources as they are and for the torch and Python that are running."""
     deps = SRCS + [PROBE_SRC, TORCH_SRC, os.path.join(HERE, "csrc", "exodus_common.hpp"), os.path.join(HERE, "csrc", "exodus_layer.hpp"), os.path.join(INCLUDE, "exodus_hip.h")]
     outs = (OUT, PROBE_OUT, TORCH_OUT)
-    if (not force and all(os.path.exists(o) for o in outs)
-            and min(os.path.getmtime(o) for o in outs) >= max(os.path.getmtime(d) for d in deps)):
+    if not all(os.path.exists(o) for o in outs) or min(map(os.path.getmtime, outs)) < max(map(os.path.getmtime, deps)):
+        return False
+    with open(TORCH_OUT, "rb") as module:
+        return built_for().encode() in module.read()
+
+
+def build(force: bool = True) -> str:
+    if not force and up_to_date():
         return OUT
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     # hipcc's host pass does not know the gfx-only target feature and says so; that line is harmless

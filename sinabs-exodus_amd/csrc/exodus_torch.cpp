@@ -569,6 +569,7 @@ Three leaky_backward_fused(const Tensor &grad_out, const Tensor &alpha, const Ma
 
 PYBIND11_MODULE(_exodus_torch, module)
 {
+    module.attr("built_for") = EXODUS_BUILT_FOR;                // the loader compares it with what is running
     // torch's own exceptions reach the caller as what they are (out of memory as torch.OutOfMemoryError)
     module.def("bind", torch::wrap_pybind_function(bind));
     // The calls run without the interpreter lock from their checks to their launch: an allocation may have to free memory and

@@ -12,6 +12,7 @@ from __future__ import annotations
 import ctypes
 import math
 import os
+import sys
 from typing import Optional
 
 import torch  # must be imported before the library so both share one HIP runtime
@@ -120,8 +121,11 @@ def _dev(x: torch.Tensor, name: str, like: Optional[torch.Tensor] = None) -> tor
 
 def _native_module():
     """The host side of the calls in native code, given this library's entry points."""
+    running = f"torch {torch.__version__}, Python {sys.version_info[0]}.{sys.version_info[1]};"
     try:
         from . import _exodus_torch as native
+        if native.built_for != running:        # torch's C++ interfaces change with its version
+            raise ImportError(f"it was built for {native.built_for} this is {running}")
     except ImportError as err:
         raise ImportError(f"{os.path.join(_HERE, '_exodus_torch.so')} cannot be loaded ({err}). Build it with "
                           "`python build_hip.py` in the package root.") from err

@@ -1,6 +1,7 @@
 """The native host side of the kernel calls: what it refuses, which exceptions callers see, and calls from several threads on
 several streams at once."""
 import ctypes
+import importlib.util
 import os
 import subprocess
 import sys
@@ -63,6 +64,25 @@ def test_library_without_an_entry_point_is_named():
                          env={**os.environ, "EXODUS_HIP_LIBRARY": os.path.abspath(probes),
                               "PYTHONPATH": os.path.join(os.path.dirname(hip().__file__), "..", "..")})
     assert got.returncode != 0 and "ImportError" in got.stderr and "exodus_check_parameters" in got.stderr, got.stderr
+
+
+def builder():
+    path = os.path.join(os.path.dirname(hip().__file__), "..", "..", "build_hip.py")
+    spec = importlib.util.spec_from_file_location("build_hip_under_test", path)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
+
+
+def test_module_built_for_another_torch_is_refused_and_built_again(monkeypatch):
+    build_hip, h = builder(), hip()
+    assert h._native.built_for == build_hip.built_for()
+    monkeypatch.setattr(build_hip.os.path, "getmtime", lambda path: 0.0)    # as if no source had changed
+    assert build_hip.up_to_date()
+    monkeypatch.setattr(torch, "__version__", "1.13.1")
+    assert not build_hip.up_to_date()
+    with pytest.raises(ImportError, match="torch 1.13.1.*[Bb]uild it"):
+        h._native_module()
 
 
 @pytest.mark.gpu
