@@ -86,9 +86,11 @@ def build(force: bool = True) -> str:
                                       text=True))
         outputs = [proc.communicate()[0] for proc in procs]
         log = "\n".join(filter(None, (quiet(o).strip() for o in outputs)))
-        if any(proc.returncode != 0 for proc in procs):
+        failed = [f"{os.path.basename(proc.args[0])} failed compiling {os.path.basename(src)}"
+                  for proc, src in zip(procs, SRCS + [PROBE_SRC, TORCH_SRC]) if proc.returncode != 0]
+        if failed:
             sys.stderr.write(log + "\n")
-            raise RuntimeError("hipcc failed compiling libexodus_hip.so / libexodus_bench_probes.so / _exodus_torch.so")
+            raise RuntimeError("; ".join(failed))
         link = subprocess.run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", OUT + ".tmp"] + objs,
                               stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
         log = "\n".join(filter(None, (log, quiet(link.stdout).strip())))

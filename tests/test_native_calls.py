@@ -85,6 +85,18 @@ def test_module_built_for_another_torch_is_refused_and_built_again(monkeypatch):
         h._native_module()
 
 
+def test_build_failure_names_compiler_and_source(monkeypatch, tmp_path):
+    build_hip = builder()
+    broken = tmp_path / "broken.cpp"
+    broken.write_text("#error on purpose\n")
+    monkeypatch.setattr(build_hip, "SRCS", [])
+    monkeypatch.setattr(build_hip, "TORCH_SRC", str(broken))
+    for name in ("OUT", "PROBE_OUT", "TORCH_OUT"):
+        monkeypatch.setattr(build_hip, name, str(tmp_path / name))
+    with pytest.raises(RuntimeError, match=r"^g\+\+ failed compiling broken.cpp$"):
+        build_hip.build()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", NAMES)
 def test_wrong_types_shapes_and_strides(name):
