@@ -59,6 +59,22 @@ def test_parameter_given_other_memory():
         layer.spike_threshold.data = torch.zeros(3)
 
 
+def test_attribute_found_by_a_rule_of_the_class():
+    import sinabs.exodus.layers as el
+
+    class Shared(el.LIF):
+        settings = {"min_v_mem": -1.0}
+
+        def __getattr__(self, name):
+            return self.settings[name] if name in self.settings else super().__getattr__(name)
+
+    layer = Shared(tau_mem=20.0)
+    del layer.min_v_mem
+    for low in (-1.0, -2.0, -3.0):
+        layer.settings["min_v_mem"] = low
+        assert torch.equal(vectors(layer, 8)[2], torch.full((8,), low))
+
+
 def test_kept_while_nothing_changes_and_not_in_copies():
     layer = layer_with(min_v_mem=-1.0)
     first = vectors(layer, 8)
