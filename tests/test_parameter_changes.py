@@ -75,6 +75,30 @@ def test_attribute_found_by_a_rule_of_the_class():
         assert torch.equal(vectors(layer, 8)[2], torch.full((8,), low))
 
 
+@pytest.mark.parametrize("kind", ["LIF", "IAF"])
+def test_decay_factor_by_a_rule_of_the_class(kind):
+    import sinabs.exodus.layers as el
+
+    class Own(getattr(el, kind)):
+        @property
+        def alpha_mem_calculated(self):
+            return torch.sigmoid(self.w)
+
+    layer = Own(**dict(tau_mem=20.0) if kind == "LIF" else {})
+    layer.w = torch.nn.Parameter(torch.zeros(()))
+    shape, dev = (1, 8), torch.device("cpu")
+    seen = []
+    for w in (0.0, 1.0, 2.0):
+        with torch.no_grad():
+            layer.w.fill_(w)
+            stamps = layer._parameter_stamps()
+            assert not any(stamps is s for s in seen)          # the range check is not skipped
+            seen.append(stamps)
+            assert torch.equal(layer._decay_factor("mem", stamps, shape, dev, False), torch.sigmoid(torch.full((8,), w)))
+    layer._decay_factor("mem", layer._parameter_stamps(), shape, dev, False).sum().backward()
+    assert layer.w.grad is not None and layer.w.grad != 0
+
+
 def test_kept_while_nothing_changes_and_not_in_copies():
     layer = layer_with(min_v_mem=-1.0)
     first = vectors(layer, 8)
