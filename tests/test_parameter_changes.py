@@ -142,3 +142,25 @@ def test_the_range_check_sees_every_change():
             layer.parametrizations.spike_threshold.original.fill_(-1.0)
             with pytest.raises(ValueError, match="greater than"):
                 layer(x)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", ["tau_mem", "tau_syn"])
+def test_gradient_of_a_parametrized_time_constant(which):
+    """Also where nothing else asks for one: an input without a gradient, no trained parameter of the layer's own."""
+    x = torch.rand(3, 20, 40).cuda()
+    grads = []
+    for parametrized in (False, True):
+        layer = layer_with(tau_mem=20.0, tau_syn=10.0).cuda().requires_grad_(False)
+        if parametrized:
+            parametrize.register_parametrization(layer, which, Scaled())
+            wanted = layer.parametrizations[which].original
+            with torch.no_grad():
+                wanted.mul_(0.5)
+        else:
+            wanted = getattr(layer, which)
+        wanted.requires_grad_(True)
+        layer(x).square().sum().backward()
+        grads.append(wanted.grad)
+    # the chain rule's factor of two is exact; the two gradients add the neurons up in another order
+    assert grads[0].abs() > 0 and torch.allclose(grads[1], 2.0 * grads[0], rtol=1e-5)
