@@ -24,8 +24,8 @@ def vectors(layer, n):
         stamps = layer._parameter_stamps()
         low = layer.min_v_mem
         return (layer._decay_factor("mem", stamps, shape, dev, False),
-                layer._per_neuron("spike_threshold", layer.spike_threshold, stamps[4], shape, dev, False),
-                None if low is None else layer._per_neuron("min_v_mem", low, stamps[5], shape, dev, False))
+                layer._per_neuron("spike_threshold", layer.spike_threshold, stamps[2], shape, dev, False),
+                None if low is None else layer._per_neuron("min_v_mem", low, stamps[3], shape, dev, False))
 
 
 @pytest.mark.parametrize("n", [64, 4096, 65536])
