@@ -148,6 +148,15 @@ def _mat(x: torch.Tensor, name: str, n: int, t: int) -> torch.Tensor:
     return x
 
 
+def _cap(spikes: int) -> int:
+    """Most spikes per step as the C ABI takes it: an int whose bits are an unsigned number, -1 = no limit.  No count reaches a
+    limit beyond 32 bits."""
+    spikes = int(spikes)
+    if spikes < 1 << 31:
+        return spikes
+    return spikes - (1 << 32) if spikes < 1 << 32 else -1
+
+
 def _ptr(x: Optional[torch.Tensor]):
     return None if x is None else x.data_ptr()             # ctypes takes a plain integer for a void pointer
 
@@ -198,7 +207,7 @@ def lifForward(outputSpikes, vmem, input, vmemPostInitial, alpha, membrSubtract,
                applyThetaLow: bool, maxNumSpikes: int) -> None:
     """reference cuda/bindings.cu:14-70; fills the caller-allocated ``outputSpikes`` and ``vmem``."""
     _native.lif_forward(outputSpikes, vmem, input, vmemPostInitial, alpha, membrSubtract, theta, thetaLow,
-                        bool(applyThetaLow), int(maxNumSpikes))
+                        bool(applyThetaLow), _cap(maxNumSpikes))
 
 
 def lifBackward(surr, outputGrad, notClipped, alpha, membrSubtract) -> torch.Tensor:
@@ -286,7 +295,7 @@ def spikeForward(vmem, alpha: float, membrSubtract: float, theta: float, thetaLo
     spikes = hbm.empty_like(vmem)
     with _on_device_of(vmem.device):
         _check(lib.exodus_spike_forward(_ptr(spikes), _ptr(vmem), float(alpha), float(membrSubtract), float(theta),
-                                        float(thetaLow), int(bool(applyThetaLow)), int(maxNumSpikes), n, t,
+                                        float(thetaLow), int(bool(applyThetaLow)), _cap(maxNumSpikes), n, t,
                                         _stream(vmem)), "exodus_spike_forward")
     return spikes
 
@@ -327,7 +336,7 @@ def lifBackwardFused(gradSpikes, gradVmem, vmem, vmemPostInitial, alpha, membrSu
     ``membrSubtract`` is the plain subtract value here (not pre-multiplied by alpha).
     """
     return _native.lif_backward_fused(gradSpikes, gradVmem, vmem, vmemPostInitial, alpha, membrSubtract, theta, thetaLow,
-                                      bool(applyThetaLow), int(maxNumSpikes), int(surrogateKind), float(surrP0),
+                                      bool(applyThetaLow), _cap(maxNumSpikes), int(surrogateKind), float(surrP0),
                                       float(surrP1), surr, bool(needAlphaGrad), inputGrad, _place(vmem))
 
 
@@ -354,7 +363,7 @@ def synLifForward(input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, membr
     with _on_device_of(input.device):
         _check(lib.exodus_synlif_forward(_ptr(spikes), _ptr(vmem), _ptr(isyn), _ptr(input), _ptr(vmemPostInitial),
                                          _ptr(isynInitial), _ptr(alphaMem), _ptr(alphaSyn), _ptr(membrSubtract),
-                                         _ptr(theta), _ptr(thetaLow), int(bool(applyThetaLow)), int(maxNumSpikes),
+                                         _ptr(theta), _ptr(thetaLow), int(bool(applyThetaLow)), _cap(maxNumSpikes),
                                          int(bool(decayEarly)), int(bool(normInput)), n, t, _stream(input)),
                "exodus_synlif_forward")
     return spikes, vmem, isyn
@@ -393,7 +402,7 @@ def synLifBackward(gradSpikes, gradVmem, gradIsyn, vmem, isyn, vmemPostInitial, 
                                           _ptr(gradVmem), _ptr(gradIsyn), _ptr(vmem), _ptr(isyn),
                                           _ptr(vmemPostInitial), _ptr(isynInitial), _ptr(alphaMem), _ptr(alphaSyn),
                                           _ptr(membrSubtract), _ptr(theta), _ptr(thetaLow),
-                                          int(bool(applyThetaLow)), int(maxNumSpikes), int(bool(decayEarly)),
+                                          int(bool(applyThetaLow)), _cap(maxNumSpikes), int(bool(decayEarly)),
                                           int(bool(normInput)), int(surrogateKind), float(surrP0), float(surrP1),
                                           n, t, _stream(vmem)), "exodus_synlif_backward")
     return (inputGrad, *per_row)
@@ -428,7 +437,7 @@ def layerLifForward(input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, mem
     ``wantPreReset`` records only the potential, before the reset (the surrogate function's argument)."""
     return dict(zip(_LAYER_LIF_OUTPUTS, _native.layer_lif_forward(
         input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, membrSubtract, theta, thetaLow, bool(applyThetaLow),
-        int(maxNumSpikes), bool(decayEarly), bool(normInput), bool(wantCheckpoints), bool(wantRecords), bool(wantPreReset),
+        _cap(maxNumSpikes), bool(decayEarly), bool(normInput), bool(wantCheckpoints), bool(wantRecords), bool(wantPreReset),
         bool(wantSpikeSum), outSpikes, stateShape, _place(input))))
 
 
@@ -480,7 +489,7 @@ def layerLifBackward(gradSpikes, gradVLast, gradILast, input, ckptV, ckptI, vmem
     own fixed device array (``scratchFloats()``) and allocates nothing; concurrent calls on one GPU must not overlap."""
     return _native.layer_lif_backward(
         gradSpikes, gradVLast, gradILast, input, ckptV, ckptI, vmemPostInitial, isynInitial, alphaMem, alphaSyn, membrSubtract,
-        theta, thetaLow, bool(applyThetaLow), int(maxNumSpikes), bool(decayEarly), bool(normInput), int(surrogateKind),
+        theta, thetaLow, bool(applyThetaLow), _cap(maxNumSpikes), bool(decayEarly), bool(normInput), int(surrogateKind),
         float(surrP0), float(surrP1), gradInput, surr, gradVRec, gradIRec, bool(wantAlphaMemGrad), bool(wantAlphaSynGrad),
         bool(wantVInitGrad), bool(wantIInitGrad), bool(gradUniform), _place(input))
 

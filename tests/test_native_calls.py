@@ -47,6 +47,27 @@ def test_tensors_that_are_not_on_the_gpu_and_things_that_are_no_tensors(name):
         calls([0.0], [0.0], [0.0])[name]()
 
 
+@pytest.mark.parametrize("most,bits", [(-1, -1), (0, 0), (7, 7), (2 ** 31 - 1, 2 ** 31 - 1), (2 ** 31, -2 ** 31),
+                                       (2 ** 32 - 2, -2), (2 ** 32 - 1, -1), (2 ** 32, -1), (2 ** 32 + 5, -1), (10 ** 20, -1)])
+def test_spike_limits_of_any_size(most, bits):
+    assert hip()._cap(most) == bits
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("most", [2 ** 31, 2 ** 32, 2 ** 63, 10 ** 20])
+def test_a_limit_that_no_count_reaches(most):
+    import sinabs.exodus.layers as el
+    from sinabs.exodus._compat import MaxSpike, MultiSpike
+    x = (10.0 * torch.rand(2, 20, 30)).cuda()
+    for native in (True, False):
+        outs = []
+        for spike_fn in (MultiSpike, MaxSpike(most)):
+            layer = el.IAF(spike_fn=spike_fn).cuda()
+            layer.native_layout = native
+            outs.append(layer(x))
+        assert outs[0].max() > 2 and torch.equal(*outs)
+
+
 def test_library_of_another_version_is_refused():
     """Neither the Python nor the native half takes it, and the native half keeps the library it has."""
     h, native = hip(), hip()._native
