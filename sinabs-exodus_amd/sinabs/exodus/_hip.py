@@ -201,13 +201,14 @@ def checkParameters(flags, alpha, alphaOther, theta, thetaLow) -> None:
 
 # ------------------------------------------------------------------------------------------
 # the six functions of the reference extension, same names and argument order
+# (an argument that a call does not use is not looked at, here and below: the native calls take tensors or None)
 # ------------------------------------------------------------------------------------------
 
 def lifForward(outputSpikes, vmem, input, vmemPostInitial, alpha, membrSubtract, theta, thetaLow,
                applyThetaLow: bool, maxNumSpikes: int) -> None:
     """reference cuda/bindings.cu:14-70; fills the caller-allocated ``outputSpikes`` and ``vmem``."""
-    _native.lif_forward(outputSpikes, vmem, input, vmemPostInitial, alpha, membrSubtract, theta, thetaLow,
-                        bool(applyThetaLow), _cap(maxNumSpikes))
+    _native.lif_forward(outputSpikes, vmem, input, vmemPostInitial, alpha, membrSubtract, theta,
+                        thetaLow if applyThetaLow else None, bool(applyThetaLow), _cap(maxNumSpikes))
 
 
 def lifBackward(surr, outputGrad, notClipped, alpha, membrSubtract) -> torch.Tensor:
@@ -323,6 +324,8 @@ def spikeBackward(surr, outputGrad, notClipped, alpha: float, membrSubtract: flo
 def leakyBackwardFused(outputGrad, alpha, output=None, vmemInitial=None, needAlphaGrad: bool = False,
                        inputGrad: Optional[torch.Tensor] = None):
     """One reverse pass: returns (inputGrad, alphaGrad | None, initGrad)."""
+    if not needAlphaGrad:
+        output = vmemInitial = None
     return _native.leaky_backward_fused(outputGrad, alpha, output, vmemInitial, bool(needAlphaGrad), inputGrad,
                                         _place(outputGrad))
 
@@ -335,9 +338,10 @@ def lifBackwardFused(gradSpikes, gradVmem, vmem, vmemPostInitial, alpha, membrSu
 
     ``membrSubtract`` is the plain subtract value here (not pre-multiplied by alpha).
     """
-    return _native.lif_backward_fused(gradSpikes, gradVmem, vmem, vmemPostInitial, alpha, membrSubtract, theta, thetaLow,
-                                      bool(applyThetaLow), _cap(maxNumSpikes), int(surrogateKind), float(surrP0),
-                                      float(surrP1), surr, bool(needAlphaGrad), inputGrad, _place(vmem))
+    return _native.lif_backward_fused(gradSpikes, gradVmem, vmem, vmemPostInitial if needAlphaGrad else None, alpha,
+                                      membrSubtract, theta, thetaLow if applyThetaLow else None, bool(applyThetaLow),
+                                      _cap(maxNumSpikes), int(surrogateKind), float(surrP0), float(surrP1),
+                                      surr if surrogateKind == SURR_TENSOR else None, bool(needAlphaGrad), inputGrad, _place(vmem))
 
 
 def synLifForward(input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, membrSubtract, theta, thetaLow,
@@ -436,7 +440,8 @@ def layerLifForward(input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, mem
     ``wantRecords`` records potential (after the reset) and synaptic current of every step;
     ``wantPreReset`` records only the potential, before the reset (the surrogate function's argument)."""
     return dict(zip(_LAYER_LIF_OUTPUTS, _native.layer_lif_forward(
-        input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, membrSubtract, theta, thetaLow, bool(applyThetaLow),
+        input, vmemPostInitial, None if alphaSyn is None else isynInitial, alphaMem, alphaSyn, membrSubtract, theta,
+        thetaLow if applyThetaLow else None, bool(applyThetaLow),
         _cap(maxNumSpikes), bool(decayEarly), bool(normInput), bool(wantCheckpoints), bool(wantRecords), bool(wantPreReset),
         bool(wantSpikeSum), outSpikes, stateShape, _place(input))))
 
@@ -487,9 +492,15 @@ def layerLifBackward(gradSpikes, gradVLast, gradILast, input, ckptV, ckptI, vmem
     missing while the other is given counts as zero.
     ``ckptV is None`` calls ``exodus_layer_lif_backward_from_input``: the library rebuilds the checkpoints in its
     own fixed device array (``scratchFloats()``) and allocates nothing; concurrent calls on one GPU must not overlap."""
+    if alphaSyn is None:
+        gradILast = ckptI = isynInitial = gradIRec = None
+    if ckptV is None:
+        ckptI = None
+    if surrogateKind != SURR_TENSOR:
+        surr = None
     return _native.layer_lif_backward(
         gradSpikes, gradVLast, gradILast, input, ckptV, ckptI, vmemPostInitial, isynInitial, alphaMem, alphaSyn, membrSubtract,
-        theta, thetaLow, bool(applyThetaLow), _cap(maxNumSpikes), bool(decayEarly), bool(normInput), int(surrogateKind),
+        theta, thetaLow if applyThetaLow else None, bool(applyThetaLow), _cap(maxNumSpikes), bool(decayEarly), bool(normInput), int(surrogateKind),
         float(surrP0), float(surrP1), gradInput, surr, gradVRec, gradIRec, bool(wantAlphaMemGrad), bool(wantAlphaSynGrad),
         bool(wantVInitGrad), bool(wantIInitGrad), bool(gradUniform), _place(input))
 
@@ -509,7 +520,9 @@ def layerLeakyBackward(gradOut, gradVLast, out, input, vmemInitial, alpha, decay
     one-element tensor whose value is the gradient of every output (the gradient of a sum)."""
     if shape is not None:
         shape = tuple(int(v) for v in shape)
+    if not needAlphaGrad:
+        out = input = vmemInitial = None
+    elif not (decayEarly or normInput):
+        input = None
     return _native.layer_leaky_backward(gradOut, gradVLast, out, input, vmemInitial, alpha, bool(decayEarly), bool(normInput),
                                         bool(needAlphaGrad), shape, _place(gradOut, shape))
-
-

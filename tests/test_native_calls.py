@@ -47,6 +47,21 @@ def test_tensors_that_are_not_on_the_gpu_and_things_that_are_no_tensors(name):
         calls([0.0], [0.0], [0.0])[name]()
 
 
+@pytest.mark.gpu
+def test_arguments_that_a_call_does_not_use_may_be_anything():
+    h, no = hip(), "nothing"
+    x, r, two = torch.rand(1, 4, 6).cuda(), torch.rand(6).cuda() * 0.5 + 0.3, torch.rand(6, 4).cuda()
+    ck = torch.rand(1, 1, 6).cuda()
+    h.lifForward(two.clone(), two.clone(), two, r, r, r, r, no, False, -1)
+    h.leakyBackwardFused(two, r, no, no, False)
+    h.lifBackwardFused(two, None, two, no, r, r, r, no, False, -1, 1, surr=no)
+    h.layerLifForward(x, r, no, r, None, r, r, no, False, -1, True, True)
+    h.layerLifBackward(x, None, no, x, ck, no, r, no, r, None, r, r, no, False, -1, True, True, 1, 0.5, 1.0, surr=no, gradIRec=no)
+    h.layerLifBackward(x, None, None, x, None, no, r, r, r, r, r, r, no, False, -1, True, True, 1, 0.5, 1.0)
+    h.layerLeakyBackward(x, None, no, no, no, r, True, True, False)
+    h.layerLeakyBackward(x, None, x, no, r, r, False, False, True)
+
+
 @pytest.mark.parametrize("most,bits", [(-1, -1), (0, 0), (7, 7), (2 ** 31 - 1, 2 ** 31 - 1), (2 ** 31, -2 ** 31),
                                        (2 ** 32 - 2, -2), (2 ** 32 - 1, -1), (2 ** 32, -1), (2 ** 32 + 5, -1), (10 ** 20, -1)])
 def test_spike_limits_of_any_size(most, bits):
