@@ -216,6 +216,17 @@ int exodus_layer_lif_forward_total(float *out_spikes, float *out_vmem_rec, float
                                    int record_pre_reset, int64_t batch, int64_t t, int64_t neurons, void *stream);
 int64_t exodus_layer_sum_slots(int64_t batch, int64_t neurons);
 
+/* Neurons per lane and lanes per block that a layer kernel is launched with on the current device, for tensors on 64-byte
+ * boundaries (results do not depend on either).  EXODUS_SHAPE_BACKWARD is the backward with one lane per neuron, whatever
+ * exodus_layer_backward_time_split says. */
+#define EXODUS_SHAPE_FORWARD 0
+#define EXODUS_SHAPE_FORWARD_RECORDS 1
+#define EXODUS_SHAPE_LEAKY_FORWARD 2
+#define EXODUS_SHAPE_LEAKY_BACKWARD 3
+#define EXODUS_SHAPE_LEAKY_BACKWARD_ALPHA 4
+#define EXODUS_SHAPE_BACKWARD 5
+int exodus_layer_launch_shape(int kernel, int64_t batch, int64_t neurons, int *neurons_per_lane, int *lanes);
+
 /* Backward of the above.  Re-reads `input`, rebuilds membrane potential and synaptic current of
  * each checkpoint interval from ckpt_v / ckpt_i and walks it in reverse.  grad_v_last /
  * grad_i_last (batch*neurons, optional) are gradients arriving at the final states.  Outputs:

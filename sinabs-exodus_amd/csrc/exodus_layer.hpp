@@ -312,6 +312,30 @@ inline int lanes_per_block(int64_t batch, int64_t neurons)
     return batch * ((neurons + WAVE - 1) / WAVE) <= 2 * compute_units() ? WAVE : BLOCK;
 }
 
+// What a launch of a forward or leaky kernel looks like.  `widest` is 1 for a kernel that knows no other width.
+struct LaunchShape {
+    int npl, lanes;      // neurons per lane, lanes per block
+};
+
+inline LaunchShape launch_shape(int64_t batch, int64_t neurons, unsigned align, int widest, int waves_per_cu, bool whole)
+{
+    const int npl = pick_neurons_per_lane(batch, neurons, align, widest, waves_per_cu, whole);
+    return {npl, npl == 1 ? lanes_per_block(batch, neurons) : BLOCK};
+}
+
+constexpr int FORWARD_WAVES = 16;
+
+// Lanes per block of the one-lane backward.  One wave per block up to four waves per compute unit, as the forward has it up to
+// two: a unit's way to
+// memory is shared by fewer waves.  256 lanes / 64, us, without synapse: 504 waves (24, 250, 1323) 41.7 / 37.3, 512
+// (32, 250, 1024) 42.9 / 37.3, 1024 (32, 250, 2048) 53.2 / 45.7, 2048 (64, 300, 2048) 95 / 105; with one 57.4 / 52.7,
+// - , 69.0 / 65.0, (16, 300, 8192) 110 / 118; with state records 47.0 / 44.1, 46.6 / 41.1, 59.5 / 56.6, with both 65.4 / 57.3
+// (1024 neurons) and 90.7 / 91.4 (2048).
+inline int backward_lanes(int64_t batch, int64_t neurons)
+{
+    return batch * ((neurons + WAVE - 1) / WAVE) <= 4 * compute_units() ? WAVE : BWD_BLOCK;
+}
+
 inline unsigned common_alignment(std::initializer_list<const void *> ptrs)
 {
     uintptr_t bits = 0;

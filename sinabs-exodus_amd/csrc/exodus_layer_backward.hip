@@ -217,12 +217,7 @@ int launch_bwd(float *grad_x, float *am_g, float *as_g, float *v0_g, float *i0_g
                const float *gir, const float *ckpt_v, const float *ckpt_i, const LayerConsts &p, float p0, float p1,
                bool uniform, int64_t B, int64_t T, int64_t M, hipStream_t s)
 {
-    // One wave per block up to four waves per compute unit, as the forward has it up to two (lanes_per_block): a unit's way to
-    // memory is shared by fewer waves.  256 lanes / 64, us, without synapse: 504 waves (24, 250, 1323) 41.7 / 37.3, 512
-    // (32, 250, 1024) 42.9 / 37.3, 1024 (32, 250, 2048) 53.2 / 45.7, 2048 (64, 300, 2048) 95 / 105; with one 57.4 / 52.7,
-    // - , 69.0 / 65.0, (16, 300, 8192) 110 / 118; with state records 47.0 / 44.1, 46.6 / 41.1, 59.5 / 56.6, with both 65.4 / 57.3
-    // (1024 neurons) and 90.7 / 91.4 (2048).
-    const int lanes = B * ((M + WAVE - 1) / WAVE) <= 4 * compute_units() ? WAVE : BWD_BLOCK;
+    const int lanes = backward_lanes(B, M);
     const int64_t blocks_per_batch = (M + lanes - 1) / lanes;
     if (blocks_per_batch > 0x7fffffffLL / B) return hipErrorInvalidValue;
     const int64_t blocks = blocks_per_batch * B;

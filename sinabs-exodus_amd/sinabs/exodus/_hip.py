@@ -59,6 +59,7 @@ _SIGNATURES = {
     "exodus_layer_leaky_forward_total": ([_p] * 7 + [_int, _int, _i64, _i64, _i64, _p], _int),
     "exodus_layer_leaky_backward": ([_p] * 9 + [_int, _int, _int, _i64, _i64, _i64, _p], _int),
     "exodus_decay_expand": ([_p, _p, _p, _i64, _i64, _i64, _p], _int),
+    "exodus_layer_launch_shape": ([_int, _i64, _i64, _p, _p], _int),
     "exodus_decay_work": ([_i64] * 3, _i64),
     "exodus_decay_grad": ([_p] * 4 + [_i64, _i64, _i64, _p], _int),
     "exodus_hbm_regions_create": ([_int, ctypes.c_uint64, ctypes.c_uint64, ctypes.c_uint64, _int, ctypes.c_uint64, _p], _int),
@@ -449,6 +450,17 @@ def layerLifForward(input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, mem
 # stamps(kept, values): a tuple with one entry per value, the entries of ``kept`` (an earlier result, or None) where a value is
 # unchanged since, and ``kept`` itself where all are
 stamps = _native.stamps
+
+
+_SHAPES = ("forward", "forward records", "leaky forward", "leaky backward", "leaky backward alpha", "backward")
+
+
+def launchShape(kernel: str, batch: int, neurons: int) -> tuple:
+    """(neurons per lane, lanes per block) of a layer kernel's launch: which of its variants a layer of this size gets."""
+    npl, lanes = _int(), _int()
+    _check(lib.exodus_layer_launch_shape(_SHAPES.index(kernel), batch, neurons, ctypes.byref(npl), ctypes.byref(lanes)),
+           "exodus_layer_launch_shape")
+    return npl.value, lanes.value
 
 
 def decayExpand(tau, batch: int, neurons: int):

@@ -6,14 +6,16 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("b,t,m", [
-    (1, 3, 1), (3, 40, 63), (3, 40, 64), (3, 40, 65), (2, 33, 257), (5, 7, 1000),
-    (8, 40, 4096),            # 512 waves: two per compute unit, the last size with one wave per block
-    (8, 40, 4097),            # 520 waves
-    (513, 5, 10), (512, 5, 10),
+@pytest.mark.parametrize("b,t,m,lanes", [
+    (1, 3, 1, 64), (3, 40, 63, 64), (3, 40, 64, 64), (3, 40, 65, 64), (2, 33, 257, 64), (5, 7, 1000, 64),
+    (8, 40, 4096, 64),        # 512 waves: two per compute unit, the last size with one wave per block
+    (8, 40, 4097, 256),       # 520 waves
+    (513, 5, 10, 256), (512, 5, 10, 64),
 ])
-def test_small_and_larger_blocks(b, t, m):
+def test_small_and_larger_blocks(b, t, m, lanes):
     from sinabs.exodus import _hip as hip
+    for kernel in ("forward", "leaky forward", "leaky backward alpha"):
+        assert hip.launchShape(kernel, b, m) == (1, lanes)
     g = torch.Generator(device="cuda").manual_seed(b * m)
     x = torch.empty(b, t, m, device="cuda").normal_(0.2, 0.8, generator=g)
     go = torch.empty(b, t, m, device="cuda").normal_(0.0, 1.0, generator=g)
@@ -36,9 +38,11 @@ def test_small_and_larger_blocks(b, t, m):
             assert torch.equal(p[k] if p.ndim == 3 else p[k * m:(k + 1) * m], q[0] if q.ndim == 3 else q)
 
 
-@pytest.mark.parametrize("b,t,m", [(2, 40, 8200), (16, 40, 4096), (16, 40, 4097)])   # 258, 1024 and 1040 waves
-def test_one_lane_backward_with_both_blocks(b, t, m):
+# 258, 1024 and 1040 waves
+@pytest.mark.parametrize("b,t,m,lanes", [(2, 40, 8200, 64), (16, 40, 4096, 64), (16, 40, 4097, 256)])
+def test_one_lane_backward_with_both_blocks(b, t, m, lanes):
     from sinabs.exodus import _hip as hip
+    assert hip.launchShape("backward", b, m) == (1, lanes)
     g = torch.Generator(device="cuda").manual_seed(m)
     x = torch.empty(b, t, m, device="cuda").normal_(0.2, 0.8, generator=g)
     go = torch.empty(b, t, m, device="cuda").normal_(0.0, 1.0, generator=g)
