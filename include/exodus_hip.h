@@ -217,14 +217,16 @@ int exodus_layer_lif_forward_total(float *out_spikes, float *out_vmem_rec, float
 int64_t exodus_layer_sum_slots(int64_t batch, int64_t neurons);
 
 /* Neurons per lane and lanes per block that a layer kernel is launched with on the current device, for tensors on 64-byte
- * boundaries (results do not depend on either).  EXODUS_SHAPE_BACKWARD is the backward with one lane per neuron, whatever
- * exodus_layer_backward_time_split says. */
+ * boundaries (results do not depend on either).  EXODUS_SHAPE_FORWARD_RECORDS records potential and current,
+ * EXODUS_SHAPE_BACKWARD is the backward with one lane per neuron, whatever exodus_layer_backward_time_split says,
+ * EXODUS_SHAPE_BACKWARD_MORE the one with gradients on state records or a surrogate tensor. */
 #define EXODUS_SHAPE_FORWARD 0
 #define EXODUS_SHAPE_FORWARD_RECORDS 1
 #define EXODUS_SHAPE_LEAKY_FORWARD 2
 #define EXODUS_SHAPE_LEAKY_BACKWARD 3
 #define EXODUS_SHAPE_LEAKY_BACKWARD_ALPHA 4
 #define EXODUS_SHAPE_BACKWARD 5
+#define EXODUS_SHAPE_BACKWARD_MORE 6
 int exodus_layer_launch_shape(int kernel, int64_t batch, int64_t neurons, int *neurons_per_lane, int *lanes);
 
 /* Backward of the above.  Re-reads `input`, rebuilds membrane potential and synaptic current of

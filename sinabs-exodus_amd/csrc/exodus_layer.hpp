@@ -302,14 +302,30 @@ inline int pick_neurons_per_lane(int64_t batch, int64_t neurons, unsigned align,
     return 1;
 }
 
-// Lanes per block of the forward and leaky kernels.  Four waves that keep each other at the same step suit memory (see the
-// barriers); but up to two waves per compute unit they only crowd on a few units, whose way to memory their accesses then
-// share, while the others stand idle: one wave per block there, which also leaves no wave without a neuron.  256 / 64 lanes,
-// us, spiking (at most one spike) and leaky forward: (4, 2000, 512) 96.6 / 70.4 and 80.0 / 55.6, (64, 300, 10) 20.2 / 16.1 and
-// 15.0 / 11.3, (24, 250, 1323) with 504 waves 20.9 / 20.2 and 15.7 / 16.7, (32, 250, 2048) with 1024 26.9 / 30.3 and 23.7 / 26.3.
-inline int lanes_per_block(int64_t batch, int64_t neurons)
+// Lanes per block.  Four waves that keep each other at the same step suit memory (see the barriers); but up to a few waves per
+// compute unit they only crowd on a few units, whose way to memory their accesses then share, while the others stand idle: one
+// wave per block there, which also leaves no wave without a neuron.  `half_waves`: half waves per compute unit up to which.
+inline int lanes_per_block(int64_t batch, int64_t neurons, int half_waves)
 {
-    return batch * ((neurons + WAVE - 1) / WAVE) <= 2 * compute_units() ? WAVE : BLOCK;
+    return 2 * batch * ((neurons + WAVE - 1) / WAVE) <= half_waves * compute_units() ? WAVE : BLOCK;
+}
+
+// Forward and leaky kernels: two waves per compute unit.  256 / 64 lanes, us, spiking (at most one spike) and leaky forward, the
+// same tensors again and again: (4, 2000, 512) 96.6 / 70.4 and 80.0 / 55.6, (64, 300, 10) 20.2 / 16.1 and 15.0 / 11.3,
+// (24, 250, 1323) with 504 waves 20.9 / 20.2 and 15.7 / 16.7, (32, 250, 2048) with 1024 26.9 / 30.3 and 23.7 / 26.3; other
+// tensors in every call, so that they come from memory: (24, 250, 1323) 26.9 / 25.8 and 25.9 / 24.8, (24, 1000, 1323)
+// 86.0 / 82.2 and 83.3 / 79.9, (8, 500, 4090) with 512 waves 44.4 / 43.2 and 42.6 / 41.5, (32, 250, 1024) 20.1 / 18.5 and
+// 19.3 / 17.3.
+constexpr int FORWARD_HALF_WAVES = 4;
+// The spiking forward that records both states moves four tensors.  Where its steps do not fill whole sectors (`whole` false) and
+// blocks are neighbours in a step, blocks of one wave share more sectors than blocks of four, and only one and a half pay.
+// 256 / 64, us, other tensors in every call: 512 waves (8, 500, 4090) 87 / 97, (64, 200, 500) 42.1 / 44.5, 504 (24, 1000, 1323)
+// 168 / 189, (24, 250, 1323) 50.2 / 54.6, 500 (250, 200, 100) 38.0 / 40.2, 448 (7, 500, 4090) 85 / 89, 384 (6, 500, 4090)
+// 83.2 / 82.2, (24, 300, 1000) 54.7 / 54.3; whole sectors, 512 (32, 250, 1024) 43.5 / 42.6; one wave per element (500, 200, 40)
+// 44.1 / 37.1.
+inline int forward_half_waves(int64_t neurons, bool both_records, bool whole)
+{
+    return both_records && !whole && neurons > WAVE ? 3 : FORWARD_HALF_WAVES;
 }
 
 // What a launch of a forward or leaky kernel looks like.  `widest` is 1 for a kernel that knows no other width.
@@ -317,23 +333,29 @@ struct LaunchShape {
     int npl, lanes;      // neurons per lane, lanes per block
 };
 
-inline LaunchShape launch_shape(int64_t batch, int64_t neurons, unsigned align, int widest, int waves_per_cu, bool whole)
+inline LaunchShape launch_shape(int64_t batch, int64_t neurons, unsigned align, int widest, int waves_per_cu, bool whole,
+                                int half_waves = FORWARD_HALF_WAVES)
 {
     const int npl = pick_neurons_per_lane(batch, neurons, align, widest, waves_per_cu, whole);
-    return {npl, npl == 1 ? lanes_per_block(batch, neurons) : BLOCK};
+    return {npl, npl == 1 ? lanes_per_block(batch, neurons, half_waves) : BLOCK};
 }
 
 constexpr int FORWARD_WAVES = 16;
 
-// Lanes per block of the one-lane backward.  One wave per block up to four waves per compute unit, as the forward has it up to
-// two: a unit's way to
-// memory is shared by fewer waves.  256 lanes / 64, us, without synapse: 504 waves (24, 250, 1323) 41.7 / 37.3, 512
-// (32, 250, 1024) 42.9 / 37.3, 1024 (32, 250, 2048) 53.2 / 45.7, 2048 (64, 300, 2048) 95 / 105; with one 57.4 / 52.7,
-// - , 69.0 / 65.0, (16, 300, 8192) 110 / 118; with state records 47.0 / 44.1, 46.6 / 41.1, 59.5 / 56.6, with both 65.4 / 57.3
-// (1024 neurons) and 90.7 / 91.4 (2048).
-inline int backward_lanes(int64_t batch, int64_t neurons)
+// The one-lane backward: one wave per block up to four waves per compute unit.  256 lanes / 64, us, other tensors in every call,
+// without and with a synapse: 504 waves (24, 250, 1323) 49.3 / 41.4 and 63.1 / 57.5, 1024 (32, 250, 2048) 54.0 / 46.3 and
+// 67.1 / 64.4, (16, 500, 4096) 94.7 / 82.6 and 122 / 115; 2048 (the same tensors) (64, 300, 2048) 95 / 105 and
+// (16, 300, 8192) 110 / 118.
+// More tensors (gradients on state records, a surrogate tensor: `extra`) leave it at that where steps fill whole sectors: records
+// and surrogate tensor, 1024 waves (32, 250, 2048) 62.4 / 60.3 and 61.4 / 59.3, with a synapse 88.9 / 88.3 and 76.7 / 73.8, though
+// (16, 1000, 4096) 217 / 231 and 205 / 217.  Where blocks share sectors, three waves per unit: 768 (48, 300, 1000) 70.4 / 65.7 and
+// 68.0 / 63.7, (12, 500, 4090) 113.3 / 109.6 and 108.6 / 107.1; 832 (13, 500, 4090) 115 / 119 and 110 / 119; 1024
+// (16, 500, 4090) 129 / 144 and 123 / 142, (64, 1000, 1000) 241 / 265 and 238 / 265.  Without more tensors shared sectors leave
+// it at four: 1024 (64, 300, 1000) 69.6 / 68.5 and 80.7 / 80.0, 960 (60, 300, 1000) 67.1 / 65.0 and 84.8 / 80.1, though without a
+// synapse (16, 500, 4090) 105 / 113.
+inline int backward_lanes(int64_t batch, int64_t neurons, bool extra, bool whole)
 {
-    return batch * ((neurons + WAVE - 1) / WAVE) <= 4 * compute_units() ? WAVE : BWD_BLOCK;
+    return lanes_per_block(batch, neurons, extra && !whole ? 6 : 8) == WAVE ? WAVE : BWD_BLOCK;
 }
 
 inline unsigned common_alignment(std::initializer_list<const void *> ptrs)

@@ -217,7 +217,8 @@ int launch_bwd(float *grad_x, float *am_g, float *as_g, float *v0_g, float *i0_g
                const float *gir, const float *ckpt_v, const float *ckpt_i, const LayerConsts &p, float p0, float p1,
                bool uniform, int64_t B, int64_t T, int64_t M, hipStream_t s)
 {
-    const int lanes = backward_lanes(B, M);
+    const bool whole = uniform ? whole_lines(M, {grad_x, x}) : whole_lines(M, {grad_x, grad_spikes, x, surr, gvr, gir});
+    const int lanes = backward_lanes(B, M, gvr || surr, whole);
     const int64_t blocks_per_batch = (M + lanes - 1) / lanes;
     if (blocks_per_batch > 0x7fffffffLL / B) return hipErrorInvalidValue;
     const int64_t blocks = blocks_per_batch * B;
@@ -232,13 +233,13 @@ int launch_bwd(float *grad_x, float *am_g, float *as_g, float *v0_g, float *i0_g
             return hipErrorInvalidValue;
         } else {
             if (gvr) return hipErrorInvalidValue;
-            if (whole_lines(M, {grad_x, x})) EXODUS_LAUNCH(CAPK, true, false, true);
+            if (whole) EXODUS_LAUNCH(CAPK, true, false, true);
             else EXODUS_LAUNCH(CAPK, false, false, true);
         }
     } else if (gvr) {
         // gradients on the state records: one general instance per surrogate kind
         EXODUS_LAUNCH(0, false, true, false);
-    } else if (whole_lines(M, {grad_x, grad_spikes, x, surr})) {
+    } else if (whole) {
         EXODUS_LAUNCH(CAPK, true, false, false);
     } else {
         EXODUS_LAUNCH(CAPK, false, false, false);

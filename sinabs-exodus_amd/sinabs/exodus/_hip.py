@@ -452,7 +452,8 @@ def layerLifForward(input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, mem
 stamps = _native.stamps
 
 
-_SHAPES = ("forward", "forward records", "leaky forward", "leaky backward", "leaky backward alpha", "backward")
+_SHAPES = ("forward", "forward records", "leaky forward", "leaky backward", "leaky backward alpha", "backward",
+           "backward more")
 
 
 def launchShape(kernel: str, batch: int, neurons: int) -> tuple:
