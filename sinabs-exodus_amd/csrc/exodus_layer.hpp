@@ -280,8 +280,9 @@ inline int compute_units()
 // of one neuron per lane: `even` is the share of lanes that have work while the units that got one block more than the others
 // finish it (and that lie inside the layer).  Memory-bound blocks advance at one pace, so the other units stand idle by then.
 // One / two, us, spiking and leaky forward, leaky backward: (64, 300, 12544), even 0.94 / 0.88, 375 / 394, 355 / 374 and
-// 550 / 566; (40, 250, 11008), 0.96 / 0.89, 176 / 176, 163 / 174 and 252 / 263; where both are even (64, 300, 8192) 227 / 219,
-// 211 / 204 and 322 / 314.  With shared sectors two stay ahead: (64, 300, 17000) 631 / 584.
+// 550 / 566; (40, 250, 11008), 0.96 / 0.84, 176 / 176 (13 waves per unit would be left: forced here), 163 / 174 and 252 / 263;
+// where both are even (64, 300, 8192) 227 / 219, 211 / 204 and 322 / 314.  With shared sectors two stay ahead:
+// (64, 300, 17000) 631 / 584.
 // `align` is the common alignment (bytes) of all (batch, time, neurons) pointers involved.
 inline int pick_neurons_per_lane(int64_t batch, int64_t neurons, unsigned align, int widest, int waves_per_cu, bool whole)
 {

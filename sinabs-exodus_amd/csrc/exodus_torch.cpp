@@ -5,7 +5,7 @@
 // Why it exists: a training step of a small layer is host time, and the autograd engine runs the backward pass on a thread
 // of its own, where the 55 us of Python and ctypes that a backward pass was took up to 165 (caches and a core of its own).
 // Python and ctypes / these, us per step through the layer, forward and backward: IAF (8, 100, 256) 238 / 149, LIF
-// (32, 100, 512) with a trained time constant 271 / 173, a streamed chunk (1, 10, 1024) without gradients 46 / 27.
+// (32, 100, 512) with a trained time constant 271 / 173, a streamed chunk (1, 10, 1024) without gradients 47 / 24.
 #include <ATen/Functions.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
