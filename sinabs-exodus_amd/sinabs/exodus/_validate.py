@@ -110,7 +110,7 @@ def _begin(alphas, threshold, min_v_mem):
         return _DONE
     if len(alphas) <= 2 and _one_kernel_checks(checked):
         first = checked[0]
-        host = torch.zeros(2, dtype=torch.int32, pin_memory=True)
+        host = torch.zeros(2, dtype=torch.int32, device="cpu", pin_memory=True)
         _hip.checkParameters(host, alphas[0] if alphas else None, alphas[1] if len(alphas) > 1 else None,
                              threshold if min_v_mem is not None else None, min_v_mem)
         messages = (_ALPHA_MSG, _THRESHOLD_MSG)
@@ -129,7 +129,7 @@ def _begin(alphas, threshold, min_v_mem):
     if _MODE == "sync" or not stacked.is_cuda:
         _raise_if_flagged(stacked.tolist(), messages)
         return _DONE
-    host = torch.empty(stacked.shape, dtype=stacked.dtype, pin_memory=True)
+    host = torch.empty(stacked.shape, dtype=stacked.dtype, device="cpu", pin_memory=True)
     host.copy_(stacked, non_blocking=True)
     event = torch.cuda.Event()
     event.record(torch.cuda.current_stream(stacked.device))

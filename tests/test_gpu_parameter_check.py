@@ -51,3 +51,37 @@ def test_the_call_that_carries_the_value_raises():
             IntegrateAndFire.apply(x, bad, one * 0, one, None, None, ref.Heaviside())
         with pytest.raises(ValueError, match="greater than"):
             IntegrateAndFire.apply(x, one * 0.9, one * 0, one, None, one, ref.Heaviside())
+
+
+@pytest.mark.parametrize("mode", ["sync", "deferred"])
+@pytest.mark.parametrize("one_kernel", [True, False])
+def test_flags_are_host_memory_whatever_the_default_device(mode, one_kernel):
+    from sinabs.exodus import _validate as val
+    n = 40
+    low = torch.zeros(n if one_kernel else 1, device="cuda")           # broadcast: checked by torch's operations
+    good, bad, one = (torch.full((n,), v, device="cuda") for v in (0.5, 1.5, 1.0))
+    val.set_mode(mode)
+    try:
+        with torch.device("cuda"):
+            val.check_parameters([good], one, low)
+            val.flush()
+            with pytest.raises(ValueError, match="between 0 and 1"):
+                val.check_parameters([bad], one, low)
+                val.flush()
+    finally:
+        val.set_mode("sync")
+
+
+@pytest.mark.parametrize("kind", ["LIF", "IAF"])
+def test_layers_under_a_default_device(kind):
+    import sinabs.exodus.layers as el
+    x = torch.rand(2, 10, 30).cuda()
+    layer = getattr(el, kind)(**dict(tau_mem=20.0) if kind == "LIF" else {}).cuda()
+    want = layer(x)
+    with torch.device("cuda"):
+        layer = getattr(el, kind)(**dict(tau_mem=20.0) if kind == "LIF" else {})
+        assert torch.equal(layer(x), want)
+        with torch.no_grad():
+            layer.spike_threshold.fill_(1.0)
+            layer.reset_states()
+            assert torch.equal(layer(x), want)
