@@ -103,8 +103,10 @@ const Tensor &dev(const Tensor &x, const char *name, const Tensor *like = nullpt
 {
     if (!x.is_cuda())
         refuse(std::string(name) + " must be a tensor on a HIP device (got " + x.device().str() + "); there is no CPU path");
-    if (x.scalar_type() != at::kFloat)
-        refuse(std::string(name) + " must be float32 (got " + c10::toString(x.scalar_type()) + ")");
+    if (x.scalar_type() != at::kFloat) {
+        py::gil_scoped_acquire locked;
+        refuse(std::string(name) + " must be float32 (got " + std::string(py::str(py::cast(x).attr("dtype"))) + ")");
+    }
     if (!x.is_contiguous()) refuse(std::string(name) + " must be contiguous");
     if (like && x.device() != like->device()) refuse(std::string(name) + " and the first tensor must be on the same device");
     return x;

@@ -138,7 +138,7 @@ def test_build_failure_names_compiler_and_source(monkeypatch, tmp_path):
 def test_wrong_types_shapes_and_strides(name):
     x, r, two = torch.rand(1, 4, 6).cuda(), torch.rand(6).cuda() * 0.5 + 0.3, torch.rand(6, 4).cuda()
     calls(x, r, two)[name]()
-    with pytest.raises(RuntimeError, match="float32"):
+    with pytest.raises(RuntimeError, match=r"must be float32 \(got torch.float64\)"):
         calls(x.double(), r.double(), two.double())[name]()
     with pytest.raises(RuntimeError, match="contiguous"):
         calls(x.transpose(1, 2), r.repeat_interleave(2)[::2], two.t())[name]()
