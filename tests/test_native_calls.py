@@ -180,7 +180,11 @@ def test_other_threads_run_while_an_allocation_waits():
     torch.cuda.synchronize()
     cycles = int(10_000_000 * 500 / began.elapsed_time(ended))
     torch.cuda.empty_cache()
-    torch.empty(1 << 30, dtype=torch.uint8, device="cuda")                 # cached, free
+    # memory that can be given back: a segment of its own, not a piece of one that something else still uses
+    held, before = [], torch.cuda.memory_reserved()
+    while torch.cuda.memory_reserved() == before:
+        held.append(torch.empty(1 << 30, dtype=torch.uint8, device="cuda"))
+    held.pop()
     gaps, stop = [], threading.Event()
 
     def tick():
