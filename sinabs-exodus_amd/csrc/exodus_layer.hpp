@@ -377,6 +377,33 @@ inline bool whole_lines(int64_t neurons, std::initializer_list<const void *> ptr
     return (neurons % EXODUS_WHOLE_NEURONS) == 0 && (bits & (4u * EXODUS_WHOLE_NEURONS - 1u)) == 0;
 }
 
+// Blocks that are neighbours in a step, on one XCD.  The machine deals the blocks of a grid out to its eight XCDs one by one, each
+// with an L2 of its own: the line that two neighbouring blocks share is then fetched twice and written in two parts.  Where steps
+// do not fill whole lines of 128 bytes, runs of NEIGHBOURS blocks go to one XCD instead.  Before / after, us, forward and backward,
+// other tensors in every call, spiking and leaky: (64, 300, 17000) 574 + 904 / 562 + 852 and 570 + 827 / 552 + 801, (64, 300, 4999)
+// 198 + 280 / 182 + 266 and 191 + 264 / 174 + 245, (32, 400, 65533) 1616 + 2175 / 1491 + 2103 and 1489 + 2165 / 1409 + 2015,
+// (8, 500, 4090) 34.4 + 67.7 / 32.5 + 65.2 and 34.3 + 53.0 / 29.0 + 51.7, (24, 250, 1323) 22.3 + 39.8 / 20.7 + 37.3 and
+// 20.4 + 28.9 / 18.0 + 27.8; half lines shared, (64, 300, 4976) 165 + 258 / 163 + 254 and 160 + 237 / 157 + 232.  Runs of 8 and 16
+// are level or up to 2 % behind, of 64 up to 5 %.  Whole lines stay as they are dealt: nothing is shared, and the XCDs then walk
+// addresses further apart, (32, 300, 131072) 1879 + 2801 / 2023 + 2806, (64, 300, 12544) 370 + 558 / 369 + 559.
+constexpr int NEIGHBOURS = 32, XCDS = 8;
+inline unsigned neighbours_per_xcd(int64_t blocks, int64_t neurons, std::initializer_list<const void *> ptrs)
+{
+    uintptr_t bits = static_cast<uintptr_t>(neurons) * 4u;
+    for (const void *q : ptrs) bits |= reinterpret_cast<uintptr_t>(q);
+    if (bits % 128u == 0) return 1;
+    const int64_t share = blocks / XCDS;                        // a small grid is one run for each XCD
+    return share >= 2 * NEIGHBOURS ? NEIGHBOURS : (share > 1 ? static_cast<unsigned>(share) : 1u);
+}
+
+// The block of the layer that block blockIdx.x works on: XCDS runs of `run` blocks trade places so that each lies on one XCD; what
+// is left at the end of the grid stays where it is (a permutation of the grid's blocks, the identity for run == 1).
+__device__ __forceinline__ unsigned layer_block(unsigned run)
+{
+    const unsigned many = XCDS * run, start = blockIdx.x / many * many, at = blockIdx.x - start;
+    return gridDim.x - start < many ? blockIdx.x : start + at % XCDS * run + at / XCDS;
+}
+
 inline bool bad3(int64_t b, int64_t t, int64_t m)
 {
     if (b < 0 || t < 0 || m < 0) return true;

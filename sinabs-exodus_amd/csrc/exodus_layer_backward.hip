@@ -38,11 +38,12 @@ layer_lif_backward(
     const float *__restrict__ grad_v_last, const float *__restrict__ grad_i_last, const float *__restrict__ x,
     const float *__restrict__ surr, const float *__restrict__ grad_v_rec, const float *__restrict__ grad_i_rec,
     const float *__restrict__ ckpt_v, const float *__restrict__ ckpt_i, const LayerConsts p, const float p0,
-    const float p1, const float inv_p0, const int64_t blocks_per_batch, const int64_t T, const int64_t M)
+    const float p1, const float inv_p0, const int64_t blocks_per_batch, const int64_t T, const int64_t M, const unsigned run)
 {
     typedef BufIO<1, NT> IO;
-    const int64_t b = blockIdx.x / blocks_per_batch;
-    const int64_t m0 = static_cast<int64_t>(blockIdx.x - b * blocks_per_batch) * blockDim.x;
+    const unsigned block_of_layer = layer_block(run);
+    const int64_t b = block_of_layer / blocks_per_batch;
+    const int64_t m0 = static_cast<int64_t>(block_of_layer - b * blocks_per_batch) * blockDim.x;
     const unsigned lane_off = threadIdx.x;
     // lanes past the end of the layer walk the same loops and meet every barrier, but all memory
     // accesses and all arithmetic sit behind `active`
@@ -222,10 +223,12 @@ int launch_bwd(float *grad_x, float *am_g, float *as_g, float *v0_g, float *i0_g
     const int64_t blocks_per_batch = (M + lanes - 1) / lanes;
     if (blocks_per_batch > 0x7fffffffLL / B) return hipErrorInvalidValue;
     const int64_t blocks = blocks_per_batch * B;
+    const unsigned run =
+        uniform ? neighbours_per_xcd(blocks, M, {grad_x, x}) : neighbours_per_xcd(blocks, M, {grad_x, grad_spikes, x, surr, gvr, gir});
 #define EXODUS_LAUNCH(CK, NT, EX, G1)                                                                              \
     hipLaunchKernelGGL((layer_lif_backward<SYN, KIND, CK, NT, EX, G1>), dim3(static_cast<unsigned>(blocks)),      \
                        dim3(lanes), 0, s, grad_x, am_g, as_g, v0_g, i0_g, grad_spikes, gvl, gil, x, surr, gvr, \
-                       gir, ckpt_v, ckpt_i, p, p0, p1, p0 != 0.f ? 1.f / p0 : 0.f, blocks_per_batch, T, M)
+                       gir, ckpt_v, ckpt_i, p, p0, p1, p0 != 0.f ? 1.f / p0 : 0.f, blocks_per_batch, T, M, run)
     if (uniform) {
         // one value as the gradient of every spike: instances exist for the in-kernel surrogates, without
         // gradients on the state records
