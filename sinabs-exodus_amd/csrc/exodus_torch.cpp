@@ -12,6 +12,7 @@
 #include <pybind11/pybind11.h>
 #include <pybind11/stl.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 
@@ -54,8 +55,10 @@ struct Library {
 Library lib;
 int64_t interval = 0;                                          // steps between checkpoints
 PyObject *raise_status = nullptr;                              // (status, what): raises for a status other than 0
+PyObject *place_of = nullptr;                                  // (like): what allocates large results (see `large`), or None
 
-void bind(const py::dict &addresses, const py::object &on_status)
+// on_place: what `place_of` is, for the layers' nodes; None keeps what an earlier call gave
+void bind(const py::dict &addresses, const py::object &on_status, const py::object &on_place)
 {
     Library given;
 #define EXODUS_BIND(name) \
@@ -70,6 +73,9 @@ void bind(const py::dict &addresses, const py::object &on_status)
     interval = lib.exodus_layer_checkpoint_interval();
     Py_XDECREF(raise_status);
     raise_status = py::object(on_status).release().ptr();
+    if (on_place.is_none()) return;
+    Py_XDECREF(place_of);
+    place_of = py::object(on_place).release().ptr();
 }
 
 // call a function of the library on the tensor's device and stream
@@ -174,7 +180,7 @@ Tensor fresh(c10::IntArrayRef shape, const Tensor &like, at::ScalarType type = a
 }
 
 // the (batch, time, neurons) and (rows, time) results: `place`, if given, allocates them (shape, like)
-Tensor large(c10::IntArrayRef shape, const Tensor &like, const py::object &place)
+Tensor large(c10::IntArrayRef shape, const Tensor &like, const py::handle place)
 {
     if (place.is_none()) return fresh(shape, like);
     py::gil_scoped_acquire locked;
@@ -215,7 +221,7 @@ Eight layer_lif_forward(const Tensor &input, const Tensor &v_init, const Maybe &
                             const Maybe &alpha_syn, const Tensor &subtract, const Tensor &theta, const Maybe &theta_low,
                             bool apply_low, int64_t max_spikes, bool decay_early, bool norm_input, bool want_checkpoints,
                             bool want_records, bool want_pre_reset, bool want_sum, const Maybe &out_spikes,
-                            const std::optional<Shape> &state_shape, const py::object &place)
+                            const std::optional<Shape> &state_shape, const py::handle place)
 {
     if (want_records && want_pre_reset) refuse("wantRecords and wantPreReset exclude each other");
     three(input, "input");
@@ -257,7 +263,7 @@ Five layer_lif_backward(const Tensor &grad_spikes, const Maybe &grad_v_last, con
                              const Maybe &theta_low, bool apply_low, int64_t max_spikes, bool decay_early, bool norm_input,
                              int kind, double p0, double p1, const Maybe &grad_input_given, const Maybe &surr_given,
                              Maybe grad_v_rec, Maybe grad_i_rec, bool want_alpha_mem, bool want_alpha_syn, bool want_v_init,
-                             bool want_i_init, bool uniform, const py::object &place)
+                             bool want_i_init, bool uniform, const py::handle place)
 {
     three(input, "input");
     const int64_t b = input.size(0), t = input.size(1), m = input.size(2), n = b * m;
@@ -342,7 +348,7 @@ Five layer_lif_backward(const Tensor &grad_spikes, const Maybe &grad_v_last, con
 
 // -> (out, v_last, total)
 Three layer_leaky_forward(const Tensor &input, const Tensor &v_init, const Tensor &alpha, bool decay_early, bool norm_input,
-                              const std::optional<Shape> &state_shape, bool want_sum, const py::object &place)
+                              const std::optional<Shape> &state_shape, bool want_sum, const py::handle place)
 {
     three(input, "input");
     const int64_t b = input.size(0), t = input.size(1), m = input.size(2), n = b * m;
@@ -363,7 +369,7 @@ Three layer_leaky_forward(const Tensor &input, const Tensor &v_init, const Tenso
 // -> (grad_input, alpha, v_init)
 Three layer_leaky_backward(const Tensor &grad_out, const Maybe &grad_v_last, const Maybe &forward_out, const Maybe &input,
                                const Maybe &v_init, const Tensor &alpha, bool decay_early, bool norm_input, bool want_alpha,
-                               const std::optional<Shape> &uniform_shape, const py::object &place)
+                               const std::optional<Shape> &uniform_shape, const py::handle place)
 {
     const bool uniform = uniform_shape.has_value();
     Shape shape;
@@ -513,7 +519,7 @@ Tensor per_row(const Tensor &alpha, int64_t n, int64_t t)
 Three lif_backward_fused(const Tensor &grad_spikes, const Maybe &grad_vmem, const Tensor &v_mem, const Maybe &v_init,
                              const Tensor &alpha, const Tensor &subtract, const Tensor &theta, const Maybe &theta_low,
                              bool apply_low, int64_t max_spikes, int kind, double p0, double p1, const Maybe &surr_given,
-                             bool want_alpha, const Maybe &grad_input_given, const py::object &place)
+                             bool want_alpha, const Maybe &grad_input_given, const py::handle place)
 {
     two(v_mem, "vmem");
     const int64_t n = v_mem.size(0), t = v_mem.size(1);
@@ -535,7 +541,7 @@ Three lif_backward_fused(const Tensor &grad_spikes, const Maybe &grad_vmem, cons
     return {grad_input, a_g, v0_g};
 }
 
-Tensor leaky_forward(const Tensor &input, const Tensor &v_init, const Tensor &alpha, const Maybe &given, const py::object &place)
+Tensor leaky_forward(const Tensor &input, const Tensor &v_init, const Tensor &alpha, const Maybe &given, const py::handle place)
 {
     two(input, "input");
     const int64_t n = input.size(0), t = input.size(1);
@@ -550,7 +556,7 @@ Tensor leaky_forward(const Tensor &input, const Tensor &v_init, const Tensor &al
 
 // -> (grad_input, alpha, v_init)
 Three leaky_backward_fused(const Tensor &grad_out, const Tensor &alpha, const Maybe &forward_out, const Maybe &v_init,
-                               bool want_alpha, const Maybe &grad_input_given, const py::object &place)
+                               bool want_alpha, const Maybe &grad_input_given, const py::handle place)
 {
     two(grad_out, "outputGrad");
     const int64_t n = grad_out.size(0), t = grad_out.size(1);
@@ -567,13 +573,275 @@ Three leaky_backward_fused(const Tensor &grad_out, const Tensor &alpha, const Ma
     return {grad_input, a_g, v0_g};
 }
 
+// ---------------------------------------------------------------------------------------------
+// layers as nodes of the autograd graph
+// ---------------------------------------------------------------------------------------------
+// What layer_function.py's two Functions do, for the calls that need no Python on the way back (a surrogate that the kernels
+// know): the same tensors saved in the same order, the same gradients.  The engine runs a backward pass on a thread of its own,
+// where Python means the interpreter lock, cold caches and thirteen unpacked tensors; and the input's shape is taken and given
+// back here instead of by reshapes that are nodes of their own.  us per training step in Python and here: IAF (8, 100, 256)
+// 131 / 86, LIF (32, 100, 512) with a trained time constant 155 / 118, LIF with synapses (4, 2000, 512), both constants trained, 189 / 152.
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// the tensor in another shape, for the calls above and as a result of a node: no view in autograd's books
+Tensor shaped(const Tensor &x, c10::IntArrayRef shape) { return x.sizes() == shape ? x : at::_unsafe_view(x, shape); }
+Maybe shaped(const Maybe &x, c10::IntArrayRef shape) { return has(x) ? Maybe(shaped(*x, shape)) : Maybe(); }
+
+Shape three_of(const Tensor &x)
+{
+    if (x.dim() < 2) refuse("the input must have the dimensions batch, time, neurons");
+    return {x.size(0), x.size(1), elements(Shape(x.sizes().begin() + 2, x.sizes().end()))};
+}
+
+// what allocates the large results of a backward pass, as of now
+py::handle place_now(const Tensor &like)
+{
+    py::gil_scoped_acquire locked;
+    if (place_of == nullptr) return Py_None;
+    const py::object found = py::reinterpret_borrow<py::object>(place_of)(like);
+    return found;                                              // a function of a module, or None: both outlive this reference
+}
+
+// One value that `grad` repeats everywhere (the gradient of a sum of the output), as a tensor of one element.
+Tensor one_value(const Tensor &grad)
+{
+    if (!grad.defined() || grad.numel() < 2 || grad.scalar_type() != at::kFloat) return Tensor();
+    for (const int64_t stride : grad.strides())
+        if (stride != 0) return Tensor();
+    return grad.as_strided({1}, {1});
+}
+
+// The gradient of a layer's output as the kernels take it, from what arrived at the output and at its total: dense, or one value
+// for every element (then `uniform`) where `allowed`.
+Tensor joined_gradient(const Tensor &grad, const Tensor &grad_total, const Shape &shape, const Tensor &like, bool allowed, bool &uniform)
+{
+    const auto options = like.options().dtype(at::kFloat);
+    uniform = false;
+    if (allowed && elements(shape) > 1) {
+        Tensor one = grad.defined() ? one_value(grad) : (grad_total.defined() ? Tensor() : at::zeros({1}, options));
+        if (grad_total.defined() && (one.defined() || !grad.defined())) {
+            const Tensor total = grad_total.to(at::kFloat).reshape({1});
+            one = one.defined() ? at::add(one, total) : total;
+        }
+        if (one.defined()) {
+            uniform = true;
+            return one;
+        }
+    }
+    Tensor dense = grad.defined() ? grad.reshape(shape) : at::zeros(shape, options);
+    if (grad_total.defined()) dense = at::add(dense, grad_total.to(dense.scalar_type()));
+    return dense.contiguous();
+}
+
+Maybe dense(const Tensor &grad) { return grad.defined() ? Maybe(grad.contiguous()) : Maybe(); }
+Maybe dense(const Tensor &grad, const Shape &shape) { return grad.defined() ? Maybe(grad.reshape(shape).contiguous()) : Maybe(); }
+Maybe maybe(const Tensor &x) { return x.defined() ? Maybe(x) : Maybe(); }
+
+// The place among a node's edges of each of its arguments, -1 for one that is absent (absent tensors get no edge).
+struct Edges {
+    int next = 0;
+    int add(bool given) { return given ? next++ : -1; }
+};
+
+// What a node keeps besides tensors is one list of integers: compiled autograd looks into it.
+int64_t bits(double x)
+{
+    int64_t n;
+    std::memcpy(&n, &x, sizeof n);
+    return n;
+}
+double from_bits(int64_t n)
+{
+    double x;
+    std::memcpy(&x, &n, sizeof x);
+    return x;
+}
+
+struct LifCall {
+    bool syn, apply_low, decay_early, norm_input, records, need_grad;
+    int64_t max_spikes, kind;
+    double p0, p1;
+    const Shape &states;
+    const Maybe &kept_mem, &kept_syn;                          // the time constants as the forward pass saw them
+    py::handle place;
+};
+
+struct LifLayer : torch::autograd::Function<LifLayer> {
+    static variable_list forward(AutogradContext *ctx, const Tensor &input, const Tensor &alpha_mem, const Maybe &alpha_syn,
+                                 const Tensor &v_init, const Maybe &i_init, const Maybe &tau_mem, const Maybe &tau_syn,
+                                 const Tensor &theta, const Tensor &subtract, const Maybe &theta_low,
+                                 const LifCall &c)
+    {
+        const Shape shape = three_of(input);
+        const int64_t n = shape[0] * shape[2];
+        Edges edges;
+        edges.add(true);                                       // the input
+        const int e_am = edges.add(true), e_as = edges.add(has(alpha_syn)), e_v0 = edges.add(true), e_i0 = edges.add(has(i_init));
+        const int e_tm = edges.add(has(tau_mem)), e_ts = edges.add(has(tau_syn));
+        const auto [spikes, v_last, i_last, ckpt_v, ckpt_i, v_rec, i_rec, total] = layer_lif_forward(
+            shaped(input, shape), shaped(v_init, {n}), shaped(i_init, {n}), alpha_mem, alpha_syn, subtract, theta, theta_low,
+            c.apply_low, c.max_spikes, c.decay_early, c.norm_input, c.need_grad, c.records, false, true, Maybe(), c.states, c.place);
+        ctx->set_materialize_grads(false);
+        if (c.need_grad)
+            ctx->save_for_backward({input, ckpt_v, ckpt_i, v_init, i_init.value_or(Tensor()), alpha_mem,
+                                    alpha_syn.value_or(Tensor()), subtract, theta, theta_low.value_or(Tensor()),
+                                    c.kept_mem.value_or(Tensor()), c.kept_syn.value_or(Tensor())});
+        ctx->saved_data["call"] = Shape{c.syn, c.apply_low, c.decay_early, c.norm_input, c.records, c.max_spikes, c.kind, bits(c.p0),
+                                        bits(c.p1), e_am, e_as, e_v0, e_i0, e_tm, e_ts};
+        variable_list outputs{shaped(spikes, input.sizes()), v_last, total};
+        if (c.syn) outputs.push_back(i_last);
+        if (c.records) outputs.push_back(shaped(v_rec, input.sizes()));
+        if (c.records && c.syn) outputs.push_back(shaped(i_rec, input.sizes()));
+        return outputs;
+    }
+
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
+    {
+        const at::AutoGradMode no_graph(false);
+        const Shape call = ctx->saved_data.at("call").toIntVector();
+        const bool syn = call[0], apply_low = call[1], decay_early = call[2], norm_input = call[3], records = call[4];
+        const int e_am = call[9], e_as = call[10], e_v0 = call[11], e_i0 = call[12], e_tm = call[13], e_ts = call[14];
+        const variable_list saved = ctx->get_saved_variables();
+        variable_list result(11);
+        bool any = false;
+        for (const Tensor &g : grads) any = any || g.defined();
+        if (!any) return result;
+        size_t at = 3;
+        const Tensor &grad_spikes = grads[0], &grad_v_last = grads[1], &grad_total = grads[2];
+        const Tensor grad_i_last = syn ? grads[at++] : Tensor(), grad_v_rec = records ? grads[at++] : Tensor();
+        const Tensor grad_i_rec = records && syn ? grads[at++] : Tensor();
+        const Tensor &input = saved[0], &v_init = saved[3], &i_init = saved[4];
+        const Shape shape = three_of(input);
+        const int64_t n = shape[0] * shape[2];
+        const auto needs = [&](int edge) { return edge >= 0 && ctx->needs_input_grad(edge); };
+        const bool tau_mem = needs(e_tm), tau_syn = needs(e_ts);
+        bool uniform;
+        const Tensor gs = joined_gradient(grad_spikes, grad_total, shape, input, !grad_v_rec.defined() && !grad_i_rec.defined(), uniform);
+        const auto [g_x, g_am, g_as, g_v0, g_i0] = layer_lif_backward(
+            gs, dense(grad_v_last), dense(grad_i_last), shaped(input, shape), maybe(saved[1]), maybe(saved[2]), shaped(v_init, {n}),
+            shaped(maybe(i_init), {n}), saved[5], maybe(saved[6]), saved[7], saved[8], maybe(saved[9]), apply_low, call[5],
+            decay_early, norm_input, static_cast<int>(call[6]), from_bits(call[7]), from_bits(call[8]), Maybe(), Maybe(),
+            dense(grad_v_rec, shape), dense(grad_i_rec, shape), needs(e_am) || tau_mem, needs(e_as) || tau_syn, needs(e_v0),
+            needs(e_i0), uniform, place_now(input));
+        if (ctx->needs_input_grad(0)) result[0] = shaped(g_x, input.sizes());
+        if (needs(e_am)) result[1] = g_am;
+        if (needs(e_as)) result[2] = g_as;
+        if (needs(e_v0)) result[3] = shaped(g_v0, v_init.sizes());
+        if (needs(e_i0)) result[4] = shaped(g_i0, i_init.sizes());
+        if (tau_mem) result[5] = decay_grad(g_am, saved[10], shape[0], shape[2]);
+        if (tau_syn) result[6] = decay_grad(g_as, saved[11], shape[0], shape[2]);
+        return result;
+    }
+};
+
+bool graph_wanted(std::initializer_list<const Tensor *> given, std::initializer_list<const Maybe *> optional)
+{
+    if (!at::GradMode::is_enabled()) return false;
+    for (const Tensor *x : given)
+        if (x->requires_grad()) return true;
+    for (const Maybe *x : optional)
+        if (has(*x) && (*x)->requires_grad()) return true;
+    return false;
+}
+
+// -> (spikes, v_last, total, i_last, v_rec, i_rec) in the input's shape and the states' shape, with their place in the graph.
+// tau_mem / tau_syn: the parameters that alpha_mem / alpha_syn were worked out from (decay_expand, which also made kept_mem /
+// kept_syn) and whose gradients are wanted in the place of theirs.
+Eight layer_lif(const Tensor &input, const Tensor &alpha_mem, const Maybe &alpha_syn, const Tensor &v_init, const Maybe &i_init,
+                const Maybe &tau_mem, const Maybe &tau_syn, const Maybe &kept_mem, const Maybe &kept_syn, const Tensor &theta,
+                const Tensor &subtract, const Maybe &theta_low, int kind, double p0, double p1, int64_t max_spikes, bool decay_early,
+                bool norm_input, bool records, const Shape &states, const py::handle place)
+{
+    const bool syn = has(alpha_syn);
+    const bool need_grad = graph_wanted({&input, &alpha_mem, &v_init, &theta, &subtract}, {&alpha_syn, &i_init, &tau_mem, &tau_syn,
+                                                                                           &theta_low});
+    const LifCall call{syn, has(theta_low), decay_early, norm_input, records, need_grad, max_spikes, kind, p0, p1, states,
+                       kept_mem, kept_syn, place};
+    const variable_list out = LifLayer::apply(input, alpha_mem, alpha_syn, v_init, i_init, tau_mem, tau_syn, theta, subtract,
+                                              theta_low, call);
+    const auto nth = [&](bool given, size_t k) { return given ? out[k] : Tensor(); };
+    const size_t rec = syn ? 4 : 3;
+    return {out[0], out[1], out[2], nth(syn, 3), nth(records, rec), nth(records && syn, rec + 1), Tensor(), Tensor()};
+}
+
+struct LeakyCall {
+    bool decay_early, norm_input, need_grad, need_alpha;
+    const Shape &states;
+    const Maybe &kept;
+    py::handle place;
+};
+
+struct LeakyLayer : torch::autograd::Function<LeakyLayer> {
+    static variable_list forward(AutogradContext *ctx, const Tensor &input, const Tensor &alpha, const Tensor &v_init, const Maybe &tau,
+                                 const LeakyCall &c)
+    {
+        const Shape shape = three_of(input);
+        auto [flat, v_last, total] = layer_leaky_forward(shaped(input, shape), shaped(v_init, {shape[0] * shape[2]}), alpha,
+                                                         c.decay_early, c.norm_input, c.states, true, c.place);
+        const Tensor result = shaped(flat, input.sizes());
+        ctx->set_materialize_grads(false);
+        if (c.need_grad && c.need_alpha)
+            ctx->save_for_backward({alpha, v_init, result, c.decay_early || c.norm_input ? input : Tensor(),
+                                    c.kept.value_or(Tensor())});
+        else if (c.need_grad)
+            ctx->save_for_backward({alpha});
+        Shape call{c.decay_early, c.norm_input, c.need_alpha, has(tau), input.dim()};
+        call.insert(call.end(), input.sizes().begin(), input.sizes().end());
+        call.insert(call.end(), v_init.sizes().begin(), v_init.sizes().end());
+        ctx->saved_data["call"] = call;
+        return {result, v_last, total};
+    }
+
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads)
+    {
+        const at::AutoGradMode no_graph(false);
+        const Shape call = ctx->saved_data.at("call").toIntVector();
+        const bool decay_early = call[0], norm_input = call[1], need_alpha = call[2], tau = call[3];
+        const c10::IntArrayRef sizes = c10::IntArrayRef(call).slice(5), full = sizes.slice(0, call[4]), states = sizes.slice(call[4]);
+        const Shape shape{full[0], full[1], elements(Shape(full.begin() + 2, full.end()))};
+        variable_list saved = ctx->get_saved_variables();
+        saved.resize(5);
+        variable_list result(5);
+        if (!grads[0].defined() && !grads[1].defined() && !grads[2].defined()) return result;
+        const Tensor &alpha = saved[0], &out = saved[2], &input = saved[3];
+        const int64_t n = shape[0] * shape[2];
+        bool uniform;
+        const Tensor g = joined_gradient(grads[0], grads[2], shape, alpha, true, uniform);
+        // what of the results is allocated elsewhere depends on their size: the same kind of tensor as the gradient, expanded
+        const auto [g_x, g_a, g_v0] = layer_leaky_backward(
+            g, dense(grads[1]), need_alpha ? maybe(shaped(out, shape)) : Maybe(),
+            input.defined() ? maybe(shaped(input, shape)) : Maybe(), need_alpha ? maybe(shaped(saved[1], {n})) : Maybe(), alpha,
+            decay_early, norm_input, need_alpha, uniform ? std::optional<Shape>(shape) : std::nullopt,
+            place_now(uniform ? g.expand(shape) : g));
+        if (ctx->needs_input_grad(0)) result[0] = shaped(g_x, full);
+        if (tau) {
+            if (ctx->needs_input_grad(3)) result[3] = decay_grad(g_a, saved[4], shape[0], shape[2]);
+        } else if (ctx->needs_input_grad(1)) {
+            result[1] = g_a;
+        }
+        if (ctx->needs_input_grad(2)) result[2] = shaped(g_v0, states);
+        return result;
+    }
+};
+
+// -> (out in the input's shape, v_last, total); tau and kept as above
+Three layer_leaky(const Tensor &input, const Tensor &alpha, const Tensor &v_init, const Maybe &tau, const Maybe &kept,
+                  bool decay_early, bool norm_input, const Shape &states, const py::handle place)
+{
+    const bool need_alpha = has(tau) ? tau->requires_grad() : alpha.requires_grad();
+    const LeakyCall call{decay_early, norm_input, graph_wanted({&input, &alpha, &v_init}, {&tau}), need_alpha, states, kept, place};
+    const variable_list out = LeakyLayer::apply(input, alpha, v_init, tau, call);
+    return {out[0], out[1], out[2]};
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_exodus_torch, module)
 {
     module.attr("built_for") = EXODUS_BUILT_FOR;                // the loader compares it with what is running
     // torch's own exceptions reach the caller as what they are (out of memory as torch.OutOfMemoryError)
-    module.def("bind", torch::wrap_pybind_function(bind));
+    module.def("bind", torch::wrap_pybind_function(bind), py::arg("addresses"), py::arg("on_status"), py::arg("on_place") = py::none());
     // The calls run without the interpreter lock from their checks to their launch: an allocation may have to free memory and
     // wait for the device, and other Python threads go on meanwhile.  One release for all of it, as taking the lock back is what
     // a busy interpreter makes a caller wait for.
@@ -581,6 +849,8 @@ PYBIND11_MODULE(_exodus_torch, module)
     module.def("layer_lif_backward", torch::wrap_pybind_function_no_gil(layer_lif_backward));
     module.def("layer_leaky_forward", torch::wrap_pybind_function_no_gil(layer_leaky_forward));
     module.def("layer_leaky_backward", torch::wrap_pybind_function_no_gil(layer_leaky_backward));
+    module.def("layer_lif", torch::wrap_pybind_function_no_gil(layer_lif));
+    module.def("layer_leaky", torch::wrap_pybind_function_no_gil(layer_leaky));
     module.def("stamps", torch::wrap_pybind_function(stamps));
     module.def("decay_expand", torch::wrap_pybind_function_no_gil(decay_expand));
     module.def("decay_grad", torch::wrap_pybind_function_no_gil(decay_grad));

@@ -130,11 +130,8 @@ def _native_module():
     except ImportError as err:
         raise ImportError(f"{os.path.join(_HERE, '_exodus_torch.so')} cannot be loaded ({err}). Build it with "
                           "`python build_hip.py` in the package root.") from err
-    native.bind({name: ctypes.cast(getattr(lib, name), _p).value for name in _SIGNATURES}, _check)
+    native.bind({name: ctypes.cast(getattr(lib, name), _p).value for name in _SIGNATURES}, _check, _place)
     return native
-
-
-_native = _native_module()
 
 
 def _rows(x: torch.Tensor, name: str, n: int) -> torch.Tensor:
@@ -189,6 +186,9 @@ def _place(like: torch.Tensor, shape: Optional[tuple] = None):
     if not isinstance(like, torch.Tensor):
         return None                            # refused by the call
     return hbm.empty if hbm.places(like.numel() if shape is None else math.prod(shape), like) else None
+
+
+_native = _native_module()
 
 
 def checkParameters(flags, alpha, alphaOther, theta, thetaLow) -> None:
@@ -445,6 +445,26 @@ def layerLifForward(input, vmemPostInitial, isynInitial, alphaMem, alphaSyn, mem
         thetaLow if applyThetaLow else None, bool(applyThetaLow),
         _cap(maxNumSpikes), bool(decayEarly), bool(normInput), bool(wantCheckpoints), bool(wantRecords), bool(wantPreReset),
         bool(wantSpikeSum), outSpikes, stateShape, _place(input))))
+
+
+def layerLif(input, alphaMem, alphaSyn, vmemPostInitial, isynInitial, tauMem, tauSyn, keptMem, keptSyn, theta, membrSubtract,
+             thetaLow, surrogateKind: int, surrP0: float, surrP1: float, maxNumSpikes: int, decayEarly: bool, normInput: bool,
+             records: bool, stateShape):
+    """The pass of ``layerLifForward`` as a node of the autograd graph, for the surrogates that the kernels evaluate:
+    (spikes, v_last, spike_sum, i_last | None, v_rec | None, i_rec | None).  ``input`` and the initial states may have any
+    contiguous shape (``input`` (batch, time, ...)); spikes and records come in that of ``input``.  ``tauMem`` / ``tauSyn`` are
+    the time constants to be trained in the place of ``alphaMem`` / ``alphaSyn``, which ``decayExpand`` worked out from them
+    together with ``keptMem`` / ``keptSyn``."""
+    return _native.layer_lif(input, alphaMem, alphaSyn, vmemPostInitial, isynInitial, tauMem, tauSyn, keptMem, keptSyn, theta,
+                             membrSubtract, thetaLow, surrogateKind, surrP0, surrP1, _cap(maxNumSpikes), bool(decayEarly),
+                             bool(normInput), bool(records), stateShape, _place(input))[:6]
+
+
+def layerLeaky(input, alpha, vmemInitial, tau, kept, decayEarly: bool, normInput: bool, stateShape):
+    """The pass of ``layerLeakyForward`` as a node of the autograd graph, (out, v_last, out_sum); shapes, ``tau`` and ``kept``
+    as for ``layerLif``."""
+    return _native.layer_leaky(input, alpha, vmemInitial, tau, kept, bool(decayEarly), bool(normInput), stateShape,
+                               _place(input))
 
 
 # stamps(kept, values): a tuple with one entry per value, the entries of ``kept`` (an earlier result, or None) where a value is

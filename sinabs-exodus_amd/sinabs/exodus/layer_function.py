@@ -15,10 +15,29 @@ potential before the reset, the backward calls the function on it and hands the 
 from typing import Callable, Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _hip
 from ._validate import check_parameters
 from .spike import classify_surrogate
+
+
+# the wrappers that the Functions below call; a program that puts its own in their place (to log or to check) sees the calls
+_WRAPPERS = tuple((name, getattr(_hip, name)) for name in (
+    "layerLifForward", "layerLifBackward", "layerLeakyForward", "layerLeakyBackward", "decayGrad"))
+_PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
+def native_graph(inp: torch.Tensor) -> bool:
+    """Whether a layer's call may put its node into the autograd graph in native code (``_hip.layerLif``, ``_hip.layerLeaky``).
+    The Functions below do for everything that wants to see a Python Function: functorch's transforms, forward-mode
+    differentiation and tracing (which refuse them, or look into them, as before), tensors of another class, and wrappers of
+    ``_hip`` that somebody has replaced."""
+    if type(inp) not in _PLAIN_TENSORS or torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0:
+        return False
+    own = _hip.__dict__
+    return (torch._C._get_tracing_state() is None and not torch.compiler.is_compiling()
+            and all([own[name] is wrapper for name, wrapper in _WRAPPERS]))
 
 
 def _one_value(grad: Optional[torch.Tensor]) -> Optional[torch.Tensor]:

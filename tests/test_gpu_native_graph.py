@@ -1,0 +1,329 @@
+"""The layers' nodes of the autograd graph in native code against the Python Functions: outputs, states, records and gradients to
+the bit, over the forms that a call and its loss can have; and what autograd promises around a node (graphs used twice, values
+modified in between, hooks on saved tensors, checkpointing, memory that is given back)."""
+import gc
+import weakref
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+FORMS = {
+    "iaf": dict(kind="IAF"),
+    "iaf squeezed": dict(kind="IAFSqueeze", squeeze=True, dims=(3, 5, 4)),
+    "lif": dict(kind="LIF", tau_mem=20.0),
+    "lif maps": dict(kind="LIF", tau_mem=20.0, dims=(3, 5, 4), min_v_mem=-0.5),
+    "lif one neuron": dict(kind="LIF", tau_mem=20.0, dims=()),
+    "lif tau per neuron": dict(kind="LIF", tau_mem="vector", dims=(2, 7)),
+    "lif alphas, records": dict(kind="LIF", tau_mem=20.0, train_alphas=True, record_states=True, dims=(3, 5)),
+    "lif syn": dict(kind="LIF", tau_mem=20.0, tau_syn=5.0, norm_input=False),
+    "lif syn, alphas per neuron, records": dict(kind="LIF", tau_mem="vector", tau_syn="vector", train_alphas=True,
+                                                record_states=True, decay_early=False, dims=(2, 7)),
+    "lif syn, fixed": dict(kind="LIF", tau_mem=20.0, tau_syn=5.0, fixed=True),
+    "expleak": dict(kind="ExpLeak", tau_mem=20.0, dims=(3, 5, 4)),
+    "expleak alphas": dict(kind="ExpLeak", tau_mem="vector", train_alphas=True, norm_input=True, dims=(13,)),
+    "expleak fixed": dict(kind="ExpLeakSqueeze", tau_mem=20.0, squeeze=True, fixed=True, record_states=True, dims=(3, 5)),
+}
+LOSSES = ("dense", "sum", "rate", "dense and rate", "states", "records", "none on the spikes", "chained")
+
+
+def build(form, seed=0):
+    import sinabs.exodus.layers as el
+    kw = dict(form)
+    kind, dims = kw.pop("kind"), kw.pop("dims", (13,))
+    squeeze, fixed = kw.pop("squeeze", False), kw.pop("fixed", False)
+    g = torch.Generator().manual_seed(seed)
+    for name in ("tau_mem", "tau_syn"):
+        if kw.get(name) == "vector":
+            kw[name] = 5.0 + 20.0 * torch.rand(dims, generator=g)
+    if squeeze:
+        kw["batch_size"] = 3
+    layer = getattr(el, kind)(**kw).cuda()
+    for p in layer.parameters():
+        if fixed:
+            p.requires_grad_(False)
+    x = (torch.randn(3, 37, *dims, generator=g) * 3 + 0.5).cuda()
+    return layer, (x.flatten(0, 1) if squeeze else x).requires_grad_(True)
+
+
+def step(layer, x, loss):
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rnd = lambda t: torch.randn(t.shape, generator=g, device="cuda")
+    x.grad = None
+    layer.zero_grad()
+    layer.reset_states()
+    out = layer(x)
+    if loss == "chained":
+        out = out + layer(x)
+    total = 0.0
+    if loss in ("dense", "dense and rate", "chained"):
+        total = total + (out * rnd(out)).sum()
+    if loss == "sum":
+        total = total + out.sum()
+    if loss in ("rate", "dense and rate"):
+        total = total + 3.0 * layer.firing_rate
+    if loss in ("states", "none on the spikes"):
+        total = total + sum((b * rnd(b)).sum() for b in layer.buffers())
+        if loss == "states":
+            total = total + (out * rnd(out)).sum()
+    if loss == "records":
+        total = total + sum((r * rnd(r)).sum() for r in layer.recordings.values())
+        total = total + (out * rnd(out)).sum()
+    total.backward()
+    return ([out, x.grad] + [b.detach() for b in layer.buffers()] + list(layer.recordings.values())
+            + [p.grad for p in layer.parameters()] + [torch.as_tensor(layer.firing_rate)])
+
+
+@pytest.fixture
+def python_functions(monkeypatch):
+    import sinabs.exodus.layers.neurons as nm
+
+    def use():
+        monkeypatch.setattr(nm, "native_graph", lambda x: False)
+    return use
+
+
+@pytest.mark.parametrize("loss", LOSSES)
+@pytest.mark.parametrize("form", FORMS)
+def test_as_the_python_functions(form, loss, python_functions):
+    if loss == "records" and not FORMS[form].get("record_states"):
+        pytest.skip("no records")
+    if loss == "chained" and FORMS[form].get("squeeze"):
+        pytest.skip("covered by the other forms")
+    layer, x = build(FORMS[form])
+    got = step(layer, x, loss)
+    assert FORMS[form].get("squeeze") or "LayerFunction" not in layer(x).grad_fn.name()    # (behind a reshape in the others)
+    python_functions()
+    layer, x = build(FORMS[form])
+    want = step(layer, x, loss)
+    assert len(got) == len(want)
+    for k, (p, q) in enumerate(zip(got, want)):
+        assert (p is None) == (q is None), k
+        if p is not None:
+            assert p.shape == q.shape and torch.equal(p, q), k
+
+
+def test_other_layouts_of_input_and_gradient(python_functions):
+    """Transposed inputs, expanded inputs, gradients in another memory order, an offset view."""
+    def run():
+        results = []
+        layer, _ = build(FORMS["lif maps"])
+        g = torch.Generator(device="cuda").manual_seed(1)
+        base = torch.randn(37, 3, 3, 5, 4, generator=g, device="cuda") * 3
+        odd = torch.randn(3 * 37 * 60 + 1, generator=g, device="cuda")[1:] * 3
+        for x in (base.transpose(0, 1), base.permute(1, 0, 3, 4, 2), base[:, :1].transpose(0, 1).expand(3, -1, -1, -1, -1),
+                  odd.view(3, 37, 3, 5, 4)):
+            x = x.detach().requires_grad_(True)
+            layer.reset_states()
+            out = layer(x)
+            out.backward(torch.randn(out.shape, generator=g, device="cuda").transpose(3, 4).contiguous().transpose(3, 4)
+                         if out.shape[3:] == (4, 4) else torch.randn(*out.shape[:2], out.shape[4], out.shape[2], out.shape[3],
+                                                                     generator=g, device="cuda").permute(0, 1, 3, 4, 2))
+            results += [out, x.grad]
+        return results
+    got = run()
+    python_functions()
+    for p, q in zip(got, run()):
+        assert torch.equal(p, q)
+
+
+def test_a_graph_used_twice_and_after_it_was_freed():
+    layer, x = build(FORMS["lif syn"])
+    out = layer(x)
+    go = torch.randn_like(out)
+    out.backward(go, retain_graph=True)
+    once = x.grad.clone()
+    out.backward(go)
+    assert torch.equal(x.grad, once + once)
+    with pytest.raises(RuntimeError, match="second time"):
+        out.backward(go)
+    layer.zero_grad()
+    out = layer(x)
+    only, = torch.autograd.grad(out, [layer.tau_syn], go)          # nothing else is asked for
+    layer.zero_grad(); layer.reset_states()
+    assert only.shape == layer.tau_syn.shape and x.grad is not None
+
+
+def test_values_modified_in_between_are_noticed():
+    for form in ("lif", "expleak alphas"):
+        layer, x = build(FORMS[form])
+        y = x * 1.0
+        out = layer(y)
+        with torch.no_grad():
+            y.add_(1.0)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            out.sum().backward()
+    layer, x = build(FORMS["lif"])                                 # a time constant may change before the backward pass
+    out = layer(x)
+    go = torch.randn_like(out)
+    out.backward(go, retain_graph=True)
+    was = layer.tau_mem.grad.clone()
+    layer.tau_mem.grad = None
+    with torch.no_grad():
+        layer.tau_mem.mul_(2.0)
+    out.backward(go)
+    assert torch.equal(layer.tau_mem.grad, was)
+
+
+@pytest.mark.parametrize("form", ["lif", "lif syn, alphas per neuron, records", "expleak alphas", "expleak fixed"])
+def test_hooks_on_saved_tensors_see_what_the_python_functions_save(form, python_functions):
+    def run():
+        seen = []
+
+        def pack(t):
+            seen.append(("pack", tuple(t.reshape(-1).shape), t.dtype))
+            return t.cpu()
+
+        layer, x = build(FORMS[form])
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: (seen.append("unpack"), t.cuda())[1]):
+            out = layer(x)
+        out.backward(torch.ones_like(out) * 0.3)
+        return seen, x.grad
+    seen, grad = run()
+    python_functions()
+    want, want_grad = run()
+    assert seen == want and torch.equal(grad, want_grad)
+
+
+def test_checkpointing_gives_the_same_gradients():
+    from torch.utils.checkpoint import checkpoint
+    layer, x = build(FORMS["lif syn"])
+    layer.reset_states()
+
+    def call(y):
+        layer.reset_states()
+        return layer(y)
+    out = call(x)
+    go = torch.randn_like(out)
+    out.backward(go)
+    want, want_tau = x.grad.clone(), layer.tau_mem.grad.clone()
+    x.grad = None
+    layer.zero_grad()
+    checkpoint(call, x, use_reentrant=False).backward(go)
+    assert torch.equal(x.grad, want) and torch.equal(layer.tau_mem.grad, want_tau)
+
+
+@pytest.mark.parametrize("form", ["lif syn, alphas per neuron, records", "expleak alphas", "iaf"])
+def test_memory_is_given_back_with_the_output(form):
+    layer, x = build(FORMS[form])
+    y = x * 1.0
+    out = layer(y)
+    gone = [weakref.ref(y), weakref.ref(out)]
+    before = torch.cuda.memory_allocated()
+    del out, y
+    layer.recordings = dict()
+    layer.zero_grad()
+    layer.firing_rate = None
+    gc.collect()
+    assert all(r() is None for r in gone)
+    assert torch.cuda.memory_allocated() < before
+    layer.reset_states()
+    torch.cuda.synchronize()
+    steady = []
+    for _ in range(3):
+        step(layer, x, "dense")
+        layer.zero_grad(); layer.recordings = dict(); layer.firing_rate = None; x.grad = None
+        gc.collect()
+        steady.append(torch.cuda.memory_allocated())
+    assert steady[1] == steady[2]
+
+
+@pytest.mark.parametrize("form", ["iaf", "iaf squeezed", "lif syn", "expleak", "expleak fixed"])
+@pytest.mark.parametrize("loss", ["sum", "rate"])
+def test_one_value_as_the_gradient_is_not_written_out(form, loss):
+    layer, _ = build(FORMS[form])
+    dims = FORMS[form].get("dims", (13,))
+    x = torch.randn(3, 1000, *dims[:-1], dims[-1] * 128, device="cuda")
+    x = (x.flatten(0, 1) if FORMS[form].get("squeeze") else x).requires_grad_(True)
+    out = layer(x)
+    value = out.sum() if loss == "sum" else layer.firing_rate * 2.0
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    value.backward()
+    assert torch.cuda.max_memory_allocated() - before < 1.5 * 4 * x.numel()     # the input's gradient and little else
+
+
+def test_replaced_wrappers_see_the_calls(monkeypatch):
+    from sinabs.exodus import _hip
+    for form, names in (("lif", ("layerLifForward", "layerLifBackward", "decayGrad")),
+                        ("expleak", ("layerLeakyForward", "layerLeakyBackward", "decayGrad"))):
+        for name in names:
+            seen, original = [], getattr(_hip, name)
+            monkeypatch.setattr(_hip, name, lambda *a, **k: (seen.append(name), original(*a, **k))[1])
+            layer, x = build(FORMS[form])
+            layer(x).sum().backward()
+            monkeypatch.undo()
+            assert seen == [name]
+
+
+def test_transforms_are_refused_as_before():
+    import torch.autograd.forward_ad as fw
+    for form in ("lif", "expleak"):
+        layer, x = build(FORMS[form])
+        layer(x)
+        layer.zero_grad()
+        with pytest.raises(RuntimeError, match="setup_context"):
+            torch.func.grad(lambda y: layer(y).sum())(x.detach())
+        with fw.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
+            layer(fw.make_dual(x.detach(), torch.ones_like(x)))
+
+
+@pytest.mark.parametrize("form", ["lif syn, alphas per neuron, records", "expleak", "expleak alphas"])
+def test_compiled_autograd(form):
+    from torch._dynamo import compiled_autograd
+    layer, x = build(FORMS[form])
+    out = layer(x)
+    out.backward(torch.full_like(out, 0.3))
+    want = [x.grad] + [p.grad for p in layer.parameters()]
+    layer, x = build(FORMS[form])
+    out = layer(x)
+    with compiled_autograd._enable(torch.compile(backend="eager")):
+        out.backward(torch.full_like(out, 0.3))
+    for p, q in zip([x.grad] + [p.grad for p in layer.parameters()], want):
+        assert (p is None) == (q is None) and (p is None or torch.equal(p, q))
+
+
+def test_batched_gradients_are_refused_as_before(python_functions):
+    for python in (False, True):
+        if python:
+            python_functions()
+        for form in ("lif", "expleak"):
+            layer, x = build(FORMS[form])
+            out = layer(x)
+            for gradient in (torch.randn(2, *out.shape, device="cuda"),
+                             torch.ones(2, device="cuda").view(2, *[1] * out.ndim).expand(2, *out.shape)):
+                with pytest.raises(RuntimeError):
+                    torch.autograd.grad(out, [x], gradient, is_grads_batched=True, retain_graph=True)
+
+
+def test_a_backward_pass_of_the_backward_pass_knows_no_more_than_before(python_functions):
+    def run():
+        layer, x = build(FORMS["lif"])
+        out = layer(x)
+        g, = torch.autograd.grad((out * 0.5).sum(), [x], create_graph=True)
+        return g, g.requires_grad
+    got = run()
+    python_functions()
+    want = run()
+    assert torch.equal(got[0], want[0]) and got[1] == want[1]
+
+
+def test_on_a_side_stream_and_without_steps():
+    layer, x = build(FORMS["lif syn"])
+    want = step(layer, x, "dense")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    layer, x = build(FORMS["lif syn"])
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        got = step(layer, x, "dense")
+    torch.cuda.current_stream().wait_stream(side)
+    for p, q in zip(got, want):
+        assert p is None or torch.equal(p, q)
+    empty = torch.zeros(3, 0, 13, device="cuda", requires_grad=True)
+    layer.reset_states()
+    out = layer(empty)
+    out.sum().backward()
+    assert out.shape == (3, 0, 13) and empty.grad.shape == (3, 0, 13)
