@@ -19,6 +19,12 @@ struct LayerConsts {
     int rec_pre;        // the potential record holds the value before the reset instead of after it
 };
 
+// where a forward kernel puts what its blocks counted
+struct Sums {
+    double *at;          // null: no total wanted
+    bool slots;          // one double per block's lanes neurons of a batch element, else one double in all
+};
+
 namespace {
 
 #ifndef EXODUS_LAYER_BLOCK
@@ -255,6 +261,24 @@ __device__ __forceinline__ float reset_amount(float v, const Neuron &n, const Ca
     return taken;
 }
 
+__device__ __forceinline__ float saturate(float x) { return fminf(fmaxf(x, 0.f), 1.f); }   // the clamp of the instruction before
+
+// v >= th ? 1 : 0 as saturate(v * scale + shift), for thresholds between 2^-100 and 2^100.  scale is the power of two that
+// takes th to [2^24, 2^25), or to 2^25 where th is a power of two itself: the float before th then lies 2 below it, th * scale
+// is an even integer and shift = 2 - th * scale a float.  So v == th gives 2, the float before it 0, and the one rounding of
+// the fused multiply-add cannot carry any other v to the wrong side (NaN saturates to 0, as the comparison fails for it).
+// The threshold of two spikes, 2 th, takes half the scale and the same shift.  Any other neuron gets a line that is always 0
+// and is done again from its threshold on (from every potential where 0 * c is no number).
+__device__ __forceinline__ void spike_line(float &scale, float &shift, float &redo, const Neuron &n, const Cap &cc)
+{
+    const bool usable = n.th >= 0x1p-100f && n.th <= 0x1p100f && fabsf(n.c) <= 0x1p126f;
+    const int bits = __float_as_int(n.th), exponent = (bits >> 23) - 127;
+    const float up = __uint_as_float(static_cast<unsigned>(((bits & 0x7fffff) ? 24 : 25) - exponent + 127) << 23);
+    scale = usable ? cc.one * up : 0.f;
+    shift = usable ? cc.one * (2.f - n.th * up) : 0.f;
+    redo = usable ? n.thd : (fabsf(n.c) < __builtin_inff() ? n.th : -__builtin_inff());
+}
+
 // compute units of the current device, asked for once per device
 inline int compute_units()
 {
@@ -420,6 +444,11 @@ inline bool too_wide(int64_t neurons) { return neurons >= (int64_t{1} << 25); }
 // the forward pass again, keeping nothing but the checkpoints (exodus_layer.hip)
 int exodus_layer_checkpoints_only(float *ckpt_v, float *ckpt_i, const float *x, const LayerConsts &p, bool syn, int64_t B,
                                   int64_t T, int64_t M, hipStream_t s);
+
+// the forward pass with three or four waves for 64 neurons (exodus_layer_forward_roles.hip)
+bool exodus_layer_forward_roles_apply(int64_t B, int64_t T, int64_t M);
+int exodus_layer_forward_roles(float *spikes, float *ckpt_v, float *ckpt_i, float *v_last, float *i_last, const Sums &sums,
+                               const float *x, const LayerConsts &p, int64_t B, int64_t T, int64_t M, hipStream_t s);
 
 // the backward pass with one lane per neuron and chunk of CKPT steps (exodus_layer_backward_split.hip)
 struct SplitArgs {
