@@ -19,6 +19,8 @@
 // Two drivers implement this scheme: scan_span_kernel for rows whose length is a multiple of 4 in
 // 16-byte aligned tensors (raw buffer instructions on the wave's span of memory, sectors shared by two
 // rows written whole), scan_kernel for everything else (global loads, element-wise at row boundaries).
+// Short rows in 16-byte aligned tensors have a driver of their own, whole_rows_kernel, which takes them as the
+// one piece of memory that they are.
 //
 // Arithmetic of the forward recurrences is written with explicit round-to-nearest multiplies and
 // adds (no fused multiply-add), in the operation order of the reference device code, so spike
@@ -478,6 +480,160 @@ scan_span_kernel(const Op op, const int64_t n_rows, const int n_steps, const int
 }
 
 // ---------------------------------------------------------------------------------------------
+// The driver for short rows.  ROWS rows of a wave are one piece of memory that starts and ends on 64 bytes (ROWS is a multiple
+// of 16, tensors are 16-byte aligned): all of it goes to LDS as it lies, in 16-byte pieces, whatever a row's length; a lane then
+// walks its row there, and the piece leaves the way it came.  No access touches a row's neighbour but inside the piece.
+// The drivers above fetch a row in tiles of 128 bytes, and what rows share at their ends again and in parts, which for rows of a few
+// tiles is most of it.  Before / here, us for 2^26 steps, spiking forward and backward, leaky forward and backward: 10 steps
+// 740 / 138, 1307 / 154, 357 / 88, 1162 / 148; 27 steps 618 / 142, 520 / 147, 279 / 88, 487 / 134; 65 steps 406 / 160, 265 / 193,
+// 189 / 97, 240 / 140; synaptic forward and backward 17 steps 829 / 187, 1977 / 192.  4.5 to 6.1 TB/s: what copies reach.
+// Word e of the piece lies at e + pad * (e / 64) in LDS: without a pad the lanes, whose rows lie an even number of words apart,
+// would meet in the same banks.
+// ---------------------------------------------------------------------------------------------
+constexpr int WHOLE_BATCH = 8;                                // accesses of a lane in flight per tensor, and steps read ahead
+constexpr int WHOLE_FOLD = 32;                                // steps whose sums are taken in fp32
+
+template <class Op, int ROWS>
+__global__ void __launch_bounds__(WAVE) whole_rows_kernel(const Op op, const int64_t n_rows, const int n_steps, const int pad,
+                                                          const int slot_words, const unsigned over_steps)
+{
+    constexpr int NIN = Op::NIN, NOUT = Op::NOUT, NDER = Op::NDER, NROWP = Op::NROWP;
+    constexpr int NSLOT = NIN > NOUT ? NIN : NOUT;
+    extern __shared__ f32x4 lds_raw[];
+    float *lds = reinterpret_cast<float *>(lds_raw);
+    float *rowp = lds + NSLOT * slot_words;                   // [ROWS][NROWP] constants for derive()
+
+    const int lane = threadIdx.x;
+    const int64_t row0 = static_cast<int64_t>(blockIdx.x) * ROWS;
+    const int n_loc = n_rows - row0 < ROWS ? static_cast<int>(n_rows - row0) : ROWS;   // rows of this wave
+    const bool row_ok = lane < n_loc;
+    const int words = n_loc * n_steps, chunks = words / 4, tail = words % 4;           // a tail in the last wave only
+    const int64_t e0 = row0 * n_steps;
+    const auto at = [&](int e) { return e + pad * (e >> 6); };
+
+    Rsrc rin[NIN > 0 ? NIN : 1], rout[NOUT > 0 ? NOUT : 1], rder;
+#pragma unroll
+    for (int j = 0; j < NIN; ++j) rin[j] = span_rsrc(op.in[j] + e0, 4u * words);
+#pragma unroll
+    for (int j = 0; j < NOUT; ++j) rout[j] = span_rsrc(op.out[j] + e0, 4u * words);
+    if constexpr (NDER > 0) rder = span_rsrc(op.der + e0, 4u * words);
+
+    for (int c0 = lane; c0 < chunks + lane; c0 += WAVE * WHOLE_BATCH) {
+        f32x4 v[NIN][WHOLE_BATCH];
+#pragma unroll
+        for (int k = 0; k < WHOLE_BATCH; ++k) {
+            const int c = c0 + k * WAVE;
+            const unsigned off = c < chunks ? 16u * c : OUTSIDE;
+#pragma unroll
+            for (int j = 0; j < NIN; ++j) v[j][k] = span_load<true>(rin[j], off);
+        }
+#pragma unroll
+        for (int k = 0; k < WHOLE_BATCH; ++k) {
+            const int c = c0 + k * WAVE;
+            if (c < chunks) {
+#pragma unroll
+                for (int j = 0; j < NIN; ++j) *reinterpret_cast<f32x4 *>(lds + j * slot_words + at(4 * c)) = v[j][k];
+            }
+        }
+    }
+    if (lane < tail) {
+#pragma unroll
+        for (int j = 0; j < NIN; ++j) lds[j * slot_words + at(4 * chunks + lane)] = op.in[j][e0 + 4 * chunks + lane];
+    }
+    typename Op::State st;
+    op.init(st, row_ok ? row0 + lane : n_rows - 1, row_ok);
+    if constexpr (NDER > 0) {
+        float consts[NROWP > 0 ? NROWP : 1];
+        op.stash(st, consts);
+        if (lane < ROWS) {
+#pragma unroll
+            for (int k = 0; k < NROWP; ++k) rowp[lane * NROWP + k] = consts[k];
+        }
+    }
+    wave_sync();
+
+    if (row_ok) {
+        const int first = lane * n_steps;
+        const auto word = [&](int i) { return at(first + (Op::REVERSE ? n_steps - 1 - i : i)); };   // of the i-th step walked
+        float x[WHOLE_BATCH][NIN], ahead[WHOLE_BATCH][NIN];
+        const auto read = [&](float(&to)[WHOLE_BATCH][NIN], int i) {
+#pragma unroll
+            for (int k = 0; k < WHOLE_BATCH; ++k) {
+                const int w = word(i + k < n_steps ? i + k : n_steps - 1);
+#pragma unroll
+                for (int j = 0; j < NIN; ++j) to[k][j] = lds[j * slot_words + w];
+            }
+        };
+        const auto walk = [&](const float *in, int i) {
+            float y[NOUT > 0 ? NOUT : 1];
+            op.step(st, in, y);
+            const int w = word(i);
+#pragma unroll
+            for (int j = 0; j < NOUT; ++j) lds[j * slot_words + w] = y[j];
+        };
+        read(x, 0);
+        int i = 0;
+        for (; i + WHOLE_BATCH <= n_steps; i += WHOLE_BATCH) {
+            read(ahead, i + WHOLE_BATCH);                     // (the last step's inputs may be read again: not used)
+#pragma unroll
+            for (int k = 0; k < WHOLE_BATCH; ++k) walk(x[k], i + k);
+            if (i % WHOLE_FOLD == WHOLE_FOLD - WHOLE_BATCH) op.end_tile(st);
+#pragma unroll
+            for (int k = 0; k < WHOLE_BATCH; ++k)
+#pragma unroll
+                for (int j = 0; j < NIN; ++j) x[k][j] = ahead[k][j];
+        }
+#pragma unroll
+        for (int k = 0; k < WHOLE_BATCH - 1; ++k)
+            if (i + k < n_steps) walk(x[k], i + k);
+        op.end_tile(st);
+    }
+    wave_sync();
+
+    if constexpr (NOUT > 0) {
+        // the row of a word by a multiplication: exact for e * (n_steps - 1) < 2^32, over_steps = 2^32 / n_steps rounded up
+        const auto row_of = [&](int e) {
+            const int r = n_steps == 1 ? e : static_cast<int>(__umulhi(static_cast<unsigned>(e), over_steps));
+            return r < ROWS ? r : ROWS - 1;
+        };
+        for (int c0 = lane; c0 < chunks; c0 += WAVE) {
+            const unsigned off = 16u * c0;
+#pragma unroll
+            for (int j = 0; j < NOUT; ++j) {
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(lds + j * slot_words + at(4 * c0));
+                span_store(v, rout[j], off);
+                if constexpr (NDER > 0) {
+                    if (j == Op::DER_SRC) {
+                        const int r = row_of(4 * c0);
+                        f32x4 d = op.derive(rowp + r * NROWP, v);
+                        if (row_of(4 * c0 + 3) != r) {
+#pragma unroll
+                            for (int k = 1; k < 4; ++k) {
+                                const float dk = op.derive(rowp + row_of(4 * c0 + k) * NROWP, v)[k];
+                                d[k] = dk;
+                            }
+                        }
+                        span_store(d, rder, off);
+                    }
+                }
+            }
+        }
+        if (lane < tail) {
+            const int e = 4 * chunks + lane;
+#pragma unroll
+            for (int j = 0; j < NOUT; ++j) {
+                const float v = lds[j * slot_words + at(e)];
+                op.out[j][e0 + e] = v;
+                if constexpr (NDER > 0) {
+                    if (j == Op::DER_SRC) op.der[e0 + e] = op.derive(rowp + row_of(e) * NROWP, f32x4{v, v, v, v})[0];
+                }
+            }
+        }
+    }
+    if (row_ok) op.finish(st, row0 + lane);
+}
+
+// ---------------------------------------------------------------------------------------------
 // Ops
 // ---------------------------------------------------------------------------------------------
 struct LeakyFwdOp {
@@ -913,6 +1069,38 @@ struct SpanPlan {
     static constexpr int UQ = EXODUS_SPAN_UNROLL_Q;
 };
 
+// The driver for short rows: words of LDS between the 64-word blocks of a piece.  The lanes' rows lie t words apart, 17 t / 16 with
+// a pad of 4: where that is close to a multiple of 64 the pad itself brings them together (t = 60: leaky forward 107 -> 131 us).
+inline int whole_pad(int64_t t)
+{
+    if (t % 2) return 0;
+    const int64_t sixteenths = 17 * t % 1024;
+    return sixteenths < 48 || sixteenths > 1024 - 48 ? 12 : 4;
+}
+inline size_t whole_slot_words(int64_t rows, int64_t t)
+{
+    const int64_t words = (rows * t + 3) / 4 * 4;
+    return static_cast<size_t>(words + whole_pad(t) * (words / 64 + 1));
+}
+
+// How many rows of t steps a wave of that driver takes; 0: one of the others.  Fewer rows leave lanes without one but let more waves
+// share a compute unit's LDS; `slots` tensors lie there.  us for 2^26 steps, spiking forward (one slot) and backward (two),
+// synaptic backward (three), 64 rows / 32: 16 steps 140 / 143, 142 / 180, 203 / 299; 24 steps 142 / 140, 145 / 153, 210 / 252;
+// 33 steps 152 / 148, 149 / 146, 232 / 216; one slot, 32 rows / 16: 61 steps 153 / 158, 65 steps 166 / 160, 121 steps 230 / 202.
+// Against scan_kernel, where rows are no multiple of 4 steps: one slot 150 steps 239 / 236 (leaky 121 / 106), 201 steps 234 / 277;
+// more slots 90 steps 294 / 244, 110 steps 272 / 276 (leaky 249 / 162), 130 steps 215 / 345.
+// Against scan_span_kernel, multiples of 4: 12 steps 331 / 137, 425 / 142; 28 steps 420 / 142, 235 / 138; 44 steps 206 / 144,
+// 229 / 162, 392 / 261; 56 steps 179 / 147, 196 / 172, 328 / 274; 60 steps 171 / 148, 193 / 195, 319 / 354; 68 steps 155 / 159,
+// 171 / 204, 276 / 365.  Rows of whole 64-byte
+// sectors suit that driver: 16 steps 160 / 140, 226 / 142, 366 / 203, but 32 steps 135 / 140, 145 / 149, 213 / 234, 48 steps
+// 172 / 146, 165 / 169, 240 / 257.
+inline int whole_rows(int slots, int64_t t)
+{
+    const int64_t most = t % 16 == 0 ? 16 : (t % 4 == 0 ? (slots > 2 ? 56 : 60) : (slots == 1 ? 150 : 100));
+    if (t > most || slots * 32 * t * 4 > 40 * 1024) return 0;
+    return t <= 24 ? 64 : (slots > 1 || t <= 64 ? 32 : 16);
+}
+
 template <class Op, int TT>
 int launch_rows(const Op &op, int64_t n, int64_t t, bool vec, void *stream)
 {
@@ -950,14 +1138,36 @@ int launch_rows(const Op &op, int64_t n, int64_t t, bool vec, void *stream)
     return static_cast<int>(hipGetLastError());
 }
 
+template <class Op, int ROWS>
+int launch_whole(const Op &op, int64_t n, int64_t t, void *stream)
+{
+    constexpr int NSLOT = Op::NIN > Op::NOUT ? Op::NIN : Op::NOUT;
+    const int64_t n_blocks = (n + ROWS - 1) / ROWS;
+    if (n_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+    const int pad = whole_pad(t);
+    const size_t slot = whole_slot_words(ROWS, t);
+    hipLaunchKernelGGL((whole_rows_kernel<Op, ROWS>), dim3(static_cast<unsigned>(n_blocks)), dim3(WAVE),
+                       (NSLOT * slot + ROWS * Op::NROWP) * sizeof(float), static_cast<hipStream_t>(stream), op, n, static_cast<int>(t), pad,
+                       static_cast<int>(slot), static_cast<unsigned>(((uint64_t{1} << 32) + t - 1) / t));
+    return static_cast<int>(hipGetLastError());
+}
+
 // `TT_GENERIC` is the tile length of the driver for rows of any length and alignment
 template <class Op, int TT_GENERIC>
 int launch(const Op &op, int64_t n, int64_t t, void *stream)
 {
-    bool vec = (t % 4) == 0;
-    for (int j = 0; j < Op::NIN; ++j) vec = vec && aligned16(op.in[j]);
-    for (int j = 0; j < Op::NOUT; ++j) vec = vec && aligned16(op.out[j]);
-    if constexpr (Op::NDER > 0) vec = vec && aligned16(op.der);   // the derived output leaves through the same stores
+    bool aligned = true;
+    for (int j = 0; j < Op::NIN; ++j) aligned = aligned && aligned16(op.in[j]);
+    for (int j = 0; j < Op::NOUT; ++j) aligned = aligned && aligned16(op.out[j]);
+    if constexpr (Op::NDER > 0) aligned = aligned && aligned16(op.der);   // the derived output leaves through the same stores
+    if (aligned) {
+        switch (whole_rows(Op::NIN > Op::NOUT ? Op::NIN : Op::NOUT, t)) {
+        case 64: return launch_whole<Op, 64>(op, n, t, stream);
+        case 32: return launch_whole<Op, 32>(op, n, t, stream);
+        case 16: return launch_whole<Op, 16>(op, n, t, stream);
+        }
+    }
+    const bool vec = aligned && t % 4 == 0;
     if (vec && t <= (1 << 22)) return launch_rows<Op, SpanPlan<Op>::TT>(op, n, t, true, stream);
     return launch_rows<Op, TT_GENERIC>(op, n, t, false, stream);
 }
