@@ -266,6 +266,27 @@ int64_t exodus_decay_work(int64_t batch, int64_t neurons, int64_t period);
 int exodus_decay_grad(float *grad_tau, double *work, const float *grad_alpha, const float *tau, int64_t batch,
                       int64_t neurons, int64_t period, void *stream);
 
+/* Time constants in the place of decay factors, for the two calls below: the forward kernel does what exodus_decay_expand does, and
+ * no launch of its own is needed for it.  For each constant that is given (period 1 or neurons, as above) the factors of all
+ * batch * neurons entries are written to alpha and a copy of the constants to kept; the call's own pointer to the factors is not
+ * looked at.  A constant that is NULL leaves its factors to that pointer. */
+typedef struct exodus_layer_decays {
+    const float *tau_mem, *tau_syn;
+    int64_t period_mem, period_syn;
+    float *alpha_mem, *alpha_syn, *kept_mem, *kept_syn;
+} exodus_layer_decays;
+int exodus_layer_lif_forward_decays(float *out_spikes, float *out_vmem_rec, float *out_isyn_rec, float *ckpt_v,
+                                    float *ckpt_i, float *v_last, float *i_last, double *spike_sum, double *sum_work,
+                                    const exodus_layer_decays *decays, const float *input, const float *vmem_post_initial,
+                                    const float *isyn_initial, const float *alpha_mem, const float *alpha_syn,
+                                    const float *membr_subtract, const float *theta, const float *theta_low,
+                                    int apply_theta_low, int max_num_spikes, int decay_early, int norm_input,
+                                    int record_pre_reset, int64_t batch, int64_t t, int64_t neurons, void *stream);
+int exodus_layer_leaky_forward_decays(float *out, float *v_last, double *out_sum, double *sum_work,
+                                      const exodus_layer_decays *decays, const float *input, const float *vmem_initial,
+                                      const float *alpha, int decay_early, int norm_input, int64_t batch, int64_t t,
+                                      int64_t neurons, void *stream);
+
 /* How exodus_layer_lif_backward spreads a layer over the machine.  Its ordinary kernel gives every neuron one lane that
  * walks the whole sequence, which leaves most of the GPU idle when a layer has few neurons (the reference's kernels
  * have the same shape: one thread per row, reference cuda/lif_kernels.h:296-311).  A second kernel gives every chunk of

@@ -102,6 +102,7 @@ __global__ void __launch_bounds__((SYN ? 4 : 3) * WAVE) layer_lif_forward_roles(
     cc.one = p.cap >= 1u ? 1.f : 0.f;
     Neuron n = {};
     neuron_load<SYN, CAPK>(n, p, row);
+    decays_load<SYN>(n, p, b, row - b * M, row, active && wave == 0);
 
     if (wave == 0) {
         float scale = SYN ? n.xs : n.k;

@@ -44,8 +44,8 @@ using Eight = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor,
 #define EXODUS_ENTRIES(X)                                                                                               \
     X(exodus_hip_abi_version)                                                                                           \
     X(exodus_lif_forward) X(exodus_lif_backward_fused) X(exodus_leaky_forward) X(exodus_leaky_backward_fused)           \
-    X(exodus_layer_sum_slots) X(exodus_layer_checkpoint_interval) X(exodus_layer_lif_forward_total)                     \
-    X(exodus_layer_lif_backward) X(exodus_layer_lif_backward_from_input) X(exodus_layer_leaky_forward_total)            \
+    X(exodus_layer_sum_slots) X(exodus_layer_checkpoint_interval) X(exodus_layer_lif_forward_decays)                    \
+    X(exodus_layer_lif_backward) X(exodus_layer_lif_backward_from_input) X(exodus_layer_leaky_forward_decays)            \
     X(exodus_layer_leaky_backward) X(exodus_decay_expand) X(exodus_decay_work) X(exodus_decay_grad)
 struct Library {
 #define EXODUS_MEMBER(name) decltype(&::name) name = nullptr;
@@ -217,7 +217,9 @@ Shape state_shape_of(const std::optional<Shape> &asked, int64_t n)
 // ---------------------------------------------------------------------------------------------
 // layers on (batch, time, neurons)
 // ---------------------------------------------------------------------------------------------
-Eight layer_lif_forward(const Tensor &input, const Tensor &v_init, const Maybe &i_init, const Tensor &alpha_mem,
+// time constants whose decay factors the forward kernel works out (`decays`) into alpha_mem / alpha_syn
+Eight layer_lif_forward_decays(const exodus_layer_decays *decays, const Tensor &input, const Tensor &v_init, const Maybe &i_init,
+                            const Tensor &alpha_mem,
                             const Maybe &alpha_syn, const Tensor &subtract, const Tensor &theta, const Maybe &theta_low,
                             bool apply_low, int64_t max_spikes, bool decay_early, bool norm_input, bool want_checkpoints,
                             bool want_records, bool want_pre_reset, bool want_sum, const Maybe &out_spikes,
@@ -248,12 +250,23 @@ Eight layer_lif_forward(const Tensor &input, const Tensor &v_init, const Maybe &
         if (syn) i_last.copy_(i_init->reshape(states));
     }
     launch(input, "exodus_layer_lif_forward_total", [&](void *stream) {
-        return lib.exodus_layer_lif_forward_total(
+        return lib.exodus_layer_lif_forward_decays(
             out(spikes), out(v_rec), out(i_rec), out(ckpt_v), out(ckpt_i), out(v_last), out(i_last), out64(total), out64(work),
-            input.const_data_ptr<float>(), v0, i0, am, as, c, th, lo, apply_low, static_cast<int>(max_spikes), decay_early,
+            decays, input.const_data_ptr<float>(), v0, i0, am, as, c, th, lo, apply_low, static_cast<int>(max_spikes), decay_early,
             norm_input, want_pre_reset, b, t, m, stream);
     });
     return {spikes, v_last, i_last, ckpt_v, ckpt_i, v_rec, i_rec, total};
+}
+
+Eight layer_lif_forward(const Tensor &input, const Tensor &v_init, const Maybe &i_init, const Tensor &alpha_mem,
+                        const Maybe &alpha_syn, const Tensor &subtract, const Tensor &theta, const Maybe &theta_low, bool apply_low,
+                        int64_t max_spikes, bool decay_early, bool norm_input, bool want_checkpoints, bool want_records,
+                        bool want_pre_reset, bool want_sum, const Maybe &out_spikes, const std::optional<Shape> &state_shape,
+                        const py::handle place)
+{
+    return layer_lif_forward_decays(nullptr, input, v_init, i_init, alpha_mem, alpha_syn, subtract, theta, theta_low, apply_low,
+                                    max_spikes, decay_early, norm_input, want_checkpoints, want_records, want_pre_reset, want_sum,
+                                    out_spikes, state_shape, place);
 }
 
 // -> (grad_input, alpha_mem, alpha_syn, v_init, i_init)
@@ -347,8 +360,9 @@ Five layer_lif_backward(const Tensor &grad_spikes, const Maybe &grad_v_last, con
 }
 
 // -> (out, v_last, total)
-Three layer_leaky_forward(const Tensor &input, const Tensor &v_init, const Tensor &alpha, bool decay_early, bool norm_input,
-                              const std::optional<Shape> &state_shape, bool want_sum, const py::handle place)
+Three layer_leaky_forward_decays(const exodus_layer_decays *decays, const Tensor &input, const Tensor &v_init, const Tensor &alpha,
+                              bool decay_early, bool norm_input, const std::optional<Shape> &state_shape, bool want_sum,
+                              const py::handle place)
 {
     three(input, "input");
     const int64_t b = input.size(0), t = input.size(1), m = input.size(2), n = b * m;
@@ -359,11 +373,17 @@ Three layer_leaky_forward(const Tensor &input, const Tensor &v_init, const Tenso
     if (want_sum) total_and_work(input, total, work);
     if (t == 0) v_last.copy_(v_init.reshape(states));
     launch(input, "exodus_layer_leaky_forward_total", [&](void *stream) {
-        return lib.exodus_layer_leaky_forward_total(out(result), out(v_last), out64(total), out64(work),
-                                                    input.const_data_ptr<float>(), v0, a, decay_early, norm_input, b, t, m,
-                                                    stream);
+        return lib.exodus_layer_leaky_forward_decays(out(result), out(v_last), out64(total), out64(work), decays,
+                                                     input.const_data_ptr<float>(), v0, a, decay_early, norm_input, b, t, m,
+                                                     stream);
     });
     return {result, v_last, total};
+}
+
+Three layer_leaky_forward(const Tensor &input, const Tensor &v_init, const Tensor &alpha, bool decay_early, bool norm_input,
+                          const std::optional<Shape> &state_shape, bool want_sum, const py::handle place)
+{
+    return layer_leaky_forward_decays(nullptr, input, v_init, alpha, decay_early, norm_input, state_shape, want_sum, place);
 }
 
 // -> (grad_input, alpha, v_init)
@@ -580,7 +600,7 @@ Three leaky_backward_fused(const Tensor &grad_out, const Tensor &alpha, const Ma
 // know): the same tensors saved in the same order, the same gradients.  The engine runs a backward pass on a thread of its own,
 // where Python means the interpreter lock, cold caches and thirteen unpacked tensors; and the input's shape is taken and given
 // back here instead of by reshapes that are nodes of their own.  us per training step in Python and here: IAF (8, 100, 256)
-// 131 / 86, LIF (32, 100, 512) with a trained time constant 155 / 118, LIF with synapses (4, 2000, 512), both constants trained, 189 / 152.
+// 136 / 99, LIF (32, 100, 512) with a trained time constant 160 / 114, LIF with synapses (4, 2000, 512), both constants trained, 199 / 143.
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
@@ -658,7 +678,23 @@ double from_bits(int64_t n)
     return x;
 }
 
+// What a forward kernel is to work out from the time constant `tau`, where nobody has (`alpha` absent): allocates alpha and kept.
+void to_work_out(const Maybe &tau, Maybe &alpha, Maybe &kept, const float *&source, int64_t &period, float *&to, float *&copy,
+                 const Tensor &like, int64_t neurons, int64_t n)
+{
+    if (!has(tau) || has(alpha)) return;
+    dev(*tau, "tau", &like);
+    if (tau->numel() != 1 && tau->numel() != neurons) refuse("tau must hold one value or one per neuron");
+    alpha = fresh({n}, like);
+    kept = fresh(tau->sizes(), like);
+    source = tau->const_data_ptr<float>();
+    period = tau->numel();
+    to = out(*alpha);
+    copy = out(*kept);
+}
+
 struct LifCall {
+    const exodus_layer_decays *decays;
     bool syn, apply_low, decay_early, norm_input, records, need_grad;
     int64_t max_spikes, kind;
     double p0, p1;
@@ -679,8 +715,8 @@ struct LifLayer : torch::autograd::Function<LifLayer> {
         edges.add(true);                                       // the input
         const int e_am = edges.add(true), e_as = edges.add(has(alpha_syn)), e_v0 = edges.add(true), e_i0 = edges.add(has(i_init));
         const int e_tm = edges.add(has(tau_mem)), e_ts = edges.add(has(tau_syn));
-        const auto [spikes, v_last, i_last, ckpt_v, ckpt_i, v_rec, i_rec, total] = layer_lif_forward(
-            shaped(input, shape), shaped(v_init, {n}), shaped(i_init, {n}), alpha_mem, alpha_syn, subtract, theta, theta_low,
+        const auto [spikes, v_last, i_last, ckpt_v, ckpt_i, v_rec, i_rec, total] = layer_lif_forward_decays(
+            c.decays, shaped(input, shape), shaped(v_init, {n}), shaped(i_init, {n}), alpha_mem, alpha_syn, subtract, theta, theta_low,
             c.apply_low, c.max_spikes, c.decay_early, c.norm_input, c.need_grad, c.records, false, true, Maybe(), c.states, c.place);
         ctx->set_materialize_grads(false);
         if (c.need_grad)
@@ -747,18 +783,30 @@ bool graph_wanted(std::initializer_list<const Tensor *> given, std::initializer_
 
 // -> (spikes, v_last, total, i_last, v_rec, i_rec) in the input's shape and the states' shape, with their place in the graph.
 // tau_mem / tau_syn: the parameters that alpha_mem / alpha_syn were worked out from (decay_expand, which also made kept_mem /
-// kept_syn) and whose gradients are wanted in the place of theirs.
-Eight layer_lif(const Tensor &input, const Tensor &alpha_mem, const Maybe &alpha_syn, const Tensor &v_init, const Maybe &i_init,
-                const Maybe &tau_mem, const Maybe &tau_syn, const Maybe &kept_mem, const Maybe &kept_syn, const Tensor &theta,
+// kept_syn) and whose gradients are wanted in the place of theirs; without factors the forward kernel works them out.
+Eight layer_lif(const Tensor &input, Maybe alpha_mem, Maybe alpha_syn, const Tensor &v_init, const Maybe &i_init,
+                const Maybe &tau_mem, const Maybe &tau_syn, Maybe kept_mem, Maybe kept_syn, const Tensor &theta,
                 const Tensor &subtract, const Maybe &theta_low, int kind, double p0, double p1, int64_t max_spikes, bool decay_early,
                 bool norm_input, bool records, const Shape &states, const py::handle place)
 {
+    const Shape shape = three_of(input);
+    const int64_t n = shape[0] * shape[2];
+    exodus_layer_decays decays{};
+    // (a call without steps launches nothing that would write the factors)
+    if (input.numel() > 0) {
+        to_work_out(tau_mem, alpha_mem, kept_mem, decays.tau_mem, decays.period_mem, decays.alpha_mem, decays.kept_mem, input, shape[2], n);
+        to_work_out(tau_syn, alpha_syn, kept_syn, decays.tau_syn, decays.period_syn, decays.alpha_syn, decays.kept_syn, input, shape[2], n);
+    } else {
+        if (has(tau_mem) && !has(alpha_mem)) std::tie(alpha_mem, kept_mem) = decay_expand(*tau_mem, shape[0], shape[2]);
+        if (has(tau_syn) && !has(alpha_syn)) std::tie(alpha_syn, kept_syn) = decay_expand(*tau_syn, shape[0], shape[2]);
+    }
     const bool syn = has(alpha_syn);
-    const bool need_grad = graph_wanted({&input, &alpha_mem, &v_init, &theta, &subtract}, {&alpha_syn, &i_init, &tau_mem, &tau_syn,
+    const Tensor &am = present(alpha_mem, "alphaMem");
+    const bool need_grad = graph_wanted({&input, &am, &v_init, &theta, &subtract}, {&alpha_syn, &i_init, &tau_mem, &tau_syn,
                                                                                            &theta_low});
-    const LifCall call{syn, has(theta_low), decay_early, norm_input, records, need_grad, max_spikes, kind, p0, p1, states,
+    const LifCall call{&decays, syn, has(theta_low), decay_early, norm_input, records, need_grad, max_spikes, kind, p0, p1, states,
                        kept_mem, kept_syn, place};
-    const variable_list out = LifLayer::apply(input, alpha_mem, alpha_syn, v_init, i_init, tau_mem, tau_syn, theta, subtract,
+    const variable_list out = LifLayer::apply(input, am, alpha_syn, v_init, i_init, tau_mem, tau_syn, theta, subtract,
                                               theta_low, call);
     const auto nth = [&](bool given, size_t k) { return given ? out[k] : Tensor(); };
     const size_t rec = syn ? 4 : 3;
@@ -766,6 +814,7 @@ Eight layer_lif(const Tensor &input, const Tensor &alpha_mem, const Maybe &alpha
 }
 
 struct LeakyCall {
+    const exodus_layer_decays *decays;
     bool decay_early, norm_input, need_grad, need_alpha;
     const Shape &states;
     const Maybe &kept;
@@ -777,7 +826,7 @@ struct LeakyLayer : torch::autograd::Function<LeakyLayer> {
                                  const LeakyCall &c)
     {
         const Shape shape = three_of(input);
-        auto [flat, v_last, total] = layer_leaky_forward(shaped(input, shape), shaped(v_init, {shape[0] * shape[2]}), alpha,
+        auto [flat, v_last, total] = layer_leaky_forward_decays(c.decays, shaped(input, shape), shaped(v_init, {shape[0] * shape[2]}), alpha,
                                                          c.decay_early, c.norm_input, c.states, true, c.place);
         const Tensor result = shaped(flat, input.sizes());
         ctx->set_materialize_grads(false);
@@ -825,12 +874,19 @@ struct LeakyLayer : torch::autograd::Function<LeakyLayer> {
     }
 };
 
-// -> (out in the input's shape, v_last, total); tau and kept as above
-Three layer_leaky(const Tensor &input, const Tensor &alpha, const Tensor &v_init, const Maybe &tau, const Maybe &kept,
-                  bool decay_early, bool norm_input, const Shape &states, const py::handle place)
+// -> (out in the input's shape, v_last, total); tau as above, in the place of alpha_given
+Three layer_leaky(const Tensor &input, Maybe alpha_given, const Tensor &v_init, const Maybe &tau, bool decay_early, bool norm_input,
+                  const Shape &states, const py::handle place)
 {
+    const Shape shape = three_of(input);
+    Maybe kept;
+    exodus_layer_decays decays{};
+    if (has(tau) && input.numel() == 0) std::tie(alpha_given, kept) = decay_expand(*tau, shape[0], shape[2]);
+    to_work_out(tau, alpha_given, kept, decays.tau_mem, decays.period_mem, decays.alpha_mem, decays.kept_mem, input, shape[2],
+                shape[0] * shape[2]);
+    const Tensor &alpha = present(alpha_given, "alpha");
     const bool need_alpha = has(tau) ? tau->requires_grad() : alpha.requires_grad();
-    const LeakyCall call{decay_early, norm_input, graph_wanted({&input, &alpha, &v_init}, {&tau}), need_alpha, states, kept, place};
+    const LeakyCall call{&decays, decay_early, norm_input, graph_wanted({&input, &alpha, &v_init}, {&tau}), need_alpha, states, kept, place};
     const variable_list out = LeakyLayer::apply(input, alpha, v_init, tau, call);
     return {out[0], out[1], out[2]};
 }

@@ -51,12 +51,14 @@ _SIGNATURES = {
     "exodus_layer_sum_slots": ([_i64, _i64], _i64),
     "exodus_layer_lif_forward": ([_p] * 16 + [_int, _int, _int, _int, _int, _i64, _i64, _i64, _p], _int),
     "exodus_layer_lif_forward_total": ([_p] * 17 + [_int, _int, _int, _int, _int, _i64, _i64, _i64, _p], _int),
+    "exodus_layer_lif_forward_decays": ([_p] * 18 + [_int, _int, _int, _int, _int, _i64, _i64, _i64, _p], _int),
     "exodus_layer_lif_backward": ([_p] * 18 + [_int, _int, _int, _int, _int, _f, _f, _p, _p, _p, _int, _i64, _i64, _i64, _p], _int),
     "exodus_layer_backward_time_split": ([_int], _int),
     "exodus_layer_scratch_floats": ([], _i64),
     "exodus_layer_lif_backward_from_input": ([_p] * 16 + [_int, _int, _int, _int, _int, _f, _f, _p, _p, _p, _int, _i64, _i64, _i64, _p], _int),
     "exodus_layer_leaky_forward": ([_p] * 6 + [_int, _int, _i64, _i64, _i64, _p], _int),
     "exodus_layer_leaky_forward_total": ([_p] * 7 + [_int, _int, _i64, _i64, _i64, _p], _int),
+    "exodus_layer_leaky_forward_decays": ([_p] * 8 + [_int, _int, _i64, _i64, _i64, _p], _int),
     "exodus_layer_leaky_backward": ([_p] * 9 + [_int, _int, _int, _i64, _i64, _i64, _p], _int),
     "exodus_decay_expand": ([_p, _p, _p, _i64, _i64, _i64, _p], _int),
     "exodus_layer_launch_shape": ([_int, _i64, _i64, _p, _p], _int),
@@ -453,18 +455,17 @@ def layerLif(input, alphaMem, alphaSyn, vmemPostInitial, isynInitial, tauMem, ta
     """The pass of ``layerLifForward`` as a node of the autograd graph, for the surrogates that the kernels evaluate:
     (spikes, v_last, spike_sum, i_last | None, v_rec | None, i_rec | None).  ``input`` and the initial states may have any
     contiguous shape (``input`` (batch, time, ...)); spikes and records come in that of ``input``.  ``tauMem`` / ``tauSyn`` are
-    the time constants to be trained in the place of ``alphaMem`` / ``alphaSyn``, which ``decayExpand`` worked out from them
-    together with ``keptMem`` / ``keptSyn``."""
+    time constants to be trained in the place of the decay factors; ``alphaMem`` / ``alphaSyn`` and ``keptMem`` / ``keptSyn`` are
+    then what ``decayExpand`` made of them, or None: the forward kernel does it."""
     return _native.layer_lif(input, alphaMem, alphaSyn, vmemPostInitial, isynInitial, tauMem, tauSyn, keptMem, keptSyn, theta,
                              membrSubtract, thetaLow, surrogateKind, surrP0, surrP1, _cap(maxNumSpikes), bool(decayEarly),
                              bool(normInput), bool(records), stateShape, _place(input))[:6]
 
 
-def layerLeaky(input, alpha, vmemInitial, tau, kept, decayEarly: bool, normInput: bool, stateShape):
-    """The pass of ``layerLeakyForward`` as a node of the autograd graph, (out, v_last, out_sum); shapes, ``tau`` and ``kept``
-    as for ``layerLif``."""
-    return _native.layer_leaky(input, alpha, vmemInitial, tau, kept, bool(decayEarly), bool(normInput), stateShape,
-                               _place(input))
+def layerLeaky(input, alpha, vmemInitial, tau, decayEarly: bool, normInput: bool, stateShape):
+    """The pass of ``layerLeakyForward`` as a node of the autograd graph, (out, v_last, out_sum); shapes as for ``layerLif``,
+    ``tau`` a time constant to be trained in the place of ``alpha`` (then None)."""
+    return _native.layer_leaky(input, alpha, vmemInitial, tau, bool(decayEarly), bool(normInput), stateShape, _place(input))
 
 
 # stamps(kept, values): a tuple with one entry per value, the entries of ``kept`` (an earlier result, or None) where a value is

@@ -92,7 +92,8 @@ def test_as_the_python_functions(form, loss, python_functions):
     if loss == "chained" and FORMS[form].get("squeeze"):
         pytest.skip("covered by the other forms")
     layer, x = build(FORMS[form])
-    got = step(layer, x, loss)
+    first = [None if z is None else z.detach().clone() for z in step(layer, x, loss)]    # with the checks of the parameters' values
+    got = step(layer, x, loss)                                     # without
     assert FORMS[form].get("squeeze") or "LayerFunction" not in layer(x).grad_fn.name()    # (behind a reshape in the others)
     python_functions()
     layer, x = build(FORMS[form])
@@ -101,7 +102,41 @@ def test_as_the_python_functions(form, loss, python_functions):
     for k, (p, q) in enumerate(zip(got, want)):
         assert (p is None) == (q is None), k
         if p is not None:
-            assert p.shape == q.shape and torch.equal(p, q), k
+            assert p.shape == q.shape and torch.equal(p, q) and torch.equal(first[k], q), k
+
+
+# one block, waves with roles, blocks of one and of four waves, two and four neurons per lane, a sequence without steps
+@pytest.mark.parametrize("b,t,m", [(1, 10, 300), (1, 40, 64), (3, 40, 70), (40, 33, 1000), (30, 4, 700), (9, 3, 66560), (33, 2, 131072),
+                                   (2, 0, 5)])
+@pytest.mark.parametrize("per_neuron", [False, True])
+def test_decay_factors_worked_out_by_the_forward_kernels(b, t, m, per_neuron):
+    from sinabs.exodus import _hip
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = (torch.randn(b, t, m, generator=g, device="cuda") * 4 + 0.5).requires_grad_(True)
+    go = torch.randn(b, t, m, generator=g, device="cuda")
+    taus = [(5.0 + 40.0 * torch.rand(m if per_neuron else (), generator=g, device="cuda")).requires_grad_(True) for _ in range(2)]
+    z, one = torch.zeros(b, m, device="cuda"), torch.ones(b * m, device="cuda")
+
+    def run(expand, syn):
+        tm, ts = taus[0], taus[1] if syn else None
+        am, km, as_, ks = None, None, None, None
+        if expand:
+            am, km = _hip.decayExpand(tm, b, m)
+            if syn:
+                as_, ks = _hip.decayExpand(ts, b, m)
+        out = _hip.layerLif(x, am, as_, z, z if syn else None, tm, ts, km, ks, one, one, None, 1, 0.5, 1.0, -1, True, True, False, (b, m))
+        grads = torch.autograd.grad(out[0], [x, tm] + ([ts] if syn else []), go)
+        return [out[0], out[1], out[2], *grads] + ([out[3]] if syn else [])
+    for syn in (False, True):
+        for p, q in zip(run(False, syn), run(True, syn)):
+            assert torch.equal(p, q)
+    alpha, kept = _hip.decayExpand(taus[0], b, m)
+    out, last, total = _hip.layerLeaky(x, None, z, taus[0], True, True, (b, m))
+    grads = torch.autograd.grad(out, [x, taus[0]], go)
+    want = _hip.layerLeakyForward(x.detach(), z.flatten(), alpha, True, True, wantSum=True)
+    gx, ga, _ = _hip.layerLeakyBackward(go, None, want[0], x.detach(), z.flatten(), alpha, True, True, True)
+    for p, q in zip((out, last.flatten(), total, *grads), (*want, gx, _hip.decayGrad(ga, kept, b, m))):
+        assert torch.equal(p, q)
 
 
 def test_other_layouts_of_input_and_gradient(python_functions):
