@@ -206,7 +206,8 @@ int exodus_layer_lif_forward(float *out_spikes, float *out_vmem_rec, float *out_
 
 /* The same with a total (one double, NULL = not wanted) that is written instead of added to: every block leaves its count
  * in sum_work, exodus_layer_sum_slots(batch, neurons) doubles that need no initialising (one per so many neurons of a batch
- * element, the same number for every size and device), and a second kernel of the call adds them up.  Many waves that add to one double at the end of a launch wait for each other; here none does. */
+ * element, the same number for every size and device), and a second kernel of the call adds them up (a call of one block writes
+ * its total itself).  Many waves that add to one double at the end of a launch wait for each other; here none does. */
 int exodus_layer_lif_forward_total(float *out_spikes, float *out_vmem_rec, float *out_isyn_rec, float *ckpt_v,
                                    float *ckpt_i, float *v_last, float *i_last, double *spike_sum, double *sum_work,
                                    const float *input, const float *vmem_post_initial,
@@ -219,7 +220,8 @@ int64_t exodus_layer_sum_slots(int64_t batch, int64_t neurons);
 /* Neurons per lane and lanes per block that a layer kernel is launched with on the current device, for tensors on 64-byte
  * boundaries (results do not depend on either).  EXODUS_SHAPE_FORWARD_RECORDS records potential and current,
  * EXODUS_SHAPE_BACKWARD is the backward with one lane per neuron, whatever exodus_layer_backward_time_split says,
- * EXODUS_SHAPE_BACKWARD_MORE the one with gradients on state records or a surrogate tensor. */
+ * EXODUS_SHAPE_BACKWARD_MORE the one with gradients on state records or a surrogate tensor.  The answer is for the kernels that walk a
+ * neuron in one lane; a small layer's forward may share 64 neurons out to several waves or run in one block instead. */
 #define EXODUS_SHAPE_FORWARD 0
 #define EXODUS_SHAPE_FORWARD_RECORDS 1
 #define EXODUS_SHAPE_LEAKY_FORWARD 2

@@ -15,7 +15,7 @@ import tempfile
 HERE = os.path.dirname(os.path.abspath(__file__))
 SRCS = [os.path.join(HERE, "csrc", f) for f in ("exodus_hip.hip", "exodus_layer.hip", "exodus_layer_backward.hip",
                                                   "exodus_layer_forward_roles.hip", "exodus_layer_backward_split.hip",
-                                                  "exodus_hbm.hip")]
+                                                  "exodus_layer_leaky_split.hip", "exodus_hbm.hip")]
 SRC = SRCS[0]
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 OUT = os.path.join(HERE, "sinabs", "exodus", "libexodus_hip.so")

@@ -464,6 +464,45 @@ __device__ __forceinline__ unsigned layer_block(unsigned run)
     return gridDim.x - start < many ? blockIdx.x : start + at % XCDS * run + at / XCDS;
 }
 
+constexpr int SPLIT_LANES = 512;
+constexpr int SPLIT_CHUNKS = 32;           // most chunks of a group
+constexpr int SPLIT_NEURONS = 64;          // most neurons of a block
+
+// How the kernels that give every chunk of CKPT steps a lane of its own spread a layer: chunks of a group and neurons of a block.
+struct SplitShape {
+    int64_t blocks_per_batch;
+    int neurons_log, lanes;
+};
+
+inline SplitShape split_shape(int64_t B, int64_t T, int64_t M)
+{
+    const int64_t n_ck = (T + CKPT - 1) / CKPT;
+    // 256 registers per lane leave a compute unit eight waves, one block of more than four.  A launch of more such blocks than
+    // there are compute units takes another round of them, so it takes smaller groups of chunks instead: 16 chunks of 32
+    // neurons in the place of 32 of 16, and where that is too many blocks 8 of 32, two blocks to a compute unit.  Without /
+    // with, us: 16 384 neurons 300 steps 26.8 / 21.9, 512 steps 31.0 / 25.4, with synapses 37.7 / 29.6, 2000 steps 171 / 107,
+    // with state records 309 / 203, with a surrogate tensor 188 / 130; 10 240 neurons 300 steps 22.2 / 18.8; 8192 neurons
+    // 1000 steps 41 / 30.  Where one round does, smaller groups only lengthen the chain: 8192 neurons 300 steps 12.5 / 15.8,
+    // 4096 neurons 1000 steps with synapses 25.6 / 28.2.  (Up to 8 chunks of 64 neurons are one round for 16 384 neurons.)
+    const auto blocks = [&](int log) { return ((M + (int64_t{1} << log) - 1) >> log) * B; };
+    const int64_t cus = compute_units();
+    int most = SPLIT_CHUNKS, widest = 6;
+    if (n_ck > 16 && blocks(4) > cus) most = 16;
+    if (n_ck > 8 && blocks(5) > cus) {
+        most = 8;
+        widest = 5;
+    }
+    const int64_t groups = (n_ck + most - 1) / most;
+    const int chunks = static_cast<int>((n_ck + groups - 1) / groups);
+    // as many neurons per block as its lanes hold, but no more than the layer has
+    int neurons_log = 4;
+    while (neurons_log < widest && (chunks << (neurons_log + 1)) <= SPLIT_LANES && (int64_t{1} << neurons_log) < M)
+        ++neurons_log;
+    const int64_t blocks_per_batch = (M + (int64_t{1} << neurons_log) - 1) >> neurons_log;
+    const int lanes = ((chunks << neurons_log) + WAVE - 1) / WAVE * WAVE;
+    return {blocks_per_batch, neurons_log, lanes};
+}
+
 inline bool bad3(int64_t b, int64_t t, int64_t m)
 {
     if (b < 0 || t < 0 || m < 0) return true;
@@ -494,6 +533,16 @@ struct SplitArgs {
     float p0, p1, inv_p0;
     int64_t T, M;
 };
-// the kernel keeps the offsets of 32 chunks below 2^31 bytes
+// the backward pass of the leaky layer with one lane per neuron and chunk (exodus_layer_leaky_split.hip)
+struct LeakySplitArgs {
+    float *grad_x, *alpha_grad, *v_init_grad;
+    const float *grad_out, *grad_v_last, *out, *x, *v_init, *alpha;
+    int decay_early, norm_input;
+    int64_t T, M;
+};
+bool exodus_layer_leaky_split_applies(int64_t B, int64_t T, int64_t M);
+int exodus_layer_leaky_split(const LeakySplitArgs &a, bool uniform, int64_t B, hipStream_t s);
+
+// the kernels keep the offsets of 32 chunks below 2^31 bytes
 inline bool exodus_layer_split_applies(int64_t neurons) { return neurons < (int64_t{1} << 19); }
 int exodus_layer_backward_split(const SplitArgs &a, bool syn, int kind, bool uniform, int64_t B, hipStream_t s);

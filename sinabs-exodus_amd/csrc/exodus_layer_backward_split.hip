@@ -33,9 +33,6 @@ namespace {
 // neuron).  512 lanes per block leave 256 registers per lane: the four values of 32 steps and all but 12 to 28 bytes of the
 // rest, 132 to 156 with a synapse and state records, go into them.  Sums of a neuron's gradients are fp32 over 8 steps and
 // fp64 beyond: against float64 their error is 0.7 to 0.8 times the one-lane kernel's, that of grad_x the same.
-constexpr int SPLIT_LANES = 512;
-constexpr int SPLIT_CHUNKS = 32;           // most chunks of a group
-constexpr int SPLIT_NEURONS = 64;          // most neurons of a block
 static_assert(CKPT == 32, "a chunk's clamped steps are bits of an unsigned, a_syn^CKPT is squared up, a group spans 2^10 steps");
 
 // EXTRA: gradients on the state records; GO1: one value as the gradient of every spike (see the one-lane kernel)
@@ -282,33 +279,10 @@ __global__ void __launch_bounds__(SPLIT_LANES) layer_lif_backward_split(const Sp
 template <bool SYN, int KIND, int CAPK, bool EXTRA, bool GO1>
 int launch(const SplitArgs &a, int64_t B, hipStream_t s)
 {
-    const int64_t n_ck = (a.T + CKPT - 1) / CKPT;
-    // 256 registers per lane leave a compute unit eight waves, one block of more than four.  A launch of more such blocks than
-    // there are compute units takes another round of them, so it takes smaller groups of chunks instead: 16 chunks of 32
-    // neurons in the place of 32 of 16, and where that is too many blocks 8 of 32, two blocks to a compute unit.  Without /
-    // with, us: 16 384 neurons 300 steps 26.8 / 21.9, 512 steps 31.0 / 25.4, with synapses 37.7 / 29.6, 2000 steps 171 / 107,
-    // with state records 309 / 203, with a surrogate tensor 188 / 130; 10 240 neurons 300 steps 22.2 / 18.8; 8192 neurons
-    // 1000 steps 41 / 30.  Where one round does, smaller groups only lengthen the chain: 8192 neurons 300 steps 12.5 / 15.8,
-    // 4096 neurons 1000 steps with synapses 25.6 / 28.2.  (Up to 8 chunks of 64 neurons are one round for 16 384 neurons.)
-    const auto blocks = [&](int log) { return ((a.M + (int64_t{1} << log) - 1) >> log) * B; };
-    const int64_t cus = compute_units();
-    int most = SPLIT_CHUNKS, widest = 6;
-    if (n_ck > 16 && blocks(4) > cus) most = 16;
-    if (n_ck > 8 && blocks(5) > cus) {
-        most = 8;
-        widest = 5;
-    }
-    const int64_t groups = (n_ck + most - 1) / most;
-    const int chunks = static_cast<int>((n_ck + groups - 1) / groups);
-    // as many neurons per block as its lanes hold, but no more than the layer has
-    int neurons_log = 4;
-    while (neurons_log < widest && (chunks << (neurons_log + 1)) <= SPLIT_LANES && (int64_t{1} << neurons_log) < a.M)
-        ++neurons_log;
-    const int64_t blocks_per_batch = (a.M + (int64_t{1} << neurons_log) - 1) >> neurons_log;
-    if (blocks_per_batch > 0x7fffffffLL / B) return hipErrorInvalidValue;
-    const int lanes = ((chunks << neurons_log) + WAVE - 1) / WAVE * WAVE;
-    hipLaunchKernelGGL((layer_lif_backward_split<SYN, KIND, CAPK, EXTRA, GO1>), dim3(static_cast<unsigned>(blocks_per_batch * B)),
-                       dim3(lanes), 0, s, a, blocks_per_batch, neurons_log);
+    const SplitShape shape = split_shape(B, a.T, a.M);
+    if (shape.blocks_per_batch > 0x7fffffffLL / B) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((layer_lif_backward_split<SYN, KIND, CAPK, EXTRA, GO1>), dim3(static_cast<unsigned>(shape.blocks_per_batch * B)),
+                       dim3(shape.lanes), 0, s, a, shape.blocks_per_batch, shape.neurons_log);
     return static_cast<int>(hipGetLastError());
 }
 

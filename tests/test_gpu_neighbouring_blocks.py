@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 # (63), 512 and 600 (32, 88 left over); two and four neurons per lane; half lines shared, and none
 @pytest.mark.parametrize("b,t,m", [
     (1, 3, 65), (7, 3, 65), (8, 3, 65), (9, 35, 65), (100, 3, 65), (101, 33, 65),
-    (255, 3, 300), (256, 3, 300), (300, 34, 300), (5, 2, 110002), (5, 3, 1048580), (300, 3, 272), (300, 3, 288),
+    (255, 3, 300), (256, 3, 300), (300, 30, 300), (5, 2, 110002), (5, 3, 1048580), (300, 3, 272), (300, 3, 288),
 ])
 @pytest.mark.parametrize("syn,records", [(False, False), (True, True)])
 def test_runs_of_blocks(b, t, m, syn, records):
