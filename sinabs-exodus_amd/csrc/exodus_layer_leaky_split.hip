@@ -150,9 +150,11 @@ int launch(const LeakySplitArgs &a, bool uniform, int64_t B, hipStream_t s)
     if (shape.blocks_per_batch > 0x7fffffffLL / B) return hipErrorInvalidValue;
     const dim3 grid(static_cast<unsigned>(shape.blocks_per_batch * B)), block(shape.lanes);
     if (uniform)
-        hipLaunchKernelGGL((layer_leaky_backward_split<ALPHA, WITH_X, true>), grid, block, 0, s, a, shape.blocks_per_batch, shape.neurons_log);
+        hipLaunchKernelGGL((layer_leaky_backward_split<ALPHA, WITH_X, true>), grid, block, 0, s, a, shape.blocks_per_batch,
+                           shape.neurons_log);
     else
-        hipLaunchKernelGGL((layer_leaky_backward_split<ALPHA, WITH_X, false>), grid, block, 0, s, a, shape.blocks_per_batch, shape.neurons_log);
+        hipLaunchKernelGGL((layer_leaky_backward_split<ALPHA, WITH_X, false>), grid, block, 0, s, a, shape.blocks_per_batch,
+                           shape.neurons_log);
     return static_cast<int>(hipGetLastError());
 }
 

@@ -826,7 +826,8 @@ struct LeakyLayer : torch::autograd::Function<LeakyLayer> {
                                  const LeakyCall &c)
     {
         const Shape shape = three_of(input);
-        auto [flat, v_last, total] = layer_leaky_forward_decays(c.decays, shaped(input, shape), shaped(v_init, {shape[0] * shape[2]}), alpha,
+        auto [flat, v_last, total] = layer_leaky_forward_decays(c.decays, shaped(input, shape),
+                                                                shaped(v_init, {shape[0] * shape[2]}), alpha,
                                                          c.decay_early, c.norm_input, c.states, true, c.place);
         const Tensor result = shaped(flat, input.sizes());
         ctx->set_materialize_grads(false);
@@ -886,7 +887,8 @@ Three layer_leaky(const Tensor &input, Maybe alpha_given, const Tensor &v_init, 
                 shape[0] * shape[2]);
     const Tensor &alpha = present(alpha_given, "alpha");
     const bool need_alpha = has(tau) ? tau->requires_grad() : alpha.requires_grad();
-    const LeakyCall call{&decays, decay_early, norm_input, graph_wanted({&input, &alpha, &v_init}, {&tau}), need_alpha, states, kept, place};
+    const bool need_grad = graph_wanted({&input, &alpha, &v_init}, {&tau});
+    const LeakyCall call{&decays, decay_early, norm_input, need_grad, need_alpha, states, kept, place};
     const variable_list out = LeakyLayer::apply(input, alpha, v_init, tau, call);
     return {out[0], out[1], out[2]};
 }
