@@ -614,14 +614,29 @@ Shape three_of(const Tensor &x)
     return {x.size(0), x.size(1), elements(Shape(x.sizes().begin() + 2, x.sizes().end()))};
 }
 
-// what allocates the large results of a backward pass, as of now
-py::handle place_now(const Tensor &like)
-{
-    py::gil_scoped_acquire locked;
-    if (place_of == nullptr) return Py_None;
-    const py::object found = py::reinterpret_borrow<py::object>(place_of)(like);
-    return found;                                              // a function of a module, or None: both outlive this reference
-}
+// What allocates the large results of a backward pass, as of now; held until the call has returned, as nobody else need hold it.
+// The interpreter lock is taken a second time only where something was found.
+class PlaceNow {
+    PyObject *found = Py_None;                                 // None: not held
+
+public:
+    explicit PlaceNow(const Tensor &like)
+    {
+        if (place_of == nullptr) return;
+        py::gil_scoped_acquire locked;
+        py::object place = py::reinterpret_borrow<py::object>(place_of)(like);
+        if (!place.is_none()) found = place.release().ptr();
+    }
+    PlaceNow(const PlaceNow &) = delete;
+    PlaceNow &operator=(const PlaceNow &) = delete;
+    ~PlaceNow()
+    {
+        if (found == Py_None) return;
+        py::gil_scoped_acquire locked;
+        Py_DECREF(found);
+    }
+    operator py::handle() const { return found; }
+};
 
 // One value that `grad` repeats everywhere (the gradient of a sum of the output), as a tensor of one element.
 Tensor one_value(const Tensor &grad)
@@ -759,7 +774,7 @@ struct LifLayer : torch::autograd::Function<LifLayer> {
             shaped(maybe(i_init), {n}), saved[5], maybe(saved[6]), saved[7], saved[8], maybe(saved[9]), apply_low, call[5],
             decay_early, norm_input, static_cast<int>(call[6]), from_bits(call[7]), from_bits(call[8]), Maybe(), Maybe(),
             dense(grad_v_rec, shape), dense(grad_i_rec, shape), needs(e_am) || tau_mem, needs(e_as) || tau_syn, needs(e_v0),
-            needs(e_i0), uniform, place_now(input));
+            needs(e_i0), uniform, PlaceNow(input));
         if (ctx->needs_input_grad(0)) result[0] = shaped(g_x, input.sizes());
         if (needs(e_am)) result[1] = g_am;
         if (needs(e_as)) result[2] = g_as;
@@ -863,7 +878,7 @@ struct LeakyLayer : torch::autograd::Function<LeakyLayer> {
             g, dense(grads[1]), need_alpha ? maybe(shaped(out, shape)) : Maybe(),
             input.defined() ? maybe(shaped(input, shape)) : Maybe(), need_alpha ? maybe(shaped(saved[1], {n})) : Maybe(), alpha,
             decay_early, norm_input, need_alpha, uniform ? std::optional<Shape>(shape) : std::nullopt,
-            place_now(uniform ? g.expand(shape) : g));
+            PlaceNow(uniform ? g.expand(shape) : g));
         if (ctx->needs_input_grad(0)) result[0] = shaped(g_x, full);
         if (tau) {
             if (ctx->needs_input_grad(3)) result[3] = decay_grad(g_a, saved[4], shape[0], shape[2]);

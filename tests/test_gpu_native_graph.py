@@ -362,3 +362,31 @@ def test_on_a_side_stream_and_without_steps():
     out = layer(empty)
     out.sum().backward()
     assert out.shape == (3, 0, 13) and empty.grad.shape == (3, 0, 13)
+
+
+@pytest.mark.parametrize("form", ["lif syn", "expleak"])
+def test_what_allocates_the_gradients_lives_until_it_has_done_so(form):
+    """An allocator that nobody holds but the backward pass that asked for it."""
+    import ctypes
+    from sinabs.exodus import _hip
+    addresses = {name: ctypes.cast(getattr(_hip.lib, name), ctypes.c_void_p).value for name in _hip._SIGNATURES}
+    events, kept = [], []
+
+    class Allocator:
+        def __call__(self, shape, like):
+            events.append("called")
+            return torch.empty(shape, device=like.device)
+
+        def __del__(self):
+            events.append("gone")
+            kept.append(self)                                  # whoever still calls it finds an object
+
+    layer, x = build(FORMS[form])
+    want = [None if z is None else z.detach().clone() for z in step(layer, x, "dense")]
+    _hip._native.bind(addresses, _hip._check, lambda like: Allocator())
+    try:
+        got = step(layer, x, "dense")
+    finally:
+        _hip._native.bind(addresses, _hip._check, _hip._place)
+    assert events == ["called", "gone"]
+    assert all(p is None or torch.equal(p, q) for p, q in zip(got, want))
