@@ -24,7 +24,7 @@ from .spike import classify_surrogate
 
 # the wrappers that the Functions below call; a program that puts its own in their place (to log or to check) sees the calls
 _WRAPPERS = tuple((name, getattr(_hip, name)) for name in (
-    "layerLifForward", "layerLifBackward", "layerLeakyForward", "layerLeakyBackward", "decayGrad"))
+    "layerLifForward", "layerLifBackward", "layerLeakyForward", "layerLeakyBackward", "decayExpand", "decayGrad"))
 _PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 

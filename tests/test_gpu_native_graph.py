@@ -293,6 +293,19 @@ def test_replaced_wrappers_see_the_calls(monkeypatch):
             assert seen == [name]
 
 
+@pytest.mark.parametrize("form,constants", [("lif", 1), ("lif syn", 2), ("expleak", 1)])
+def test_a_replaced_decay_expand_sees_every_call(form, constants, monkeypatch):
+    """Also a call whose parameters are those of the call before, which are not checked again."""
+    from sinabs.exodus import _hip
+    layer, x = build(FORMS[form])
+    layer(x).sum().backward()
+    layer.reset_states()
+    seen, original = [], _hip.decayExpand
+    monkeypatch.setattr(_hip, "decayExpand", lambda *a, **k: (seen.append(1), original(*a, **k))[1])
+    layer(x).sum().backward()
+    assert len(seen) == constants
+
+
 def test_transforms_are_refused_as_before():
     import torch.autograd.forward_ad as fw
     for form in ("lif", "expleak"):
