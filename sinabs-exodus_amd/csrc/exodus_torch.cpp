@@ -249,7 +249,8 @@ Eight layer_lif_forward_decays(const exodus_layer_decays *decays, const Tensor &
         v_last.copy_(v_init.reshape(states));
         if (syn) i_last.copy_(i_init->reshape(states));
     }
-    launch(input, "exodus_layer_lif_forward_total", [&](void *stream) {
+    const bool worked_out = decays && (decays->tau_mem || decays->tau_syn);
+    launch(input, worked_out ? "exodus_layer_lif_forward_decays" : "exodus_layer_lif_forward_total", [&](void *stream) {
         return lib.exodus_layer_lif_forward_decays(
             out(spikes), out(v_rec), out(i_rec), out(ckpt_v), out(ckpt_i), out(v_last), out(i_last), out64(total), out64(work),
             decays, input.const_data_ptr<float>(), v0, i0, am, as, c, th, lo, apply_low, static_cast<int>(max_spikes), decay_early,
@@ -372,7 +373,8 @@ Three layer_leaky_forward_decays(const exodus_layer_decays *decays, const Tensor
     Tensor total, work;
     if (want_sum) total_and_work(input, total, work);
     if (t == 0) v_last.copy_(v_init.reshape(states));
-    launch(input, "exodus_layer_leaky_forward_total", [&](void *stream) {
+    const bool worked_out = decays && decays->tau_mem;
+    launch(input, worked_out ? "exodus_layer_leaky_forward_decays" : "exodus_layer_leaky_forward_total", [&](void *stream) {
         return lib.exodus_layer_leaky_forward_decays(out(result), out(v_last), out64(total), out64(work), decays,
                                                      input.const_data_ptr<float>(), v0, a, decay_early, norm_input, b, t, m,
                                                      stream);

@@ -161,6 +161,20 @@ def test_a_status_of_the_library_becomes_its_own_exception():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("constant", [False, True])
+def test_the_entry_point_that_failed_is_the_one_named(constant):
+    h = hip()
+    x, r = torch.zeros(1, 1, h.LAYER_MAX_NEURONS).cuda(), torch.ones(h.LAYER_MAX_NEURONS).cuda()
+    tau, alpha = (torch.ones(1).cuda(), None) if constant else (None, r)
+    form = "decays" if constant else "total"
+    with pytest.raises(h.ExodusHipError, match=f"exodus_layer_leaky_forward_{form} failed"):
+        h.layerLeaky(x, alpha, r, tau, False, False, (1, h.LAYER_MAX_NEURONS))
+    with pytest.raises(h.ExodusHipError, match=f"exodus_layer_lif_forward_{form} failed"):
+        h.layerLif(x, alpha, None, r, None, tau, None, None, None, r, r, None, 1, 0.5, 1.0, -1, False, False, False,
+                   (1, h.LAYER_MAX_NEURONS))
+
+
+@pytest.mark.gpu
 def test_running_out_of_memory_is_torchs_exception():
     tau = torch.ones(1).cuda()
     with pytest.raises(torch.OutOfMemoryError):
