@@ -221,7 +221,8 @@ int64_t exodus_layer_sum_slots(int64_t batch, int64_t neurons);
  * boundaries (results do not depend on either).  EXODUS_SHAPE_FORWARD_RECORDS records potential and current,
  * EXODUS_SHAPE_BACKWARD is the backward with one lane per neuron, whatever exodus_layer_backward_time_split says,
  * EXODUS_SHAPE_BACKWARD_MORE the one with gradients on state records or a surrogate tensor.  The answer is for the kernels that walk a
- * neuron in one lane; a small layer's forward may share 64 neurons out to several waves or run in one block instead. */
+ * neuron in one lane; a small layer's forward may share 64 neurons out to several waves or run in one block instead, and its
+ * backward (EXODUS_SHAPE_LEAKY_BACKWARD and _ALPHA too) may be split over time (exodus_layer_backward_time_split). */
 #define EXODUS_SHAPE_FORWARD 0
 #define EXODUS_SHAPE_FORWARD_RECORDS 1
 #define EXODUS_SHAPE_LEAKY_FORWARD 2
@@ -289,15 +290,16 @@ int exodus_layer_leaky_forward_decays(float *out, float *v_last, double *out_sum
                                       const float *alpha, int decay_early, int norm_input, int64_t batch, int64_t t,
                                       int64_t neurons, void *stream);
 
-/* How exodus_layer_lif_backward spreads a layer over the machine.  Its ordinary kernel gives every neuron one lane that
+/* How exodus_layer_lif_backward and exodus_layer_leaky_backward spread a layer over the machine.  Their ordinary kernels give every neuron one lane that
  * walks the whole sequence, which leaves most of the GPU idle when a layer has few neurons (the reference's kernels
- * have the same shape: one thread per row, reference cuda/lif_kernels.h:296-311).  A second kernel gives every chunk of
+ * have the same shape: one thread per row, reference cuda/lif_kernels.h:296-311).  A second kernel of each gives every chunk of
  * 32 steps of every neuron a lane of its own (the adjoint recurrences are affine, so the chunks can be composed
- * afterwards): the same gradients to fp32 rounding, not bit for bit.  It takes every call of more than 32 steps and fewer
+ * afterwards): the same gradients to fp32 rounding, not bit for bit, and grouped by batch * neurons and by the number of
+ * compute units of the device.  It takes every call of more than 32 steps and fewer
  * than 2^19 neurons per batch element.  mode 0: never use it; 1 (default): for layers of up to 16 384 neurons (batch *
- * neurons); 2: for layers of any size without synapse, with an in-kernel surrogate (kind 1..3), without grad_v_rec and
- * with at most 512 steps, and no others; 3: whenever it applies; any other value changes nothing.  Returns the mode that
- * was set before.  Process-wide. */
+ * neurons); 2: for spiking layers of any size without synapse, with an in-kernel surrogate (kind 1..3), without grad_v_rec
+ * and with at most 512 steps, and no other spiking ones (leaky layers as with 1); 3: whenever it applies; any other value
+ * changes nothing.  Returns the mode that was set before.  Process-wide. */
 int exodus_layer_backward_time_split(int mode);
 
 /* exodus_layer_lif_backward for callers that cannot allocate device memory -- code under HIP graph
@@ -344,7 +346,8 @@ int exodus_layer_leaky_forward_total(float *out, float *v_last, double *out_sum,
  * and `vmem_initial`, and `input` when one of the input scalings is on) and vmem_init_grad;
  * grad_v_last (batch*neurons, optional) is a gradient arriving at the final state.
  * grad_out_uniform != 0: `grad_out` points at ONE float that stands for every element (as grad_spikes_uniform of
- * exodus_layer_lif_backward). */
+ * exodus_layer_lif_backward).  Small layers run the second kernel of exodus_layer_backward_time_split, whose gradients agree
+ * with the other's to fp32 rounding: a batch that is split or padded to another size may get other last bits (mode 0: never). */
 int exodus_layer_leaky_backward(float *grad_input, float *alpha_grad, float *vmem_init_grad,
                                 const float *grad_out, const float *grad_v_last, const float *out,
                                 const float *input, const float *vmem_initial, const float *alpha,

@@ -541,6 +541,7 @@ struct LeakySplitArgs {
     int64_t T, M;
 };
 bool exodus_layer_leaky_split_applies(int64_t B, int64_t T, int64_t M);
+int exodus_layer_split_mode();             // what exodus_layer_backward_time_split has set
 int exodus_layer_leaky_split(const LeakySplitArgs &a, bool uniform, int64_t B, hipStream_t s);
 
 // the kernels keep the offsets of 32 chunks below 2^31 bytes

@@ -261,6 +261,8 @@ int dispatch_bwd_cap(unsigned cap, A... a)
 
 }  // namespace
 
+int exodus_layer_split_mode() { return split_mode.load(std::memory_order_relaxed); }
+
 // ---------------------------------------------------------------------------------------------
 // Checkpoint memory of exodus_layer_lif_backward_from_input, the one entry point that must not
 // allocate.  Every GPU the library runs on holds its own copy of this array, at its own address,
@@ -340,7 +342,7 @@ EXODUS_API int exodus_layer_lif_backward(float *grad_input, float *alpha_mem_gra
     p.rec_pre = 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
     // few neurons, many steps: one lane per chunk of 32 steps instead of one lane per neuron
-    const int mode = split_mode.load(std::memory_order_relaxed);
+    const int mode = exodus_layer_split_mode();
     const bool plain = !syn && surrogate_kind != EXODUS_SURR_TENSOR && !grad_v_rec && t <= SPLIT_PLAIN_CHUNKS * CKPT;
     if (t > CKPT && exodus_layer_split_applies(neurons) &&
         ((mode == 1 && batch * neurons <= SPLIT_MOST_NEURONS) || (mode == 2 && plain) || mode == 3))

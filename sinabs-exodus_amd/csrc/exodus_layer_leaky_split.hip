@@ -166,7 +166,9 @@ int launch(const LeakySplitArgs &a, bool uniform, int64_t B, hipStream_t s)
 constexpr int64_t LEAKY_SPLIT_MOST_NEURONS = 16384;
 bool exodus_layer_leaky_split_applies(int64_t B, int64_t T, int64_t M)
 {
-    return T > CKPT && B * M <= LEAKY_SPLIT_MOST_NEURONS && exodus_layer_split_applies(M);
+    const int mode = exodus_layer_split_mode();
+    if (mode == 0 || T <= CKPT || !exodus_layer_split_applies(M)) return false;
+    return mode == 3 || B * M <= LEAKY_SPLIT_MOST_NEURONS;
 }
 
 int exodus_layer_leaky_split(const LeakySplitArgs &a, bool uniform, int64_t B, hipStream_t s)

@@ -497,10 +497,10 @@ def decayGrad(gradAlpha, tau, batch: int, neurons: int):
 
 
 def backwardTimeSplit(mode: int = -1) -> int:
-    """How ``layerLifBackward`` treats layers with few neurons and many steps (``exodus_layer_backward_time_split``):
-    0 never splits the sequence over lanes, 1 (default) does for layers of up to 16 384 neurons, 2 for layers of any size
-    without synapse, with an in-kernel surrogate, at most 512 steps and no gradients on state records, 3 whenever the
-    kernel applies; -1 only asks.  Returns the mode that was set before."""
+    """How ``layerLifBackward`` and ``layerLeakyBackward`` treat layers with few neurons and many steps
+    (``exodus_layer_backward_time_split``): 0 never splits the sequence over lanes, 1 (default) does for layers of up to 16 384
+    neurons, 2 for spiking layers of any size without synapse, with an in-kernel surrogate, at most 512 steps and no gradients
+    on state records (leaky ones as 1), 3 whenever the kernels apply; -1 only asks.  Returns the mode that was set before."""
     return int(lib.exodus_layer_backward_time_split(int(mode)))
 
 

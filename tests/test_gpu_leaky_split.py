@@ -34,19 +34,22 @@ def run(b, t, m, early, norm, gvl, uniform, alpha, split, poke=None):
     go = torch.full((b, t, m), 0.7, device="cuda") if uniform else R(b, t, m)
     if poke is not None:
         poke(go)
-    if not split:                                              # the same elements in a batch too large for the kernel
-        more = -(-16385 // m)
-        rep = lambda z: None if z is None else torch.cat([z, z[:1].expand(more, *z.shape[1:])]).contiguous()
-        x, v0, gl, a, go = map(rep, (x, v0, gl, a, go))
-    k = x.shape[0]
+    before = hip.backwardTimeSplit(3 if split else 0)
+    try:
+        return calls(hip, b, t, m, early, norm, x, v0, gl, a, go, uniform)
+    finally:
+        hip.backwardTimeSplit(before)
+
+
+def calls(hip, b, t, m, early, norm, x, v0, gl, a, go, uniform):
     out = hip.layerLeakyForward(x, v0.flatten(), a.flatten(), early, norm)[0]
     one = torch.full((1,), 0.7, device="cuda")
     gx, ga, gv = hip.layerLeakyBackward(one if uniform else go, None if gl is None else gl.flatten(), out, x, v0.flatten(), a.flatten(),
-                                        early, norm, True, shape=(k, t, m) if uniform else None)
+                                        early, norm, True, shape=(b, t, m) if uniform else None)
     plain = hip.layerLeakyBackward(one if uniform else go, None if gl is None else gl.flatten(), None, None, None, a.flatten(), early,
-                                   norm, False, shape=(k, t, m) if uniform else None)
+                                   norm, False, shape=(b, t, m) if uniform else None)
     assert torch.equal(torch.nan_to_num(plain[0]), torch.nan_to_num(gx)) and plain[1] is None
-    return (gx[:b], ga.view(k, m)[:b], gv.view(k, m)[:b]), (go[:b], None if gl is None else gl[:b], out[:b], x[:b], v0[:b], a[:b], early, norm)
+    return (gx, ga.view(b, m), gv.view(b, m)), (go, gl, out, x, v0, a, early, norm)
 
 
 @pytest.mark.parametrize("t", [33, 63, 64, 65, 96, 257, 300, 512, 513, 1024, 1025, 1100])
@@ -82,3 +85,26 @@ def test_what_a_fold_would_spoil(kind):
     for p, q in zip(got, want):
         some = q[torch.isfinite(q)].abs()
         assert torch.allclose(p, q, rtol=1e-5, atol=1e-5 * float(some.max()) if some.numel() else 0.0, equal_nan=True)
+
+
+@pytest.mark.parametrize("early,norm", [(False, False), (True, True)])
+def test_the_switch_of_the_spiking_layers_is_theirs_too(early, norm):
+    """Mode 0 gives the kernel with one lane per neuron, which a batch beyond the limit of 16 384 neurons has in mode 1."""
+    from sinabs.exodus import _hip as hip
+    b, t, m = 41, 300, 400                                     # 16 400 neurons
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x, go = (torch.randn(b, t, m, generator=g, device="cuda") for _ in range(2))
+    a, v0 = 0.6 + 0.399 * torch.rand(b, m, generator=g, device="cuda"), torch.randn(b, m, generator=g, device="cuda")
+
+    def backward(mode, some):
+        before = hip.backwardTimeSplit(mode)
+        try:
+            out = hip.layerLeakyForward(x[some], v0[some].flatten(), a[some].flatten(), early, norm)[0]
+            return hip.layerLeakyBackward(go[some], None, out, x[some], v0[some].flatten(), a[some].flatten(), early, norm, True)[0]
+        finally:
+            hip.backwardTimeSplit(before)
+    whole, some = slice(0, b), slice(0, 40)
+    one_lane = backward(1, whole)[some]
+    assert torch.equal(backward(0, some), one_lane) and torch.equal(backward(0, whole)[some], one_lane)
+    assert not torch.equal(backward(1, some), one_lane)
+    assert torch.equal(backward(3, some), backward(1, some)) and not torch.equal(backward(3, whole)[some], one_lane)

@@ -7,10 +7,12 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# blocks of the forward kernels: 2, 14 and 16 (runs of 1 and 2), 18 (two left over), 200 and 202 (25); in blocks of four waves 510
-# (63), 512 and 600 (32, 88 left over); two and four neurons per lane; half lines shared, and none
+# blocks of the forward kernels: 2, 14 and 16 (runs of 1 and 2), 18 (two left over), 200, 202 (25) and 300 (37, four left over); in
+# blocks of four waves 510 (63), 512 and 600 (32, 88 left over); two and four neurons per lane; half lines shared, and none.  More
+# than 32 steps of at most one block per compute unit are another kernel's in the forward without records: 30 steps there
 @pytest.mark.parametrize("b,t,m", [
-    (1, 3, 65), (7, 3, 65), (8, 3, 65), (9, 35, 65), (100, 3, 65), (101, 33, 65),
+    (1, 3, 65), (7, 3, 65), (8, 3, 65), (9, 30, 65), (9, 35, 65), (100, 3, 65), (101, 30, 65),
+    (101, 33, 65), (150, 35, 65),
     (255, 3, 300), (256, 3, 300), (300, 30, 300), (5, 2, 110002), (5, 3, 1048580), (300, 3, 272), (300, 3, 288),
 ])
 @pytest.mark.parametrize("syn,records", [(False, False), (True, True)])
