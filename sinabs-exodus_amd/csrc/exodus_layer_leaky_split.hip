@@ -160,9 +160,15 @@ int launch(const LeakySplitArgs &a, bool uniform, int64_t B, hipStream_t s)
 
 }  // namespace
 
-// Up to 16 384 neurons it is ahead at every length, one lane / this, us: (8, t, 2048) 33 steps 5.7 / 5.1, 64 steps 7.8 / 6.1, 300 steps
-// 32.5 / 14.8.  At 32 768 (16, t, 2048) 33 steps 6.1 / 6.4, 300 steps 34.8 / 29.4, 1000 steps 106 / 91; at 65 536 300 steps
-// 43.4 / 51.5.
+// Up to 16 384 neurons a call with a gradient per output is ahead at every length, level for 33 to 48 steps without alpha gradient.
+// One lane / this, us, with alpha gradient and scalings, (8, t, 2048) 33 steps 7.6 / 6.1, 64 steps 9.7 / 6.4, 300 steps 44 / 18.6, 1000
+// steps 138 / 47; without, 33 steps 5.0 / 5.0, 300 steps 21.2 / 10.7.  At 32 768 (16, t, 2048) 33 steps 6.1 / 6.4, 300 steps
+// 34.8 / 29.4, 1000 steps 106 / 91; at 65 536 300 steps 43.4 / 51.5.  Blocks hold 16 neurons at least, but many samples of few neurons
+// leave the one-lane kernel's waves as empty: (16384, 300, 1) 1187 / 212, (4096, 300, 4) 311 / 45, (1024, 33, 4) 16.9 / 6.8.
+// A gradient of one value for all outputs leaves the one-lane kernel a tensor less to read, none without alpha gradient, and it is ahead
+// there up to 96 steps, (8, t, 2048) 33 steps 3.8 / 4.8, 64 steps 4.5 / 5.0, 160 steps 6.7 / 6.4, and by up to 8 % at 300 steps of
+// 8192 neurons and more, 9.5 / 9.9 (1000 steps 20.4 / 15.8); with alpha gradient up to 40 steps without scalings, 33 steps
+// 5.1 / 6.0.  It takes this kernel all the same: the call then gives the bits of the one with that value written out.
 constexpr int64_t LEAKY_SPLIT_MOST_NEURONS = 16384;
 bool exodus_layer_leaky_split_applies(int64_t B, int64_t T, int64_t M)
 {
