@@ -486,7 +486,8 @@ scan_span_kernel(const Op op, const int64_t n_rows, const int n_steps, const int
 // The drivers above fetch a row in tiles of 128 bytes, and what rows share at their ends again and in parts, which for rows of a few
 // tiles is most of it.  Before / here, us for 2^26 steps, spiking forward and backward, leaky forward and backward: 10 steps
 // 740 / 138, 1307 / 154, 357 / 88, 1162 / 148; 27 steps 618 / 142, 520 / 147, 279 / 88, 487 / 134; 65 steps 406 / 160, 265 / 193,
-// 189 / 97, 240 / 140; synaptic forward and backward 17 steps 829 / 187, 1977 / 192.  4.5 to 6.1 TB/s: what copies reach.
+// 189 / 97, 240 / 140; synaptic forward and backward 17 steps 829 / 187, 1977 / 192.  4.2 to 6.1 TB/s; copies reach 4.9 to 6.2.  Where fewer rows fit a compute
+// unit's LDS the rate falls, and still beats tiles: spiking backward 90 steps 3.3 TB/s, one tensor of 150 steps and five of 63 3.2 to 3.4.
 // Word e of the piece lies at e + pad * (e / 64) in LDS: without a pad the lanes, whose rows lie an even number of words apart,
 // would meet in the same banks.
 // ---------------------------------------------------------------------------------------------
@@ -1087,13 +1088,18 @@ inline size_t whole_slot_words(int64_t rows, int64_t t)
 // share a compute unit's LDS; `slots` tensors lie there.  us for 2^26 steps, spiking forward (one slot) and backward (two),
 // synaptic backward (three), 64 rows / 32: 16 steps 140 / 143, 142 / 180, 203 / 299; 24 steps 142 / 140, 145 / 153, 210 / 252;
 // 33 steps 152 / 148, 149 / 146, 232 / 216; one slot, 32 rows / 16: 61 steps 153 / 158, 65 steps 166 / 160, 121 steps 230 / 202.
-// Against scan_kernel, where rows are no multiple of 4 steps: one slot 150 steps 239 / 236 (leaky 121 / 106), 201 steps 234 / 277;
-// more slots 90 steps 294 / 244, 110 steps 272 / 276 (leaky 249 / 162), 130 steps 215 / 345.
+// Against scan_kernel, where rows are no multiple of 4 steps: one slot 122 steps 254 / 216, 150 steps 241 / 237 (leaky 121 / 106), 201
+// steps 234 / 277 (with two spikes or more somewhere among the 64 rows of almost every step, where a lane's quotient holds all up, 122
+// steps 256 / 252, 150 steps 241 / 272); two and three slots 90 steps 294 / 244, 95 steps 262 / 255, 98 steps 241 / 257, 110 steps 272 / 276
+// (leaky 249 / 162), 130 steps 215 / 345; four 27 steps 1415 / 304, 63 steps 755 / 407, 65 steps 642 / 447; five 27 steps 1830 / 391,
+// 63 steps 966 / 505: LDS ends these before the drivers meet.
 // Against scan_span_kernel, multiples of 4: 12 steps 331 / 137, 425 / 142; 28 steps 420 / 142, 235 / 138; 44 steps 206 / 144,
 // 229 / 162, 392 / 261; 56 steps 179 / 147, 196 / 172, 328 / 274; 60 steps 171 / 148, 193 / 195, 319 / 354; 68 steps 155 / 159,
-// 171 / 204, 276 / 365.  Rows of whole 64-byte
-// sectors suit that driver: 16 steps 160 / 140, 226 / 142, 366 / 203, but 32 steps 135 / 140, 145 / 149, 213 / 234, 48 steps
-// 172 / 146, 165 / 169, 240 / 257.
+// 171 / 204, 276 / 365.  Four and five slots (spiking backward with a surrogate tensor and a gradient on the potentials, synaptic
+// backward with gradients on both records): 12 steps 930 / 276, 1117 / 359; 28 steps 493 / 292, 596 / 369; 44 steps 462 / 309,
+// 695 / 449; 56 steps 391 / 347, 589 / 527; 60 steps 382 / 417, 575 / 671.
+// Rows of whole 64-byte sectors suit that driver: 16 steps 160 / 140, 226 / 142, 366 / 203, 477 / 247, 577 / 324, but 32 steps
+// 135 / 140, 145 / 149, 213 / 234, 286 / 278, 345 / 383, 48 steps 172 / 146, 165 / 169, 240 / 257, 327 / 306, 391 / 540: one line for all.
 inline int whole_rows(int slots, int64_t t)
 {
     const int64_t most = t % 16 == 0 ? 16 : (t % 4 == 0 ? (slots > 2 ? 56 : 60) : (slots == 1 ? 150 : 100));
