@@ -272,7 +272,8 @@ __device__ __forceinline__ float reset_amount(float v, const Neuron &n, const Ca
 __device__ __forceinline__ float decay_factor(float tau) { return expf(-__fdiv_rn(1.0f, tau)); }
 
 // The decay factor of neuron m of batch element b in row `row`; `write`: this lane writes what the call is to leave behind.
-// (A launch for it was 2.4 us on the device and 5 on the host, for calls that take 100.)
+// (A launch for it was 2.4 us on the device and 5 on the host, for calls that take 100.  A spiking layer does without it where the
+// parameters are those of its last call: a step of an optimizer has them checked again, and the check wants the factors ahead.)
 __device__ __forceinline__ float decay_of(const Decay &d, int64_t b, int64_t m, int64_t row, bool write)
 {
     const float tau = d.tau[d.one ? 0 : m], alpha = decay_factor(tau);
