@@ -105,6 +105,27 @@ def test_as_the_python_functions(form, loss, python_functions):
             assert p.shape == q.shape and torch.equal(p, q) and torch.equal(first[k], q), k
 
 
+@pytest.mark.parametrize("form", ["lif", "lif tau per neuron", "lif syn", "lif alphas, records", "expleak", "expleak alphas"])
+def test_steps_of_an_optimizer_between_calls(form, python_functions):
+    """Every call sees the parameters that the step before has left, whose values are checked again."""
+    def train():
+        layer, x = build(FORMS[form])
+        opt = torch.optim.SGD(layer.parameters(), lr=1e-3, momentum=0.5)
+        seen = []
+        for k in range(4):
+            if k != 2:                                         # a call with the parameters of the one before
+                opt.step()
+            seen += [z.detach().clone() for z in step(layer, x, "dense") if z is not None]
+            seen += [p.detach().clone() for p in layer.parameters()]
+        return seen
+    got = train()
+    python_functions()
+    want = train()
+    assert len(got) == len(want) and all(torch.equal(p, q) for p, q in zip(got, want))
+    count = len(list(build(FORMS[form])[0].parameters()))
+    assert not all(torch.equal(p, q) for p, q in zip(want[-count:], want[len(want) // 4 - count:]))    # the steps changed something
+
+
 # one block, waves with roles, blocks of one and of four waves, two and four neurons per lane, a sequence without steps
 @pytest.mark.parametrize("b,t,m", [(1, 10, 300), (1, 40, 64), (3, 40, 70), (40, 33, 1000), (30, 4, 700), (9, 3, 66560), (33, 2, 131072),
                                    (2, 0, 5)])
