@@ -4,8 +4,9 @@
 //
 // Why it exists: a training step of a small layer is host time, and the autograd engine runs the backward pass on a thread
 // of its own, where the 55 us of Python and ctypes that a backward pass was took up to 165 (caches and a core of its own).
-// Python and ctypes / these, us per step through the layer, forward and backward: IAF (8, 100, 256) 238 / 149, LIF
-// (32, 100, 512) with a trained time constant 271 / 173, a streamed chunk (1, 10, 1024) without gradients 47 / 24.
+// Python and ctypes / the calls in native code / the layers' nodes as well (LifLayer, LeakyLayer below), us per step through the layer,
+// forward and backward: IAF (8, 100, 256) 238 / 149 / 96, LIF (32, 100, 512) with a trained time constant 271 / 173 / 113, a streamed
+// chunk (1, 10, 1024) without gradients, which has no node, 47 / 24 / 21.
 #include <ATen/Functions.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
@@ -601,8 +602,10 @@ Three leaky_backward_fused(const Tensor &grad_out, const Tensor &alpha, const Ma
 // What layer_function.py's two Functions do, for the calls that need no Python on the way back (a surrogate that the kernels
 // know): the same tensors saved in the same order, the same gradients.  The engine runs a backward pass on a thread of its own,
 // where Python means the interpreter lock, cold caches and thirteen unpacked tensors; and the input's shape is taken and given
-// back here instead of by reshapes that are nodes of their own.  us per training step in Python and here: IAF (8, 100, 256)
-// 136 / 99, LIF (32, 100, 512) with a trained time constant 160 / 114, LIF with synapses (4, 2000, 512), both constants trained, 199 / 143.
+// back here instead of by reshapes that are nodes of their own.  us per training step with Python Functions and with these nodes (and the
+// kernels that came with them): IAF (8, 100, 256) 134 / 96, LIF (32, 100, 512) with a trained time constant 154 / 113, LIF with synapses
+// (4, 2000, 512), both constants trained, 194 / 139; with the constants written to between the steps, as an optimizer does, 216 / 180
+// and 263 / 222 (with the same write to other tensors 179 / 136 and 225 / 174).
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
